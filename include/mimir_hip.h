@@ -242,7 +242,9 @@ int mimir_rope_fwd(mimir_ctx* ctx, const float* q, float* q_out, int64_t q_heads
  * head_dim <= 2048 (above 128 a plain fp32 vector kernel runs instead of the
  * matrix-core one).  fp32 throughout (fp32 matrix-core products), no score
  * matrix in memory.  out must not overlap q, k or v.  kv_len == 0 gives zeros;
- * batch == 0 or q_len == 0 is a no-op.  Device pointers, stream order. */
+ * batch == 0 or q_len == 0 is a no-op.  Device pointers, stream order.  Up to
+ * 8 queries without a mask may use the context's fixed workspace (allocated
+ * with the context). */
 int mimir_attention_fwd(mimir_ctx* ctx, const float* q, int64_t ld_q, const float* k, const float* v,
                         int64_t ld_kv, float* out, int64_t ld_out, int64_t batch, int64_t q_len,
                         int64_t kv_len, int64_t heads, int64_t head_dim, float scale, int causal);

@@ -523,6 +523,11 @@ int mimir_attention_fwd(mimir_ctx* ctx, const float* q, int64_t ld_q, const floa
     const bool vec = head_dim % 4 == 0 && ld_q % 4 == 0 && ld_kv % 4 == 0 && ld_out % 4 == 0 && aligned16(q) &&
                      aligned16(a.k) && aligned16(a.v) && aligned16(out) &&
                      ld_kv < (int64_t{1} << 31) / (4 * kKeyTile);
+    // Few queries: each key row is read once by vector code, where the
+    // matrix-core kernel would use one of its waves (attention_decode.hip).
+    if (attention_decode_applies(q_len, kv_len, head_dim, a.causal))
+        return attention_decode_launch(ctx, q, ld_q, a.k, a.v, ld_kv, out, ld_out, batch, q_len, kv_len, heads, head_dim,
+                                       a.qscale, vec);
     if (head_dim <= 32) return launch<32>(ctx, a, vec);
     if (head_dim <= 64) return launch<64>(ctx, a, vec);
     if (head_dim <= 128) return launch<128>(ctx, a, vec);

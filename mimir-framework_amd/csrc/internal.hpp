@@ -31,6 +31,10 @@ struct mimir_ctx {
     // Device address of this GPU's fixed scratch array (backward.hip), for
     // the entry point that allocates nothing; set at context creation.
     void* noalloc_scratch = nullptr;
+    // Workspace of kFixedWorkBytes, allocated with the context (so that the
+    // ops that use it allocate nothing): the partial outputs of a decoding
+    // step's splits (attention_decode.hip), in stream order.
+    void* fixed_work = nullptr;
     // This GPU's columns of 1.0f then -0.0f (mimir::kUnitCols each), the
     // weights of a row kernel's absent scale / bias (norm.hip).
     const float* unit_weights = nullptr;
@@ -122,6 +126,16 @@ void gemm_release(mimir_ctx* ctx);
 // Whether products go to hipBLASLt (unless MIMIR_TUNE blas=0), where the
 // transposed-operand forms run as fast as the plain ones.
 bool gemm_lt(mimir_ctx* ctx);
+
+// The attention core, not causal, for at most kDecodeQueries queries per sequence
+// (attention_decode.hip), of heads up to 128; qscale = scale * log2(e).  vec:
+// head_dim, the strides and the pointers are 16-byte multiples.
+constexpr int kDecodeQueries = 8;
+constexpr size_t kFixedWorkBytes = size_t(4) << 20;
+bool attention_decode_applies(int64_t q_len, int64_t kv_len, int64_t head_dim, bool causal);
+int attention_decode_launch(mimir_ctx* ctx, const float* q, int64_t ld_q, const float* k, const float* v, int64_t ld_kv,
+                            float* out, int64_t ld_out, int64_t batch, int64_t q_len, int64_t kv_len, int64_t heads,
+                            int64_t head_dim, float qscale, bool vec);
 
 // A chain of elementwise layers run as one kernel (store.hip's fusion):
 // v = ins[0]; then each step k sets v = op_k(v, operand) -- GELU, SiLU, or

@@ -114,9 +114,16 @@ int mimir_ctx_create(int device, mimir_ctx** out) {
         return MIMIR_EDEVICE;
     }
     ctx->stream = ctx->own_stream;
+    if (hipMalloc(&ctx->fixed_work, kFixedWorkBytes) != hipSuccess) {
+        (void)hipGetLastError();
+        (void)hipStreamDestroy(ctx->own_stream);
+        delete ctx;
+        return MIMIR_ENOMEM;
+    }
     int init_st = noalloc_scratch_init(ctx);
     if (init_st == MIMIR_OK) init_st = norm_init(ctx);
     if (int st = init_st) {
+        (void)hipFree(ctx->fixed_work);
         (void)hipStreamDestroy(ctx->own_stream);
         delete ctx;
         return st;
@@ -133,6 +140,7 @@ int mimir_ctx_destroy(mimir_ctx* ctx) {
         gemm_release(ctx);
         for (auto& kv : ctx->allocs) (void)hipFree(kv.first);
         if (ctx->scratch) (void)hipFree(ctx->scratch);
+        (void)hipFree(ctx->fixed_work);
         for (void* p : ctx->retired) (void)hipFree(p);
         (void)hipStreamDestroy(ctx->own_stream);
     }

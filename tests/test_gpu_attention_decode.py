@@ -1,0 +1,46 @@
+"""The attention core for a few queries against many keys (a decoding step):
+the vector kernel and its splits over workgroups against float64, at the edges
+of its groups of keys, its vector widths and its split sizes."""
+import numpy as np
+import pytest
+
+import oracle as O
+from _attention import assert_attention_close, attention64
+from test_gpu_attention import gpu_attention, rand_qkv
+
+pytestmark = pytest.mark.gpu
+
+
+# 64 keys per step of a workgroup (16 lanes per key; 128 for heads up to 32),
+# one split per 256 keys where few heads share the GPU; 1, 2 and 4 queries per
+# workgroup; heads of 1 to 4 vectors per lane, odd ones in scalar loads.
+@pytest.mark.parametrize("b,lq,lk,heads,hd", [
+    (1, 1, 1, 1, 4), (2, 1, 15, 3, 32), (1, 1, 64, 2, 64), (3, 1, 65, 2, 64), (1, 1, 256, 2, 128), (1, 1, 257, 1, 128),
+    (2, 2, 1000, 3, 80), (1, 3, 513, 2, 96), (1, 4, 127, 2, 32), (1, 5, 300, 1, 100), (2, 8, 2049, 2, 64),
+    (1, 1, 5000, 1, 7), (1, 2, 130, 3, 33), (40, 1, 70, 16, 36), (1, 6, 64, 2, 125)])
+def test_decode(ctx, b, lq, lk, heads, hd):
+    q, k, v = rand_qkv(lq + lk + hd, b, lq, lk, heads * hd)
+    got = gpu_attention(ctx, q, k, v, heads, False)
+    for i in range(b):
+        out, mag, cond = attention64(q[i], k[i], v[i], heads, False, O.attention_scale(hd))
+        assert_attention_close(got[i], out, mag, cond, f"decode {b} {lq} {lk} {heads} {hd} [{i}]")
+
+
+@pytest.mark.parametrize("lk", [40, 700])
+def test_decode_special_values(ctx, lk):
+    """A key of -inf scores weighs nothing, an infinite value row reaches only
+    its own dimension, NaN only the queries and dimensions that see it: as
+    the float64 softmax has it."""
+    q, k, v = rand_qkv(5, 1, 2, lk, 64)
+    q[0, :, 3] = np.abs(q[0, :, 3]) + 0.5
+    k[0, 7, 3] = -np.inf
+    v[0, lk - 1, 5] = np.inf
+    v[0, 2, 9] = np.nan
+    got = gpu_attention(ctx, q, k, v, 1, False)[0]
+    s = (q[0].astype(np.float64) @ k[0].astype(np.float64).T) * O.attention_scale(64)
+    p = np.exp(s - s.max(1, keepdims=True))
+    p /= p.sum(1, keepdims=True)
+    keep = [d for d in range(64) if d not in (5, 9)]
+    v64 = v[0].astype(np.float64)
+    np.testing.assert_allclose(got[:, keep], p @ v64[:, keep], rtol=0, atol=1e-5)
+    assert np.isposinf(got[:, 5]).all() and np.isnan(got[:, 9]).all()
