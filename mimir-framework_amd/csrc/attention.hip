@@ -12,38 +12,29 @@
 // Q is multiplied by scale * log2(e) once, so the scores come out of the
 // matrix core in base-2 units and each probability is one v_exp_f32.
 //
-// Matrix-core mapping.  v_mfma_f32_32x32x2_f32 computes D[32x32] += A[32x2] *
-// B[2x32]; lane l supplies A[l%32][l/32] and B[l/32][l%32] and receives
-// D[8*(r/4) + 4*(l/32) + r%4][l%32] in accumulator register r (r = 0..15).
-// - Scores: S^T = K Q^T, keys as rows, queries as columns.  A = K (row = the
-//   key, k index = one head dimension), B = Q^T, so lane l owns query l%32 and
-//   16 of the 32 keys of the tile.  The head dimensions are split between the
-//   two lane halves: at step s the half h = l/32 supplies dimension
-//   h*DP/2 + s, so each lane reads four steps of K with one 16-byte LDS read
-//   and holds its query's DP/2 Q values in registers for the whole kernel.
-// - Softmax: per lane over its 16 keys; the running max is shared with the
-//   other half (lane l ^ 32, same query) once per tile.
-// - Output: O^T = V^T P^T.  The accumulator register r of S^T already holds
-//   P^T[key(r, h)][query] in the layout of the B operand when the MFMA's two
-//   k-slots are the keys key(r, 0), key(r, 1), key(r, h) = 8*(r/4) + 4h + r%4,
-//   so the probabilities feed the second product without a lane exchange.
-//   The A operand row i of dimension block db is head dimension (DP/32)*i + db,
-//   so a lane reads its DP/32 values of one V row with one LDS read, and its
-//   output rows come out as DP/32 consecutive dimensions (one 16-byte store
-//   for DP = 128).
+// Products.  Every fp32 operand (Q, K, V and the probabilities) is held as
+// three bf16 terms and every product is six bf16 MFMAs (split.hpp): 6/16 of
+// the fp32 matrix time.  v_mfma_f32_32x32x16_bf16 computes D[32x32] +=
+// A[32x16] B[16x32]; lane l supplies A[l%32][8(l/32) + i], B[8(l/32) + i][l%32]
+// (i = 0..7) and receives D[8(r/4) + 4(l/32) + r%4][l%32] in register r.
+// - Scores: S^T = K Q^T, keys as rows, queries as columns.  Lane l owns query
+//   l%32 (its share of Q split once, in registers for the whole kernel) and
+//   16 of the 32 keys of the tile.
+// - Softmax: per lane over its 16 keys; the max is shared with the other half
+//   (lane l ^ 32, same query).
+// - Output: O^T = V^T P^T.  Registers 8c .. 8c+7 of S^T hold P^T at the keys
+//   16c + 4(l/32) + {0..3, 8..11}: the B operand of a product over 16 keys in
+//   that order, so the probabilities feed it without a lane exchange, and V is
+//   laid out in LDS in the same order.
 //
-// Pipeline.  A wave issues its instructions in order, and a v_mfma holds the
-// matrix pipe for 64 cycles, so the softmax's vector work only overlaps the
-// matrix core if it sits between independent MFMAs.  Iteration t therefore
-// computes the scores of tile t+1 (S_next = K_{t+1} Q^T) interleaved
-// instruction by instruction with the softmax of tile t (whose scores came
-// from iteration t-1), then O += V_t^T P_t.  K runs one tile ahead of V: LDS
-// holds a K ring and a V ring of two tiles each; iteration t reads K_{t+1}
-// and V_t and refills the slots of K_t and V_{t-1} with K_{t+2} and V_{t+1},
-// whose global loads were issued at the start of the iteration, then one
-// barrier.
+// LDS: K planes [3][32 keys][DP] and V^T planes [3][DP][32 keys] in bf16, rows
+// padded by 16 bytes (eight rows' 16-byte reads touch every bank once).  The
+// tile is split on its way in, once for all queries of the workgroup: K in
+// groups of eight dimensions of a row, V in groups of eight keys of a column.
+// Two buffers: iteration t computes tile t while tile t+1 moves from registers
+// to the other one and tile t+2 is on its way to the registers; one barrier.
 //
-// Workgroup: 4 waves, 32 queries each (128 queries of one (sequence, head)).
+// Workgroup: WAVES waves, 32 queries each, of one (sequence, head).
 // Causal: a workgroup stops at its last query's diagonal, a wave skips the
 // tiles past its own diagonal and masks inside its last tile only (the
 // diagonal, or the sequence's ragged end).
@@ -51,8 +42,19 @@
 // (sequence, head) count divides by 8, each XCD owns an eighth of them (their
 // K and V stay in that XCD's L2) and runs its query blocks longest first
 // across all of its heads, so the short causal blocks fill the tail.
+//
+// Bound by the power the matrix cores draw: at 8 x 32 heads x 1024 tokens x 128,
+// causal, the bf16 MFMAs hold the matrix pipes 51% of the cycles at 1.9 GHz (a
+// loop of nothing else runs at 1.6 GHz), beside 350 VALU operations per 96
+// MFMAs.  Measured there 400 us = 172 TFLOP/s of fp32 work, against 627 us on
+// the fp32 MFMAs (157 TFLOP/s peak); 16 heads x 1024 x 128 99 / 152 us, 96 heads
+// x 333 x 777 x 80 77 / 213 us.  Within noise of that: two accumulators in
+// turns, LDS reads ordered ahead of the MFMAs, the split interleaved with them,
+// raised priority for half the waves; four waves with two workgroups' worth of
+// LDS are slower (the tile is split twice as often).
 #include "common.hpp"
 #include "internal.hpp"
+#include "split.hpp"
 
 #include <math.h>
 
@@ -62,16 +64,14 @@ using namespace mimir;
 
 namespace {
 
-typedef float f16v __attribute__((ext_vector_type(16)));
-typedef float f2 __attribute__((ext_vector_type(2)));
-
 constexpr int kQPerWave = 32;
-constexpr int kWaves = 4;
-constexpr int kQPerBlock = kQPerWave * kWaves;  // 128
 constexpr int kKeyTile = 32;
-constexpr int kThreads = kWaves * kWave;        // 256
 constexpr int kXcds = 8;
 constexpr float kLog2e = 1.4426950408889634f;
+// The running max follows a growing score only past this many base-2 units:
+// probabilities up to 2^8 of the final scale lose nothing in fp32, and the
+// rescale of the output (DP / 2 multiplies) runs in few tiles instead of most.
+constexpr float kMaxSlack = 8.0f;
 
 struct AttnArgs {
     const float* q;
@@ -80,68 +80,11 @@ struct AttnArgs {
     float* out;
     int64_t ld_q, ld_kv, ld_out;  // row strides (floats)
     int32_t q_len, kv_len, heads, head_dim;
-    int32_t n_qblocks;            // ceil(q_len / 128)
+    int32_t n_qblocks;            // query blocks of one (sequence, head)
     uint32_t total_blocks;        // batch * heads * n_qblocks
     float qscale;                 // scale * log2(e), applied to Q
     int32_t causal;
 };
-
-// LDS: the K ring [2][32][DP + 4] (the pad staggers the rows across banks for
-// the column-wise reads), then the V ring [2][32][DP].
-template <int DP>
-struct Lds {
-    static constexpr int kLd = DP + 4;
-    static constexpr int vLd = DP;
-    static constexpr int kTile = kKeyTile * kLd;
-    static constexpr int vTile = kKeyTile * vLd;
-    static constexpr int vRing = 2 * kTile;
-    static constexpr int total = 2 * kTile + 2 * vTile;
-    static constexpr int f4PerRow = DP / 4;
-    static constexpr int loads = kKeyTile * f4PerRow / kThreads;  // float4 per thread per tile
-    static_assert(loads >= 1 && kKeyTile * f4PerRow == loads * kThreads, "tile / block mismatch");
-};
-
-// 4 floats of a row at column c (a multiple of 4), zero past `valid` columns.
-// VEC: head_dim, the strides and the base pointers are 16-byte multiples.
-template <bool VEC>
-__device__ __forceinline__ f4 load4(const float* row, int c, int valid) {
-    if constexpr (VEC) {
-        if (c < valid) return *reinterpret_cast<const f4*>(row + c);
-        return f4{0.f, 0.f, 0.f, 0.f};
-    } else {
-        f4 r;
-        r.x = c + 0 < valid ? row[c + 0] : 0.f;
-        r.y = c + 1 < valid ? row[c + 1] : 0.f;
-        r.z = c + 2 < valid ? row[c + 2] : 0.f;
-        r.w = c + 3 < valid ? row[c + 3] : 0.f;
-        return r;
-    }
-}
-
-// Scalar-path tile load: four loads from clamped, always valid columns
-// (< head_dim); the caller clamps the row below kv_len.  What lies outside
-// the tile's valid rows / columns is replaced by zeros when the values are
-// written to LDS (zero_outside).
-__device__ __forceinline__ f4 load4_clamped(const float* row, int c, int head_dim) {
-    f4 r;
-    r.x = row[min(c + 0, head_dim - 1)];
-    r.y = row[min(c + 1, head_dim - 1)];
-    r.z = row[min(c + 2, head_dim - 1)];
-    r.w = row[min(c + 3, head_dim - 1)];
-    return r;
-}
-
-// Word 3 of a raw (stride 0) buffer descriptor on gfx9-family GPUs: 32-bit
-// data format, no swizzle; out-of-range offsets return zeros.
-constexpr int kBufferWord3 = 0x00020000;
-
-__device__ __forceinline__ f4 zero_outside(f4 x, bool row_ok, int c, int head_dim) {
-    x.x = row_ok && c + 0 < head_dim ? x.x : 0.f;
-    x.y = row_ok && c + 1 < head_dim ? x.y : 0.f;
-    x.z = row_ok && c + 2 < head_dim ? x.z : 0.f;
-    x.w = row_ok && c + 3 < head_dim ? x.w : 0.f;
-    return x;
-}
 
 // Workgroup -> (sequence * heads + head, query block): see the file comment.
 __device__ __forceinline__ void block_coords(const AttnArgs& a, uint32_t bid, uint32_t* bh, int* qb) {
@@ -156,12 +99,166 @@ __device__ __forceinline__ void block_coords(const AttnArgs& a, uint32_t bid, ui
     *bh = first + idx % owned;
 }
 
-template <int DP, bool VEC>
-__global__ __launch_bounds__(kThreads, 2) void attention_fwd_mfma(AttnArgs a) {
-    using L = Lds<DP>;
-    constexpr int kHalf = DP / 2;  // dimensions per lane half = MFMA k-steps of S
-    constexpr int kDb = DP / 32;   // output dimension blocks
-    __shared__ __attribute__((aligned(16))) float lds[L::total];
+// One query by one wave in plain fp32, the head's dimensions spread over the
+// lanes (CH per lane, lane + 64 c): each score a DPP wave sum, the same online
+// softmax and the same division by (sum + 1e-9).
+template <int CH>
+__device__ __forceinline__ void one_query(const float* qrow, const float* kb, const float* vb, float* orow,
+                                          int64_t ld_kv, int64_t keys, int head_dim, float qscale) {
+    const int lane = threadIdx.x % kWave;
+    float q[CH], acc[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const int d = lane + c * kWave;
+        q[c] = d < head_dim ? qrow[d] * qscale : 0.f;
+        acc[c] = 0.f;
+    }
+    float m_run = -1e30f, l_run = 0.f;
+    for (int64_t j = 0; j < keys; ++j) {
+        const float* krow = kb + j * ld_kv;
+        const float* vrow = vb + j * ld_kv;
+        float part = 0.f;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            const int d = lane + c * kWave;
+            if (d < head_dim) part += q[c] * krow[d];
+        }
+        const float s = wave_sum(part);  // wave-uniform
+        const float m_new = fmaxf(m_run, s);
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        const float p = __builtin_amdgcn_exp2f(s - m_new);
+        m_run = m_new;
+        l_run = l_run * alpha + p;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            const int d = lane + c * kWave;
+            acc[c] = acc[c] * alpha + (d < head_dim ? p * vrow[d] : 0.f);
+        }
+    }
+    const float inv = 1.0f / (l_run + 1e-9f);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const int d = lane + c * kWave;
+        if (d < head_dim) orow[d] = acc[c] * inv;
+    }
+}
+
+// A tile of 32 keys on its way from memory to LDS.  Items of eight values: K
+// item = (key, eight dimensions), V item = (dimension, eight keys in the order
+// of the file comment); 4 * DP of each, dealt to THREADS threads.  Loads go
+// through a descriptor that starts at the tile's first row and ends after the
+// sequence's last, so rows past kv_len read as zeros; columns are clamped into
+// the head (past head_dim, Q is zero and the output is not stored).
+// VEC: K moves in 16-byte loads (head_dim, the stride and the base pointer are
+// 16-byte multiples).
+template <int DP, int THREADS, bool VEC>
+struct KvTile {
+    static constexpr int kKeyBytes = 2 * DP + 16, kDimBytes = 2 * kKeyTile + 16;
+    static constexpr int kKPlane = kKeyTile * kKeyBytes, kVPlane = DP * kDimBytes;
+    static constexpr int kBytes = 3 * (kKPlane + kVPlane);
+    static constexpr int kKind = 4 * DP;  // items of each kind
+    static constexpr int kItems = (kKind + THREADS - 1) / THREADS;
+    static constexpr int kSpare = kItems * THREADS - kKind;  // threads without an item of one kind
+    float k[kItems][8], v[kItems][8];
+    uint32_t koff[kItems], voff[kItems];  // byte offsets of an item's first element
+    int32_t kstep[kItems];                // VEC: bytes from the first four to the second four of a K item
+    uint32_t ld4;
+
+    // Where the items do not fill the threads, the first ones take K and the
+    // last ones V.
+    static __device__ __forceinline__ int k_item(int j) { return static_cast<int>(threadIdx.x) + j * THREADS; }
+    static __device__ __forceinline__ int v_item(int j) { return k_item(j) - kSpare; }
+    static __device__ __forceinline__ int wave_start() {
+        return __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x)) & ~(kWave - 1);
+    }
+    static __device__ __forceinline__ bool has_k(int j) { return kSpare == 0 || wave_start() + j * THREADS < kKind; }
+    static __device__ __forceinline__ bool has_v(int j) { return kSpare == 0 || wave_start() + j * THREADS >= kSpare; }
+
+    __device__ __forceinline__ void init(int64_t ld, int head_dim) {
+        ld4 = static_cast<uint32_t>(ld * 4);
+#pragma unroll
+        for (int j = 0; j < kItems; ++j) {
+            const int ki = min(k_item(j), kKind - 1), key = ki / (DP / 8), d = 8 * (ki % (DP / 8));
+            if constexpr (VEC) {
+                koff[j] = key * ld4 + 4 * min(d, head_dim - 4);
+                kstep[j] = 4 * (min(d + 4, head_dim - 4) - min(d, head_dim - 4));
+            } else {
+                koff[j] = key * ld4 + 4 * d;
+            }
+            const int vi = max(v_item(j), 0), group = vi / DP;
+            voff[j] = 4 * min(vi % DP, head_dim - 1) + (16 * (group / 2) + 4 * (group % 2)) * ld4;
+        }
+    }
+    __device__ __forceinline__ void load(const float* kbase, const float* vbase, int tile, int64_t ld, int kv_len,
+                                         int head_dim) {
+        const int64_t first = static_cast<int64_t>(tile) * kKeyTile * ld;
+        const int rows = min(kKeyTile, kv_len - tile * kKeyTile);
+        // The last row ends with the head, not with the stride.
+        const int bytes = static_cast<int>((rows - 1) * ld4 + 4 * head_dim);
+        const __amdgpu_buffer_rsrc_t rk = buffer_of(kbase + first, bytes), rv = buffer_of(vbase + first, bytes);
+#pragma unroll
+        for (int j = 0; j < kItems; ++j) {
+            if (has_k(j)) {
+                if constexpr (VEC) {
+                    const f4 a = buffer_f4(rk, koff[j]), b = buffer_f4(rk, koff[j] + kstep[j]);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        k[j][e] = a[e];
+                        k[j][4 + e] = b[e];
+                    }
+                } else {
+                    const int d = 8 * (k_item(j) % (DP / 8));
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) k[j][e] = buffer_f1(rk, koff[j] + 4 * (min(d + e, head_dim - 1) - d));
+                }
+            }
+            if (has_v(j)) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[j][e] = buffer_f1(rv, voff[j] + ((e & 3) + 8 * (e >> 2)) * ld4);
+            }
+        }
+    }
+    __device__ __forceinline__ void stash(char* lds) const {
+#pragma unroll
+        for (int j = 0; j < kItems; ++j) {
+            if (has_k(j)) {
+                const int id = k_item(j);
+                char* p = lds + id / (DP / 8) * kKeyBytes + id % (DP / 8) * 16;
+                const Split8 s = split8(k[j]);
+                *reinterpret_cast<u4*>(p) = s.h;
+                *reinterpret_cast<u4*>(p + kKPlane) = s.m;
+                *reinterpret_cast<u4*>(p + 2 * kKPlane) = s.l;
+            }
+            if (has_v(j)) {
+                const int id = v_item(j);
+                char* p = lds + 3 * kKPlane + id % DP * kDimBytes + id / DP * 16;
+                const Split8 s = split8(v[j]);
+                *reinterpret_cast<u4*>(p) = s.h;
+                *reinterpret_cast<u4*>(p + kVPlane) = s.m;
+                *reinterpret_cast<u4*>(p + 2 * kVPlane) = s.l;
+            }
+        }
+    }
+    // MFMA operands: dimensions 16 c + 8 hf .. + 7 of key li; the eight keys
+    // (c, hf) of dimension 32 db + li.
+    static __device__ __forceinline__ Split8 key_rows(const char* lds, int li, int hf, int c) {
+        const char* p = lds + li * kKeyBytes + 32 * c + 16 * hf;
+        return Split8{*reinterpret_cast<const u4*>(p), *reinterpret_cast<const u4*>(p + kKPlane),
+                      *reinterpret_cast<const u4*>(p + 2 * kKPlane)};
+    }
+    static __device__ __forceinline__ Split8 value_cols(const char* lds, int li, int hf, int db, int c) {
+        const char* p = lds + 3 * kKPlane + (32 * db + li) * kDimBytes + 32 * c + 16 * hf;
+        return Split8{*reinterpret_cast<const u4*>(p), *reinterpret_cast<const u4*>(p + kVPlane),
+                      *reinterpret_cast<const u4*>(p + 2 * kVPlane)};
+    }
+};
+
+template <int DP, int WAVES, bool VEC>
+__global__ __launch_bounds__(WAVES * kWave, WAVES > 4 ? 2 : 1) void attention_fwd_mfma(AttnArgs a) {
+    using Tile = KvTile<DP, WAVES * kWave, VEC>;
+    constexpr int kC = DP / 16;   // MFMA steps of a score
+    constexpr int kDb = DP / 32;  // output dimension blocks
+    __shared__ __attribute__((aligned(16))) char lds[2 * Tile::kBytes];
 
     uint32_t bh;
     int qb;
@@ -173,12 +270,10 @@ __global__ __launch_bounds__(kThreads, 2) void attention_fwd_mfma(AttnArgs a) {
     const float* vbase = a.v + b * a.kv_len * a.ld_kv + hd_off;
     float* obase = a.out + b * a.q_len * a.ld_out + hd_off;
 
-    const int tid = threadIdx.x;
-    const int wave = tid / kWave;
-    const int lane = tid % kWave;
-    const int li = lane % 32;  // query column / MFMA row index
-    const int hf = lane / 32;  // lane half
-    const int q0 = qb * kQPerBlock;
+    const int wave = threadIdx.x / kWave;
+    const int lane = threadIdx.x % kWave;
+    const int li = lane % 32, hf = lane / 32;
+    const int q0 = qb * kQPerWave * WAVES;
     const int qw0 = q0 + wave * kQPerWave;
     const int my_q = qw0 + li;
 
@@ -186,7 +281,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_fwd_mfma(AttnArgs a) {
     int key_end = a.kv_len;
     int wave_key_end = a.kv_len;
     if (a.causal) {
-        key_end = min(key_end, min(q0 + kQPerBlock, a.q_len));
+        key_end = min(key_end, min(q0 + kQPerWave * WAVES, a.q_len));
         wave_key_end = min(wave_key_end, min(qw0 + kQPerWave, a.q_len));
     }
     if (qw0 >= a.q_len) wave_key_end = 0;
@@ -196,211 +291,132 @@ __global__ __launch_bounds__(kThreads, 2) void attention_fwd_mfma(AttnArgs a) {
     // (causal: key > query; all: key >= kv_len).
     const int lane_key_end = min(a.kv_len, a.causal ? my_q + 1 : a.kv_len);
 
-    // This lane's Q values, times scale*log2(e): query my_q, dimensions
-    // hf*kHalf + [0, kHalf).
-    float qreg[kHalf];
+    Tile tile;
+    tile.init(a.ld_kv, a.head_dim);
+    if (n_tiles > 0) tile.load(kbase, vbase, 0, a.ld_kv, a.kv_len, a.head_dim);
+
+    // This lane's Q values, times scale*log2(e), zero past head_dim.
+    Split8 q[kC];
     {
         const float* qrow = qbase + static_cast<int64_t>(min(my_q, a.q_len - 1)) * a.ld_q;
-        const int valid = my_q < a.q_len ? a.head_dim : 0;
 #pragma unroll
-        for (int j = 0; j < kHalf / 4; ++j) {
-            const f4 t = load4<VEC>(qrow, hf * kHalf + 4 * j, valid);
-            qreg[4 * j + 0] = t.x * a.qscale;
-            qreg[4 * j + 1] = t.y * a.qscale;
-            qreg[4 * j + 2] = t.z * a.qscale;
-            qreg[4 * j + 3] = t.w * a.qscale;
-        }
-    }
-
-    // Cooperative tile load: thread tid moves float4 number tid + 256*r of a
-    // tile (row = key within the tile, column group c).  VEC: buffer loads
-    // through a descriptor based at the tile's first row whose range ends
-    // after the sequence's last row, so rows past kv_len read as zeros
-    // without a memory access; the per-thread byte offsets are loop
-    // invariants (no address registers recycled while the loads are in
-    // flight).  Columns are clamped below head_dim (never past the row).
-    f4 kst[L::loads], vst[L::loads];
-    uint32_t voff[L::loads];
-    if constexpr (VEC) {
+        for (int c = 0; c < kC; ++c) {
+            float x[8];
 #pragma unroll
-        for (int r = 0; r < L::loads; ++r) {
-            const int f = tid + r * kThreads;
-            const int row = f / L::f4PerRow;
-            const int c = min(4 * (f % L::f4PerRow), a.head_dim - 4);
-            voff[r] = static_cast<uint32_t>((row * a.ld_kv + c) * 4);
-        }
-    }
-    auto fetch = [&](const float* base, int tile, f4* dst) {
-        if constexpr (VEC) {
-            const int64_t first = static_cast<int64_t>(tile) * kKeyTile * a.ld_kv;
-            const int rows = min(kKeyTile, a.kv_len - tile * kKeyTile);
-            const int bytes = static_cast<int>(rows * a.ld_kv * 4);
-            const __amdgpu_buffer_rsrc_t rs =
-                __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base + first), 0, bytes, kBufferWord3);
+            for (int v = 0; v < 2; ++v) {
+                const int d = 16 * c + 8 * hf + 4 * v;
+                if constexpr (VEC) {
+                    const f4 t = d < a.head_dim ? *reinterpret_cast<const f4*>(qrow + d) : f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int r = 0; r < L::loads; ++r)
-                dst[r] = __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(rs, voff[r], 0, 0));
-        } else {
+                    for (int e = 0; e < 4; ++e) x[4 * v + e] = t[e] * a.qscale;
+                } else {
 #pragma unroll
-            for (int r = 0; r < L::loads; ++r) {
-                const int f = tid + r * kThreads;
-                const int row = f / L::f4PerRow;
-                const int c = 4 * (f % L::f4PerRow);
-                const int64_t off = static_cast<int64_t>(min(tile * kKeyTile + row, a.kv_len - 1)) * a.ld_kv;
-                dst[r] = load4_clamped(base + off, c, a.head_dim);
+                    for (int e = 0; e < 4; ++e) x[4 * v + e] = d + e < a.head_dim ? qrow[d + e] * a.qscale : 0.f;
+                }
             }
+            q[c] = split8(x);
         }
-    };
-    auto stash = [&](const f4* src, int tile, float* dst, int ld) {
-#pragma unroll
-        for (int r = 0; r < L::loads; ++r) {
-            const int f = tid + r * kThreads;
-            const int row = f / L::f4PerRow;
-            const int c = 4 * (f % L::f4PerRow);
-            const bool row_ok = tile * kKeyTile + row < a.kv_len;
-            *reinterpret_cast<f4*>(dst + row * ld + c) = zero_outside(src[r], row_ok, c, a.head_dim);
-        }
-    };
-    float* const kring = lds;
-    float* const vring = lds + L::vRing;
-
-    // S^T = K Q^T over the head dimension, K from ring slot `slot`.
-    auto scores = [&](int slot) {
-        f16v s = f16v{};
-        const float* krow = kring + slot * L::kTile + li * L::kLd + hf * kHalf;
-#pragma unroll
-        for (int j = 0; j < kHalf / 4; ++j) {
-            const f4 kv = *reinterpret_cast<const f4*>(krow + 4 * j);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.x, qreg[4 * j + 0], s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.y, qreg[4 * j + 1], s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.z, qreg[4 * j + 2], s, 0, 0, 0);
-            s = __builtin_amdgcn_mfma_f32_32x32x2f32(kv.w, qreg[4 * j + 3], s, 0, 0, 0);
-        }
-        return s;
-    };
-
+    }
     f16v o[kDb];
 #pragma unroll
     for (int d = 0; d < kDb; ++d) o[d] = f16v{};
     float m_run = -1e30f;  // running max (base-2 units); the reference starts at -1e30 (LayerOps.hpp:1052)
     float l_run = 0.f;     // this half's share of the running sum
 
-    // Online softmax of one tile's scores (in place: s becomes P), rescale of
-    // O and the running sum, then O^T += V^T P^T with V from ring slot
-    // `slot`.  mask: keys at or past lane_key_end are excluded.
-    auto softmax_pv = [&](f16v& s, int slot, bool mask, int key0) {
-        if (mask) {
-            const int lim = lane_key_end - key0 - 4 * hf;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) s[r] = 8 * (r / 4) + (r % 4) < lim ? s[r] : -INFINITY;
-        }
-        float tmax = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
-        tmax = fmaxf(tmax, fmaxf(fmaxf(fmaxf(s[8], s[9]), fmaxf(s[10], s[11])),
-                                 fmaxf(fmaxf(s[12], s[13]), fmaxf(s[14], s[15]))));
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
-        const float m_new = fmaxf(m_run, tmax);
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-        m_run = m_new;
-        float psum = 0.f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            s[r] = __builtin_amdgcn_exp2f(s[r] - m_new);  // exp2(-inf) = 0: masked keys
-            psum += s[r];
-        }
-        l_run = l_run * alpha + psum;
-#pragma unroll
-        for (int d = 0; d < kDb; ++d) o[d] *= alpha;
-        const float* vl = vring + slot * L::vTile;
-        // k-slot h of step r is key(r, h) = 8*(r/4) + 4h + r%4.
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const float* vrow = vl + (8 * (r / 4) + 4 * hf + (r % 4)) * L::vLd + kDb * li;
-            if constexpr (kDb == 4) {
-                const f4 vv = *reinterpret_cast<const f4*>(vrow);
-                o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.x, s[r], o[0], 0, 0, 0);
-                o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.y, s[r], o[1], 0, 0, 0);
-                o[2] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.z, s[r], o[2], 0, 0, 0);
-                o[3] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.w, s[r], o[3], 0, 0, 0);
-            } else if constexpr (kDb == 2) {
-                const f2 vv = *reinterpret_cast<const f2*>(vrow);
-                o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.x, s[r], o[0], 0, 0, 0);
-                o[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.y, s[r], o[1], 0, 0, 0);
-            } else {
-                o[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[0], s[r], o[0], 0, 0, 0);
-            }
-        }
-    };
-
-    // Prologue: K_0, V_0 and K_1 in LDS, S_0 computed.
-    if (n_tiles > 0) {
-        fetch(kbase, 0, kst);
-        fetch(vbase, 0, vst);
-        stash(kst, 0, kring, L::kLd);
-        stash(vst, 0, vring, L::vLd);
-    }
-    if (n_tiles > 1) {
-        fetch(kbase, 1, kst);
-        stash(kst, 1, kring + L::kTile, L::kLd);
-    }
-    __syncthreads();
-    f16v s_cur = f16v{};
-    if (wave_tiles > 0) s_cur = scores(0);
-    // Iteration 0 refills K_0's slot: every wave must have read it first
-    // (later refills are ordered by the previous iteration's barrier).
+    if (n_tiles > 0) tile.stash(lds);
+    if (n_tiles > 0) tile.load(kbase, vbase, min(1, n_tiles - 1), a.ld_kv, a.kv_len, a.head_dim);
     __syncthreads();
 
     for (int t = 0; t < n_tiles; ++t) {
-        // Global loads of K_{t+2} and V_{t+1} (clamped to the last tile; the
-        // slots they fill are not read again once they would be past it).
-        fetch(kbase, min(t + 2, n_tiles - 1), kst);
-        fetch(vbase, min(t + 1, n_tiles - 1), vst);
-        if (t + 1 < wave_tiles) {
-            // S_{t+1} interleaved with the softmax of S_t; a tile before the
-            // wave's last one is never masked.
-            const f16v s_next = scores((t + 1) & 1);
-            softmax_pv(s_cur, t & 1, false, t * kKeyTile);
+        const char* cur = lds + (t & 1) * Tile::kBytes;
+        char* const next = lds + ((t + 1) & 1) * Tile::kBytes;
+        if (t < wave_tiles) {
+            f16v s = f16v{};
+            __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-            for (int i = 0; i < kHalf / 4; ++i) {
-                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);  // one LDS read (K)
-                __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);  // four score MFMAs
-                __builtin_amdgcn_sched_group_barrier(0x002, 6, 0);  // six softmax VALU ops
+            for (int c = 0; c < kC; ++c) s = mfma_split(Tile::key_rows(cur, li, hf, c), q[c], s);
+            // Past the last tile the stash rewrites a buffer that is not read
+            // again, and the load repeats the last tile.
+            tile.stash(next);
+            
+            __builtin_amdgcn_s_setprio(0);
+            tile.load(kbase, vbase, min(t + 2, n_tiles - 1), a.ld_kv, a.kv_len, a.head_dim);
+            if ((t + 1) * kKeyTile > a.kv_len || (a.causal && (t + 1) * kKeyTile - 1 > qw0)) {
+                const int lim = lane_key_end - t * kKeyTile - 4 * hf;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) s[r] = 8 * (r / 4) + (r % 4) < lim ? s[r] : -INFINITY;
             }
-            s_cur = s_next;
-        } else if (t < wave_tiles) {
-            const bool mask = (t + 1) * kKeyTile > a.kv_len || (a.causal && (t + 1) * kKeyTile - 1 > qw0);
-            if (mask) softmax_pv(s_cur, t & 1, true, t * kKeyTile);
-            else softmax_pv(s_cur, t & 1, false, t * kKeyTile);
+            float tmax = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
+            tmax = fmaxf(tmax, fmaxf(fmaxf(fmaxf(s[8], s[9]), fmaxf(s[10], s[11])),
+                                     fmaxf(fmaxf(s[12], s[13]), fmaxf(s[14], s[15]))));
+            tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+            if (__any(tmax > m_run + kMaxSlack)) {
+                const float m_new = fmaxf(m_run, tmax);
+                const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+                m_run = m_new;
+                l_run *= alpha;
+#pragma unroll
+                for (int d = 0; d < kDb; ++d) o[d] *= alpha;
+            }
+            float psum = 0.f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                s[r] = __builtin_amdgcn_exp2f(s[r] - m_run);  // exp2(-inf) = 0: masked keys
+                psum += s[r];
+            }
+            l_run += psum;
+            __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                float x[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) x[e] = s[8 * c + e];
+                const Split8 p = split8(x);
+#pragma unroll
+                for (int d = 0; d < kDb; ++d) o[d] = mfma_split(Tile::value_cols(cur, li, hf, d, c), p, o[d]);
+            }
+            
+            __builtin_amdgcn_s_setprio(0);
+        } else {
+            tile.stash(next);
+            tile.load(kbase, vbase, min(t + 2, n_tiles - 1), a.ld_kv, a.kv_len, a.head_dim);
         }
-        stash(kst, min(t + 2, n_tiles - 1), kring + (t & 1) * L::kTile, L::kLd);
-        stash(vst, min(t + 1, n_tiles - 1), vring + ((t + 1) & 1) * L::vTile, L::vLd);
         __syncthreads();
     }
 
-    // out = O / (sum + 1e-9) (LayerOps.hpp:1076-1079), rows of DP/32 dims.
-    if (my_q < a.q_len) {
-        const float l_tot = l_run + __shfl_xor(l_run, 32);
-        const float inv = 1.0f / (l_tot + 1e-9f);
-        float* orow = obase + static_cast<int64_t>(my_q) * a.ld_out;
+    // out = O / (sum + 1e-9) (LayerOps.hpp:1076-1079).
+    const float l_tot = l_run + __shfl_xor(l_run, 32);
+    const float inv = 1.0f / (l_tot + 1e-9f);
+    float check = l_tot - l_tot;
+    float* orow = obase + static_cast<int64_t>(min(my_q, a.q_len - 1)) * a.ld_out;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int d0 = kDb * (8 * (r / 4) + 4 * hf + (r % 4));
-            if (d0 >= a.head_dim) continue;
-            if constexpr (kDb == 4) {
-                const f4 val{o[0][r] * inv, o[1][r] * inv, o[2][r] * inv, o[3][r] * inv};
-                if constexpr (VEC) {
-                    *reinterpret_cast<f4*>(orow + d0) = val;
-                } else {
+    for (int d = 0; d < kDb; ++d) {
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (d0 + e < a.head_dim) orow[d0 + e] = val[e];
-                }
-            } else if constexpr (kDb == 2) {
-                orow[d0] = o[0][r] * inv;
-                if (d0 + 1 < a.head_dim) orow[d0 + 1] = o[1][r] * inv;
+        for (int r = 0; r < 16; r += 4) {
+            const int d0 = 32 * d + 8 * (r / 4) + 4 * hf;
+            const f4 val{o[d][r] * inv, o[d][r + 1] * inv, o[d][r + 2] * inv, o[d][r + 3] * inv};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) check += val[e] - val[e];
+            if (my_q >= a.q_len) continue;
+            if constexpr (VEC) {
+                if (d0 < a.head_dim) *reinterpret_cast<f4*>(orow + d0) = val;
             } else {
-                orow[d0] = o[0][r] * inv;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (d0 + e < a.head_dim) orow[d0 + e] = val[e];
             }
         }
+    }
+    // Queries that came out NaN or infinite, again in fp32: their operands
+    // may have had no bf16 split (split.hpp).
+    uint64_t redo = __ballot(check != check && my_q < a.q_len);
+    redo = (redo | redo >> 32) & 0xffffffffu;
+    while (redo) {
+        const int64_t i = qw0 + __builtin_ctzll(redo);
+        redo &= redo - 1;
+        one_query<(DP + kWave - 1) / kWave>(qbase + i * a.ld_q, kbase, vbase, obase + i * a.ld_out, a.ld_kv,
+                                            a.causal ? min(static_cast<int64_t>(a.kv_len), i + 1) : a.kv_len, a.head_dim,
+                                            a.qscale);
     }
 }
 
@@ -414,52 +430,14 @@ __global__ __launch_bounds__(kThreads, 2) void attention_fwd_mfma(AttnArgs a) {
 constexpr int kGenericWaves = 4;
 template <int CH>
 __global__ __launch_bounds__(kGenericWaves * kWave) void attention_fwd_generic(AttnArgs a) {
-    const int lane = threadIdx.x % kWave;
     const int64_t qi = static_cast<int64_t>(blockIdx.y) * kGenericWaves + threadIdx.x / kWave;
     if (qi >= a.q_len) return;  // whole waves leave: no barrier below
     const uint32_t bh = blockIdx.x;
     const int64_t b = bh / static_cast<uint32_t>(a.heads);
     const int64_t hd_off = static_cast<int64_t>(bh % static_cast<uint32_t>(a.heads)) * a.head_dim;
-    const float* qrow = a.q + (b * a.q_len + qi) * a.ld_q + hd_off;
-    const float* kb = a.k + b * a.kv_len * a.ld_kv + hd_off;
-    const float* vb = a.v + b * a.kv_len * a.ld_kv + hd_off;
-    float q[CH], acc[CH];
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-        const int d = lane + c * kWave;
-        q[c] = d < a.head_dim ? qrow[d] * a.qscale : 0.f;
-        acc[c] = 0.f;
-    }
-    const int64_t key_end = a.causal ? (qi + 1 < a.kv_len ? qi + 1 : a.kv_len) : a.kv_len;
-    float m_run = -1e30f, l_run = 0.f;
-    for (int64_t j = 0; j < key_end; ++j) {
-        const float* krow = kb + j * a.ld_kv;
-        const float* vrow = vb + j * a.ld_kv;
-        float part = 0.f;
-#pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            const int d = lane + c * kWave;
-            if (d < a.head_dim) part += q[c] * krow[d];
-        }
-        const float s = wave_sum(part);  // wave-uniform
-        const float m_new = fmaxf(m_run, s);
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-        const float p = __builtin_amdgcn_exp2f(s - m_new);
-        m_run = m_new;
-        l_run = l_run * alpha + p;
-#pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            const int d = lane + c * kWave;
-            acc[c] = acc[c] * alpha + (d < a.head_dim ? p * vrow[d] : 0.f);
-        }
-    }
-    const float inv = 1.0f / (l_run + 1e-9f);
-    float* orow = a.out + (b * a.q_len + qi) * a.ld_out + hd_off;
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-        const int d = lane + c * kWave;
-        if (d < a.head_dim) orow[d] = acc[c] * inv;
-    }
+    one_query<CH>(a.q + (b * a.q_len + qi) * a.ld_q + hd_off, a.k + b * a.kv_len * a.ld_kv + hd_off,
+                  a.v + b * a.kv_len * a.ld_kv + hd_off, a.out + (b * a.q_len + qi) * a.ld_out + hd_off, a.ld_kv,
+                  a.causal ? (qi + 1 < a.kv_len ? qi + 1 : a.kv_len) : a.kv_len, a.head_dim, a.qscale);
 }
 
 template <int CH>
@@ -470,11 +448,31 @@ int launch_generic(mimir_ctx* ctx, const AttnArgs& a, int64_t batch, int64_t hea
     return launched(ctx, "attention_fwd_generic");
 }
 
-template <int DP>
-int launch(mimir_ctx* ctx, const AttnArgs& a, bool vec) {
-    if (vec) attention_fwd_mfma<DP, true><<<a.total_blocks, kThreads, 0, ctx->stream>>>(a);
-    else attention_fwd_mfma<DP, false><<<a.total_blocks, kThreads, 0, ctx->stream>>>(a);
+template <int DP, int WAVES>
+int launch(mimir_ctx* ctx, AttnArgs a, int64_t bh, bool vec) {
+    constexpr int kThreads = WAVES * kWave;
+    a.n_qblocks = (a.q_len + kQPerWave * WAVES - 1) / (kQPerWave * WAVES);
+    const int64_t blocks = bh * a.n_qblocks;
+    MIMIR_REQUIRE(ctx, dispatch_fits(blocks, kThreads), "attention: grid of %lld workgroups exceeds the limit",
+                  (long long)blocks);
+    a.total_blocks = static_cast<uint32_t>(blocks);
+    if (vec) attention_fwd_mfma<DP, WAVES, true><<<a.total_blocks, kThreads, 0, ctx->stream>>>(a);
+    else attention_fwd_mfma<DP, WAVES, false><<<a.total_blocks, kThreads, 0, ctx->stream>>>(a);
     return launched(ctx, "attention_fwd_mfma");
+}
+
+template <int DP>
+int launch_mfma(mimir_ctx* ctx, const AttnArgs& a, int64_t bh, bool vec) {
+    // Eight waves split a tile once for 256 queries; four keep more of the
+    // GPU busy while one workgroup per CU holds all of them.  Measured on
+    // MI355X (4 / 8 waves, us): 8 x 32 heads x 1024 x 128 causal 508 / 395,
+    // 16 heads x 1024 x 128 causal 99 / 120, 16 x 2048 x 64 causal 107 / 134,
+    // 96 x 333 x 777 x 80 136 / 78.  Few queries (40 against 1500 keys): the
+    // tile's way in is the work, 142 / 122.
+    const int64_t blocks4 = bh * ((a.q_len + 4 * kQPerWave - 1) / (4 * kQPerWave));
+    int waves = blocks4 <= 256 && a.q_len > 64 ? 4 : 8;
+    if (ctx->tune.attn_waves == 4 || ctx->tune.attn_waves == 8) waves = ctx->tune.attn_waves;
+    return waves == 4 ? launch<DP, 4>(ctx, a, bh, vec) : launch<DP, 8>(ctx, a, bh, vec);
 }
 
 }  // namespace
@@ -498,9 +496,6 @@ int mimir_attention_fwd(mimir_ctx* ctx, const float* q, int64_t ld_q, const floa
     MIMIR_REQUIRE(ctx, std::isfinite(scale), "attention: scale must be finite");
     if (batch == 0 || q_len == 0) return MIMIR_OK;
     MIMIR_REQUIRE(ctx, q && out && (kv_len == 0 || (k && v)), "attention: null pointer");
-    const int64_t nqb = (q_len + kQPerBlock - 1) / kQPerBlock;
-    MIMIR_REQUIRE(ctx, dispatch_fits(batch * heads * nqb, kThreads), "attention: grid of %lld workgroups exceeds the limit",
-                  (long long)(batch * heads * nqb));
     if (int st = enter(ctx)) return st;
     AttnArgs a;
     a.q = q;
@@ -514,23 +509,25 @@ int mimir_attention_fwd(mimir_ctx* ctx, const float* q, int64_t ld_q, const floa
     a.kv_len = static_cast<int32_t>(kv_len);
     a.heads = static_cast<int32_t>(heads);
     a.head_dim = static_cast<int32_t>(head_dim);
-    a.n_qblocks = static_cast<int32_t>(nqb);
-    a.total_blocks = static_cast<uint32_t>(batch * heads * nqb);
+    a.n_qblocks = 0;
+    a.total_blocks = 0;
     a.qscale = scale * kLog2e;
     a.causal = causal ? 1 : 0;
-    // The vector path's buffer descriptors span one 32-row tile: 32 rows of
-    // ld_kv floats must stay below 2^31 bytes.
     const bool vec = head_dim % 4 == 0 && ld_q % 4 == 0 && ld_kv % 4 == 0 && ld_out % 4 == 0 && aligned16(q) &&
-                     aligned16(a.k) && aligned16(a.v) && aligned16(out) &&
-                     ld_kv < (int64_t{1} << 31) / (4 * kKeyTile);
+                     aligned16(a.k) && aligned16(a.v) && aligned16(out);
     // Few queries: each key row is read once by vector code, where the
     // matrix-core kernel would use one of its waves (attention_decode.hip).
     if (attention_decode_applies(q_len, kv_len, head_dim, a.causal))
         return attention_decode_launch(ctx, q, ld_q, a.k, a.v, ld_kv, out, ld_out, batch, q_len, kv_len, heads, head_dim,
                                        a.qscale, vec);
-    if (head_dim <= 32) return launch<32>(ctx, a, vec);
-    if (head_dim <= 64) return launch<64>(ctx, a, vec);
-    if (head_dim <= 128) return launch<128>(ctx, a, vec);
+    // The tile's buffer descriptors span 32 rows of ld_kv floats: below 2^31
+    // bytes, or the wide-head kernel.
+    if (ld_kv < (int64_t{1} << 31) / (4 * kKeyTile)) {
+        if (head_dim <= 32) return launch_mfma<32>(ctx, a, batch * heads, vec);
+        if (head_dim <= 64) return launch_mfma<64>(ctx, a, batch * heads, vec);
+        if (head_dim <= 96) return launch_mfma<96>(ctx, a, batch * heads, vec);
+        if (head_dim <= 128) return launch_mfma<128>(ctx, a, batch * heads, vec);
+    }
     MIMIR_REQUIRE(ctx, dispatch_fits(batch * heads, kGenericWaves * kWave) && (q_len + kGenericWaves - 1) / kGenericWaves <= 65535,
                   "attention: grid exceeds the limit of the wide-head kernel");
     if (head_dim <= 256) return launch_generic<4>(ctx, a, batch, heads);

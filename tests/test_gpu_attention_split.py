@@ -1,0 +1,62 @@
+"""The matrix-core attention core with fp32 operands split into bf16 terms:
+both workgroup sizes at the edges of their query blocks and key tiles, every
+padded head size, and values that have no split (infinities, NaN, the largest
+floats), against float64."""
+import numpy as np
+import pytest
+
+import oracle as O
+from _attention import assert_attention_close, attention64
+from test_gpu_attention import gpu_attention, rand_qkv
+
+pytestmark = pytest.mark.gpu
+
+# 128-query workgroups up to 256 of them, 256-query ones above (and for up to
+# 64 queries); 32-key tiles; heads padded to 32, 64, 96 and 128.
+SHAPES = [(1, 65, 31, 2, 32), (1, 128, 32, 1, 64), (2, 129, 33, 2, 36), (1, 257, 257, 2, 96), (1, 300, 64, 1, 100),
+          (1, 97, 160, 2, 70), (1, 70, 70, 3, 5), (40, 130, 70, 8, 32), (33, 257, 66, 8, 16), (1, 9, 95, 2, 128),
+          (1, 64, 65, 1, 128)]
+
+
+@pytest.mark.parametrize("b,lq,lk,heads,hd", SHAPES)
+@pytest.mark.parametrize("causal", [False, True])
+def test_split_core(ctx, b, lq, lk, heads, hd, causal):
+    q, k, v = rand_qkv(lq + lk + hd, b, lq, lk, heads * hd)
+    got = gpu_attention(ctx, q, k, v, heads, causal)
+    for i in range(0, b, max(1, b // 3)):
+        out, mag, cond = attention64(q[i], k[i], v[i], heads, causal, O.attention_scale(hd))
+        assert_attention_close(got[i], out, mag, cond, f"split core {b} {lq} {lk} {heads} {hd} {causal} [{i}]")
+
+
+@pytest.mark.parametrize("lq,lk", [(70, 100), (300, 300)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_split_core_special_values(ctx, lq, lk, causal):
+    """What fp32 arithmetic gives: -inf scores weigh nothing, an infinite
+    value reaches its dimension of the queries that see it, a NaN key every
+    query that sees it, and masked keys nothing at all."""
+    q, k, v = rand_qkv(3, 1, lq, lk, 64)
+    q[0, :, 3] = np.abs(q[0, :, 3]) + 0.5
+    k[0, 7, 3] = -np.inf
+    v[0, 40, 5] = np.inf
+    v[0, 41, 6] = 3.4e38  # rounds to infinity in bf16
+    k[0, 60, 8] = np.nan
+    got = gpu_attention(ctx, q, k, v, 1, causal)[0]
+    s = (q[0].astype(np.float64) @ k[0].astype(np.float64).T) * O.attention_scale(64)
+    hide = np.triu(np.ones(s.shape, bool), 1) if causal else np.zeros(s.shape, bool)
+    s[hide] = -np.inf
+    p = np.exp(s - np.nanmax(s, 1, keepdims=True))
+    p /= p.sum(1, keepdims=True)
+    seen = ~hide
+    bad = seen[:, 60]
+    assert np.isnan(got[bad]).all(), "a NaN key"
+    fine = ~bad
+    v64 = np.where(np.isfinite(v[0]), v[0], 0.0).astype(np.float64)
+    keep = [d for d in range(64) if d not in (5, 6)]
+    want = np.where(np.isnan(p), 0.0, p) @ v64
+    np.testing.assert_allclose(got[fine][:, keep], want[fine][:, keep], rtol=0, atol=1e-5)
+    inf = fine & seen[:, 40]
+    assert np.isposinf(got[inf, 5]).all(), "an infinite value"
+    big = fine & seen[:, 41]
+    np.testing.assert_allclose(got[big, 6], want[big, 6], rtol=1e-4)
+    clean = fine & ~seen[:, 40]
+    np.testing.assert_allclose(got[clean][:, 5:7], want[clean][:, 5:7], rtol=0, atol=1e-5)
