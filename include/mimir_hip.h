@@ -282,12 +282,12 @@ int mimir_cross_attention_fwd(mimir_ctx* ctx, const float* query_input, int64_t 
  * with P the core's probabilities (causal j > i masked to -1e9, max from
  * -1e30, p = e / (sum + 1e-9)).  dq rows have ld_dq, dk and dv rows ld_dkv
  * (dk and dv may be column blocks of one buffer, as the reference's dqkv).
- * Overwrites dq / dk / dv.  P and dS are materialised per group of heads
- * in the context's scratch (2 q_len kv_len floats per head, groups capped at
- * 1 GiB, one head at least), beside K^T and V^T of one sequence (2 kv_len
- * heads head_dim floats); the products are fp32 library GEMMs, the row
- * passes (mask + softmax, softmax backward) and the transposes hand-written
- * kernels.
+ * Overwrites dq / dk / dv.  Scratch (the context's), heads up to 128: dS in
+ * 32 x 32 blocks per group of (sequence, head) pairs (q_len kv_len floats per
+ * pair, groups capped at 512 MiB, one pair at least), three floats per query
+ * and, where few pairs share the GPU, partial results.  Wider heads: P and dS
+ * per group of heads (2 q_len kv_len floats per head, groups capped at 1 GiB)
+ * with library GEMMs and their operands' copies.
  * kv_len == 0: dq = 0.  Outputs must not overlap the inputs. */
 int mimir_attention_bwd(mimir_ctx* ctx, const float* q, int64_t ld_q, const float* k, const float* v,
                         int64_t ld_kv, const float* dout, int64_t ld_dout, float* dq, int64_t ld_dq, float* dk,

@@ -52,12 +52,13 @@
 // turns, LDS reads ordered ahead of the MFMAs, the split interleaved with them,
 // raised priority for half the waves; four waves with two workgroups' worth of
 // LDS are slower (the tile is split twice as often).
+#include "attention_tile.hpp"
 #include "common.hpp"
 #include "internal.hpp"
-#include "split.hpp"
 
 #include <math.h>
 
+#include <algorithm>
 #include <cmath>
 
 using namespace mimir;
@@ -72,6 +73,8 @@ constexpr float kLog2e = 1.4426950408889634f;
 // probabilities up to 2^8 of the final scale lose nothing in fp32, and the
 // rescale of the output (DP / 2 multiplies) runs in few tiles instead of most.
 constexpr float kMaxSlack = 8.0f;
+// Workgroups of eight waves that fill the GPU.
+constexpr int64_t kSplitTarget = 256;
 
 struct AttnArgs {
     const float* q;
@@ -84,7 +87,26 @@ struct AttnArgs {
     uint32_t total_blocks;        // batch * heads * n_qblocks
     float qscale;                 // scale * log2(e), applied to Q
     int32_t causal;
+    // For the backward (STATS): the gradient of the output, and per query of
+    // each (sequence, head), in rows of stats_ld queries, the running max,
+    // 1 / (sum + 1e-9) and sum_d out_d dout_d.  out may be null then.
+    const float* dout;
+    int64_t ld_dout;
+    float* stats;
+    int64_t stats_ld;
+    uint32_t bh0;                 // first (sequence, head) of the launch
+    // Keys dealt to several workgroups: partial results [split][n_bh][q_len]
+    // [head_dim | max | sum], null: one workgroup per query block.
+    int32_t splits;
+    float* part;
 };
+
+// Key tiles that a query block (queries q0 .. q0 + n) streams, and how many a
+// split takes.
+__device__ __forceinline__ int tiles_of(const AttnArgs& a, int q0, int n) {
+    const int end = a.causal ? min(a.kv_len, min(q0 + n, a.q_len)) : a.kv_len;
+    return (end + kKeyTile - 1) / kKeyTile;
+}
 
 // Workgroup -> (sequence * heads + head, query block): see the file comment.
 __device__ __forceinline__ void block_coords(const AttnArgs& a, uint32_t bid, uint32_t* bh, int* qb) {
@@ -103,168 +125,79 @@ __device__ __forceinline__ void block_coords(const AttnArgs& a, uint32_t bid, ui
 // lanes (CH per lane, lane + 64 c): each score a DPP wave sum, the same online
 // softmax and the same division by (sum + 1e-9).
 template <int CH>
-__device__ __forceinline__ void one_query(const float* qrow, const float* kb, const float* vb, float* orow,
-                                          int64_t ld_kv, int64_t keys, int head_dim, float qscale) {
-    const int lane = threadIdx.x % kWave;
-    float q[CH], acc[CH];
+struct OneQuery {
+    float acc[CH], m, inv;
+    __device__ __forceinline__ OneQuery(const float* qrow, const float* kb, const float* vb, int64_t ld_kv, int64_t keys,
+                                        int head_dim, float qscale) {
+        const int lane = threadIdx.x % kWave;
+        float q[CH];
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
-        const int d = lane + c * kWave;
-        q[c] = d < head_dim ? qrow[d] * qscale : 0.f;
-        acc[c] = 0.f;
+        for (int c = 0; c < CH; ++c) {
+            const int d = lane + c * kWave;
+            q[c] = d < head_dim ? qrow[d] * qscale : 0.f;
+            acc[c] = 0.f;
+        }
+        float l = 0.f;
+        m = -1e30f;
+        for (int64_t j = 0; j < keys; ++j) {
+            const float* krow = kb + j * ld_kv;
+            const float* vrow = vb + j * ld_kv;
+            float part = 0.f;
+#pragma unroll
+            for (int c = 0; c < CH; ++c) {
+                const int d = lane + c * kWave;
+                if (d < head_dim) part += q[c] * krow[d];
+            }
+            const float s = wave_sum(part);  // wave-uniform
+            const float m_new = fmaxf(m, s);
+            const float alpha = __builtin_amdgcn_exp2f(m - m_new);
+            const float p = __builtin_amdgcn_exp2f(s - m_new);
+            m = m_new;
+            l = l * alpha + p;
+#pragma unroll
+            for (int c = 0; c < CH; ++c) {
+                const int d = lane + c * kWave;
+                acc[c] = acc[c] * alpha + (d < head_dim ? p * vrow[d] : 0.f);
+            }
+        }
+        inv = 1.0f / (l + 1e-9f);
+#pragma unroll
+        for (int c = 0; c < CH; ++c) acc[c] *= inv;
     }
-    float m_run = -1e30f, l_run = 0.f;
-    for (int64_t j = 0; j < keys; ++j) {
-        const float* krow = kb + j * ld_kv;
-        const float* vrow = vb + j * ld_kv;
+    __device__ __forceinline__ void store(float* row, int head_dim) const {
+        const int lane = threadIdx.x % kWave;
+#pragma unroll
+        for (int c = 0; c < CH; ++c)
+            if (lane + c * kWave < head_dim) row[lane + c * kWave] = acc[c];
+    }
+    __device__ __forceinline__ float dot(const float* row, int head_dim) const {
+        const int lane = threadIdx.x % kWave;
         float part = 0.f;
 #pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            const int d = lane + c * kWave;
-            if (d < head_dim) part += q[c] * krow[d];
-        }
-        const float s = wave_sum(part);  // wave-uniform
-        const float m_new = fmaxf(m_run, s);
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-        const float p = __builtin_amdgcn_exp2f(s - m_new);
-        m_run = m_new;
-        l_run = l_run * alpha + p;
-#pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            const int d = lane + c * kWave;
-            acc[c] = acc[c] * alpha + (d < head_dim ? p * vrow[d] : 0.f);
-        }
-    }
-    const float inv = 1.0f / (l_run + 1e-9f);
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-        const int d = lane + c * kWave;
-        if (d < head_dim) orow[d] = acc[c] * inv;
-    }
-}
-
-// A tile of 32 keys on its way from memory to LDS.  Items of eight values: K
-// item = (key, eight dimensions), V item = (dimension, eight keys in the order
-// of the file comment); 4 * DP of each, dealt to THREADS threads.  Loads go
-// through a descriptor that starts at the tile's first row and ends after the
-// sequence's last, so rows past kv_len read as zeros; columns are clamped into
-// the head (past head_dim, Q is zero and the output is not stored).
-// VEC: K moves in 16-byte loads (head_dim, the stride and the base pointer are
-// 16-byte multiples).
-template <int DP, int THREADS, bool VEC>
-struct KvTile {
-    static constexpr int kKeyBytes = 2 * DP + 16, kDimBytes = 2 * kKeyTile + 16;
-    static constexpr int kKPlane = kKeyTile * kKeyBytes, kVPlane = DP * kDimBytes;
-    static constexpr int kBytes = 3 * (kKPlane + kVPlane);
-    static constexpr int kKind = 4 * DP;  // items of each kind
-    static constexpr int kItems = (kKind + THREADS - 1) / THREADS;
-    static constexpr int kSpare = kItems * THREADS - kKind;  // threads without an item of one kind
-    float k[kItems][8], v[kItems][8];
-    uint32_t koff[kItems], voff[kItems];  // byte offsets of an item's first element
-    int32_t kstep[kItems];                // VEC: bytes from the first four to the second four of a K item
-    uint32_t ld4;
-
-    // Where the items do not fill the threads, the first ones take K and the
-    // last ones V.
-    static __device__ __forceinline__ int k_item(int j) { return static_cast<int>(threadIdx.x) + j * THREADS; }
-    static __device__ __forceinline__ int v_item(int j) { return k_item(j) - kSpare; }
-    static __device__ __forceinline__ int wave_start() {
-        return __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x)) & ~(kWave - 1);
-    }
-    static __device__ __forceinline__ bool has_k(int j) { return kSpare == 0 || wave_start() + j * THREADS < kKind; }
-    static __device__ __forceinline__ bool has_v(int j) { return kSpare == 0 || wave_start() + j * THREADS >= kSpare; }
-
-    __device__ __forceinline__ void init(int64_t ld, int head_dim) {
-        ld4 = static_cast<uint32_t>(ld * 4);
-#pragma unroll
-        for (int j = 0; j < kItems; ++j) {
-            const int ki = min(k_item(j), kKind - 1), key = ki / (DP / 8), d = 8 * (ki % (DP / 8));
-            if constexpr (VEC) {
-                koff[j] = key * ld4 + 4 * min(d, head_dim - 4);
-                kstep[j] = 4 * (min(d + 4, head_dim - 4) - min(d, head_dim - 4));
-            } else {
-                koff[j] = key * ld4 + 4 * d;
-            }
-            const int vi = max(v_item(j), 0), group = vi / DP;
-            voff[j] = 4 * min(vi % DP, head_dim - 1) + (16 * (group / 2) + 4 * (group % 2)) * ld4;
-        }
-    }
-    __device__ __forceinline__ void load(const float* kbase, const float* vbase, int tile, int64_t ld, int kv_len,
-                                         int head_dim) {
-        const int64_t first = static_cast<int64_t>(tile) * kKeyTile * ld;
-        const int rows = min(kKeyTile, kv_len - tile * kKeyTile);
-        // The last row ends with the head, not with the stride.
-        const int bytes = static_cast<int>((rows - 1) * ld4 + 4 * head_dim);
-        const __amdgpu_buffer_rsrc_t rk = buffer_of(kbase + first, bytes), rv = buffer_of(vbase + first, bytes);
-#pragma unroll
-        for (int j = 0; j < kItems; ++j) {
-            if (has_k(j)) {
-                if constexpr (VEC) {
-                    const f4 a = buffer_f4(rk, koff[j]), b = buffer_f4(rk, koff[j] + kstep[j]);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        k[j][e] = a[e];
-                        k[j][4 + e] = b[e];
-                    }
-                } else {
-                    const int d = 8 * (k_item(j) % (DP / 8));
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) k[j][e] = buffer_f1(rk, koff[j] + 4 * (min(d + e, head_dim - 1) - d));
-                }
-            }
-            if (has_v(j)) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) v[j][e] = buffer_f1(rv, voff[j] + ((e & 3) + 8 * (e >> 2)) * ld4);
-            }
-        }
-    }
-    __device__ __forceinline__ void stash(char* lds) const {
-#pragma unroll
-        for (int j = 0; j < kItems; ++j) {
-            if (has_k(j)) {
-                const int id = k_item(j);
-                char* p = lds + id / (DP / 8) * kKeyBytes + id % (DP / 8) * 16;
-                const Split8 s = split8(k[j]);
-                *reinterpret_cast<u4*>(p) = s.h;
-                *reinterpret_cast<u4*>(p + kKPlane) = s.m;
-                *reinterpret_cast<u4*>(p + 2 * kKPlane) = s.l;
-            }
-            if (has_v(j)) {
-                const int id = v_item(j);
-                char* p = lds + 3 * kKPlane + id % DP * kDimBytes + id / DP * 16;
-                const Split8 s = split8(v[j]);
-                *reinterpret_cast<u4*>(p) = s.h;
-                *reinterpret_cast<u4*>(p + kVPlane) = s.m;
-                *reinterpret_cast<u4*>(p + 2 * kVPlane) = s.l;
-            }
-        }
-    }
-    // MFMA operands: dimensions 16 c + 8 hf .. + 7 of key li; the eight keys
-    // (c, hf) of dimension 32 db + li.
-    static __device__ __forceinline__ Split8 key_rows(const char* lds, int li, int hf, int c) {
-        const char* p = lds + li * kKeyBytes + 32 * c + 16 * hf;
-        return Split8{*reinterpret_cast<const u4*>(p), *reinterpret_cast<const u4*>(p + kKPlane),
-                      *reinterpret_cast<const u4*>(p + 2 * kKPlane)};
-    }
-    static __device__ __forceinline__ Split8 value_cols(const char* lds, int li, int hf, int db, int c) {
-        const char* p = lds + 3 * kKPlane + (32 * db + li) * kDimBytes + 32 * c + 16 * hf;
-        return Split8{*reinterpret_cast<const u4*>(p), *reinterpret_cast<const u4*>(p + kVPlane),
-                      *reinterpret_cast<const u4*>(p + 2 * kVPlane)};
+        for (int c = 0; c < CH; ++c)
+            if (lane + c * kWave < head_dim) part += acc[c] * row[lane + c * kWave];
+        return wave_sum(part);
     }
 };
 
-template <int DP, int WAVES, bool VEC>
+// STATS: for the backward, which needs every query's max, sum and
+// out . dout instead of (or beside) the output.
+template <int DP, int WAVES, bool VEC, bool STATS>
 __global__ __launch_bounds__(WAVES * kWave, WAVES > 4 ? 2 : 1) void attention_fwd_mfma(AttnArgs a) {
-    using Tile = KvTile<DP, WAVES * kWave, VEC>;
+    using Keys = RowTile<DP, WAVES * kWave, VEC>;
+    using Values = ColTile<DP, WAVES * kWave>;
+    constexpr int kBuf = Keys::kBytes + Values::kBytes;
     constexpr int kC = DP / 16;   // MFMA steps of a score
     constexpr int kDb = DP / 32;  // output dimension blocks
-    __shared__ __attribute__((aligned(16))) char lds[2 * Tile::kBytes];
+    __shared__ __attribute__((aligned(16))) char lds[2 * kBuf];
 
     uint32_t bh;
     int qb;
-    block_coords(a, blockIdx.x, &bh, &qb);
-    const int64_t b = bh / static_cast<uint32_t>(a.heads);
-    const int64_t hd_off = static_cast<int64_t>(bh % static_cast<uint32_t>(a.heads)) * a.head_dim;
+    const int split = static_cast<int>(blockIdx.x % static_cast<uint32_t>(a.splits));
+    block_coords(a, blockIdx.x / static_cast<uint32_t>(a.splits), &bh, &qb);
+    const uint32_t head = a.bh0 + bh;
+    const int64_t b = head / static_cast<uint32_t>(a.heads);
+    const int64_t hd_off = static_cast<int64_t>(head % static_cast<uint32_t>(a.heads)) * a.head_dim;
     const float* qbase = a.q + b * a.q_len * a.ld_q + hd_off;
     const float* kbase = a.k + b * a.kv_len * a.ld_kv + hd_off;
     const float* vbase = a.v + b * a.kv_len * a.ld_kv + hd_off;
@@ -278,69 +211,61 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES > 4 ? 2 : 1) void attention_fw
     const int my_q = qw0 + li;
 
     // Tiles this workgroup streams, and the ones this wave computes.
-    int key_end = a.kv_len;
-    int wave_key_end = a.kv_len;
-    if (a.causal) {
-        key_end = min(key_end, min(q0 + kQPerWave * WAVES, a.q_len));
-        wave_key_end = min(wave_key_end, min(qw0 + kQPerWave, a.q_len));
-    }
+    int wave_key_end = a.causal ? min(a.kv_len, min(qw0 + kQPerWave, a.q_len)) : a.kv_len;
     if (qw0 >= a.q_len) wave_key_end = 0;
-    const int n_tiles = (key_end + kKeyTile - 1) / kKeyTile;
-    const int wave_tiles = (wave_key_end + kKeyTile - 1) / kKeyTile;
+    const int all_tiles = tiles_of(a, q0, kQPerWave * WAVES);
+    const int per = (all_tiles + a.splits - 1) / a.splits;
+    const int t0 = split * per;
+    const int n_tiles = min(t0 + per, all_tiles);
+    if (split > 0 && t0 >= n_tiles) return;
+    const int wave_tiles = min(n_tiles, (wave_key_end + kKeyTile - 1) / kKeyTile);
     // Keys of this lane's query: the rest of its last tile is masked
     // (causal: key > query; all: key >= kv_len).
     const int lane_key_end = min(a.kv_len, a.causal ? my_q + 1 : a.kv_len);
 
-    Tile tile;
-    tile.init(a.ld_kv, a.head_dim);
-    if (n_tiles > 0) tile.load(kbase, vbase, 0, a.ld_kv, a.kv_len, a.head_dim);
+    Keys keys;
+    Values values;
+    keys.init(a.ld_kv, a.head_dim);
+    values.init(a.ld_kv, a.head_dim);
+    auto load = [&](int t) {
+        keys.load(kbase, t, a.ld_kv, a.kv_len, a.head_dim);
+        values.load(vbase, t, a.ld_kv, a.kv_len, a.head_dim);
+    };
+    auto stash = [&](char* buf) {
+        keys.stash(buf);
+        values.stash(buf + Keys::kBytes);
+    };
+    if (n_tiles > t0) load(t0);
 
-    // This lane's Q values, times scale*log2(e), zero past head_dim.
+    // This lane's Q values, times scale*log2(e).
     Split8 q[kC];
-    {
-        const float* qrow = qbase + static_cast<int64_t>(min(my_q, a.q_len - 1)) * a.ld_q;
-#pragma unroll
-        for (int c = 0; c < kC; ++c) {
-            float x[8];
-#pragma unroll
-            for (int v = 0; v < 2; ++v) {
-                const int d = 16 * c + 8 * hf + 4 * v;
-                if constexpr (VEC) {
-                    const f4 t = d < a.head_dim ? *reinterpret_cast<const f4*>(qrow + d) : f4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) x[4 * v + e] = t[e] * a.qscale;
-                } else {
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) x[4 * v + e] = d + e < a.head_dim ? qrow[d + e] * a.qscale : 0.f;
-                }
-            }
-            q[c] = split8(x);
-        }
-    }
+    row_operand<DP, VEC>(qbase + static_cast<int64_t>(min(my_q, a.q_len - 1)) * a.ld_q, hf, a.head_dim, a.qscale, q);
     f16v o[kDb];
 #pragma unroll
     for (int d = 0; d < kDb; ++d) o[d] = f16v{};
     float m_run = -1e30f;  // running max (base-2 units); the reference starts at -1e30 (LayerOps.hpp:1052)
     float l_run = 0.f;     // this half's share of the running sum
 
-    if (n_tiles > 0) tile.stash(lds);
-    if (n_tiles > 0) tile.load(kbase, vbase, min(1, n_tiles - 1), a.ld_kv, a.kv_len, a.head_dim);
+    if (n_tiles > t0) {
+        stash(lds);
+        load(min(t0 + 1, n_tiles - 1));
+    }
     __syncthreads();
 
-    for (int t = 0; t < n_tiles; ++t) {
-        const char* cur = lds + (t & 1) * Tile::kBytes;
-        char* const next = lds + ((t + 1) & 1) * Tile::kBytes;
+    for (int t = t0; t < n_tiles; ++t) {
+        const char* cur = lds + ((t - t0) & 1) * kBuf;
+        char* const next = lds + ((t - t0 + 1) & 1) * kBuf;
         if (t < wave_tiles) {
             f16v s = f16v{};
             __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-            for (int c = 0; c < kC; ++c) s = mfma_split(Tile::key_rows(cur, li, hf, c), q[c], s);
+            for (int c = 0; c < kC; ++c) s = mfma_split(Keys::at(cur, li, hf, c), q[c], s);
             // Past the last tile the stash rewrites a buffer that is not read
             // again, and the load repeats the last tile.
-            tile.stash(next);
+            stash(next);
             
             __builtin_amdgcn_s_setprio(0);
-            tile.load(kbase, vbase, min(t + 2, n_tiles - 1), a.ld_kv, a.kv_len, a.head_dim);
+            load(min(t + 2, n_tiles - 1));
             if ((t + 1) * kKeyTile > a.kv_len || (a.causal && (t + 1) * kKeyTile - 1 > qw0)) {
                 const int lim = lane_key_end - t * kKeyTile - 4 * hf;
 #pragma unroll
@@ -373,13 +298,13 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES > 4 ? 2 : 1) void attention_fw
                 for (int e = 0; e < 8; ++e) x[e] = s[8 * c + e];
                 const Split8 p = split8(x);
 #pragma unroll
-                for (int d = 0; d < kDb; ++d) o[d] = mfma_split(Tile::value_cols(cur, li, hf, d, c), p, o[d]);
+                for (int d = 0; d < kDb; ++d) o[d] = mfma_split(Values::at(cur + Keys::kBytes, li, hf, d, c), p, o[d]);
             }
             
             __builtin_amdgcn_s_setprio(0);
         } else {
-            tile.stash(next);
-            tile.load(kbase, vbase, min(t + 2, n_tiles - 1), a.ld_kv, a.kv_len, a.head_dim);
+            stash(next);
+            load(min(t + 2, n_tiles - 1));
         }
         __syncthreads();
     }
@@ -387,36 +312,127 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES > 4 ? 2 : 1) void attention_fw
     // out = O / (sum + 1e-9) (LayerOps.hpp:1076-1079).
     const float l_tot = l_run + __shfl_xor(l_run, 32);
     const float inv = 1.0f / (l_tot + 1e-9f);
-    float check = l_tot - l_tot;
-    float* orow = obase + static_cast<int64_t>(min(my_q, a.q_len - 1)) * a.ld_out;
+    const bool in = my_q < a.q_len;
+    const int64_t row = min(my_q, a.q_len - 1);
+    const uint32_t n_bh = a.total_blocks / static_cast<uint32_t>(a.n_qblocks);
+    if (a.part) {
+        float* p = a.part + ((split * static_cast<int64_t>(n_bh) + bh) * a.q_len + row) * (a.head_dim + 2);
+        store_columns<DP, false>(o, 1.0f, p, in, hf, a.head_dim);
+        if (in && hf == 0) {
+            p[a.head_dim] = m_run;
+            p[a.head_dim + 1] = l_tot;
+        }
+        return;
+    }
+    float check = store_columns<DP, VEC>(o, inv, a.out ? obase + row * a.ld_out : nullptr, in && a.out, hf, a.head_dim);
+    check += l_tot - l_tot;
+    float* const stats = STATS ? a.stats + bh * a.stats_ld : nullptr;
+    const int64_t plane = n_bh * a.stats_ld;
+    const float* const dobase = STATS ? a.dout + b * a.q_len * a.ld_dout + hd_off : nullptr;
+    if constexpr (STATS) {
+        float dot = 0.f;
 #pragma unroll
-    for (int d = 0; d < kDb; ++d) {
+        for (int d = 0; d < kDb; ++d)
 #pragma unroll
-        for (int r = 0; r < 16; r += 4) {
-            const int d0 = 32 * d + 8 * (r / 4) + 4 * hf;
-            const f4 val{o[d][r] * inv, o[d][r + 1] * inv, o[d][r + 2] * inv, o[d][r + 3] * inv};
-#pragma unroll
-            for (int e = 0; e < 4; ++e) check += val[e] - val[e];
-            if (my_q >= a.q_len) continue;
-            if constexpr (VEC) {
-                if (d0 < a.head_dim) *reinterpret_cast<f4*>(orow + d0) = val;
-            } else {
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (d0 + e < a.head_dim) orow[d0 + e] = val[e];
+            for (int r = 0; r < 16; ++r) {
+                const int dim = 32 * d + 8 * (r / 4) + 4 * hf + r % 4;
+                if (dim < a.head_dim) dot += o[d][r] * inv * dobase[row * a.ld_dout + dim];
             }
+        dot += __shfl_xor(dot, 32);
+        // Rows past the sequence, up to the tile's end: no weight.
+        if (hf == 0 && my_q < a.stats_ld) {
+            stats[my_q] = in ? m_run : 0.f;
+            stats[plane + my_q] = in ? inv : 0.f;
+            stats[2 * plane + my_q] = in ? dot : 0.f;
         }
     }
     // Queries that came out NaN or infinite, again in fp32: their operands
     // may have had no bf16 split (split.hpp).
-    uint64_t redo = __ballot(check != check && my_q < a.q_len);
-    redo = (redo | redo >> 32) & 0xffffffffu;
-    while (redo) {
-        const int64_t i = qw0 + __builtin_ctzll(redo);
-        redo &= redo - 1;
-        one_query<(DP + kWave - 1) / kWave>(qbase + i * a.ld_q, kbase, vbase, obase + i * a.ld_out, a.ld_kv,
-                                            a.causal ? min(static_cast<int64_t>(a.kv_len), i + 1) : a.kv_len, a.head_dim,
-                                            a.qscale);
+    for (uint32_t redo = bad_rows(check, in); redo; redo &= redo - 1) {
+        const int64_t i = qw0 + __builtin_ctz(redo);
+        const OneQuery<(DP + kWave - 1) / kWave> one(qbase + i * a.ld_q, kbase, vbase, a.ld_kv,
+                                                     a.causal ? min(static_cast<int64_t>(a.kv_len), i + 1) : a.kv_len,
+                                                     a.head_dim, a.qscale);
+        if (a.out) one.store(obase + i * a.ld_out, a.head_dim);
+        if constexpr (STATS) {
+            const float dot = one.dot(dobase + i * a.ld_dout, a.head_dim);
+            if (lane == 0) {
+                stats[i] = one.m;
+                stats[plane + i] = one.inv;
+                stats[2 * plane + i] = dot;
+            }
+        }
+    }
+}
+
+// The splits of one query, one wave per query: their sums brought to one max,
+// then what attention_fwd_mfma does with the whole.
+template <bool STATS>
+__global__ __launch_bounds__(4 * kWave) void attention_fwd_combine(AttnArgs a, int queries_per_block) {
+    constexpr int kCh = 2;  // heads up to 128
+    const uint32_t n_bh = a.total_blocks / static_cast<uint32_t>(a.n_qblocks);
+    const int64_t rows = STATS ? a.stats_ld : a.q_len;
+    const int64_t at = static_cast<int64_t>(blockIdx.x) * 4 + threadIdx.x / kWave;
+    if (at >= n_bh * rows) return;  // whole waves
+    const int lane = threadIdx.x % kWave;
+    const uint32_t bh = static_cast<uint32_t>(at / rows);
+    const int64_t i = at % rows;
+    float* const stats = STATS ? a.stats + bh * a.stats_ld + i : nullptr;
+    const int64_t plane = n_bh * a.stats_ld;
+    if (i >= a.q_len) {  // up to the tile's end: no weight
+        if constexpr (STATS)
+            if (lane < 3) stats[lane * plane] = 0.f;
+        return;
+    }
+    const uint32_t head = a.bh0 + bh;
+    const int64_t b = head / static_cast<uint32_t>(a.heads);
+    const int64_t hd_off = static_cast<int64_t>(head % static_cast<uint32_t>(a.heads)) * a.head_dim;
+    const int w = a.head_dim + 2;
+    const float* p = a.part + (static_cast<int64_t>(bh) * a.q_len + i) * w;
+    const int64_t next = static_cast<int64_t>(n_bh) * a.q_len * w;
+    const int all = tiles_of(a, static_cast<int>(i / queries_per_block) * queries_per_block, queries_per_block);
+    const int per = (all + a.splits - 1) / a.splits, n = max(1, (all + per - 1) / max(per, 1));
+    float m = -1e30f, l = 0.f, acc[kCh] = {0.f, 0.f};
+    for (int s = 0; s < n; ++s) m = fmaxf(m, p[s * next + a.head_dim]);
+    for (int s = 0; s < n; ++s) {
+        const float* x = p + s * next;
+        const float f = __builtin_amdgcn_exp2f(x[a.head_dim] - m);
+        l += x[a.head_dim + 1] * f;
+#pragma unroll
+        for (int c = 0; c < kCh; ++c)
+            if (lane + c * kWave < a.head_dim) acc[c] += x[lane + c * kWave] * f;
+    }
+    float inv = 1.0f / (l + 1e-9f), check = l - l;
+#pragma unroll
+    for (int c = 0; c < kCh; ++c) {
+        acc[c] *= inv;
+        check += acc[c] - acc[c];
+    }
+    const float* dout = STATS ? a.dout + (b * a.q_len + i) * a.ld_dout + hd_off : nullptr;
+    if (__any(check != check)) {
+        const OneQuery<kCh> one(a.q + (b * a.q_len + i) * a.ld_q + hd_off, a.k + b * a.kv_len * a.ld_kv + hd_off,
+                                a.v + b * a.kv_len * a.ld_kv + hd_off, a.ld_kv,
+                                a.causal ? min(static_cast<int64_t>(a.kv_len), i + 1) : a.kv_len, a.head_dim, a.qscale);
+        m = one.m;
+        inv = one.inv;
+#pragma unroll
+        for (int c = 0; c < kCh; ++c) acc[c] = one.acc[c];
+    }
+    float dot = 0.f;
+#pragma unroll
+    for (int c = 0; c < kCh; ++c) {
+        const int d = lane + c * kWave;
+        if (d >= a.head_dim) continue;
+        if (a.out) a.out[(b * a.q_len + i) * a.ld_out + hd_off + d] = acc[c];
+        if constexpr (STATS) dot += acc[c] * dout[d];
+    }
+    if constexpr (STATS) {
+        dot = wave_sum(dot);
+        if (lane == 0) {
+            stats[0] = m;
+            stats[plane] = inv;
+            stats[2 * plane] = dot;
+        }
     }
 }
 
@@ -435,9 +451,10 @@ __global__ __launch_bounds__(kGenericWaves * kWave) void attention_fwd_generic(A
     const uint32_t bh = blockIdx.x;
     const int64_t b = bh / static_cast<uint32_t>(a.heads);
     const int64_t hd_off = static_cast<int64_t>(bh % static_cast<uint32_t>(a.heads)) * a.head_dim;
-    one_query<CH>(a.q + (b * a.q_len + qi) * a.ld_q + hd_off, a.k + b * a.kv_len * a.ld_kv + hd_off,
-                  a.v + b * a.kv_len * a.ld_kv + hd_off, a.out + (b * a.q_len + qi) * a.ld_out + hd_off, a.ld_kv,
-                  a.causal ? (qi + 1 < a.kv_len ? qi + 1 : a.kv_len) : a.kv_len, a.head_dim, a.qscale);
+    const OneQuery<CH> one(a.q + (b * a.q_len + qi) * a.ld_q + hd_off, a.k + b * a.kv_len * a.ld_kv + hd_off,
+                           a.v + b * a.kv_len * a.ld_kv + hd_off, a.ld_kv,
+                           a.causal ? (qi + 1 < a.kv_len ? qi + 1 : a.kv_len) : a.kv_len, a.head_dim, a.qscale);
+    one.store(a.out + (b * a.q_len + qi) * a.ld_out + hd_off, a.head_dim);
 }
 
 template <int CH>
@@ -453,12 +470,40 @@ int launch(mimir_ctx* ctx, AttnArgs a, int64_t bh, bool vec) {
     constexpr int kThreads = WAVES * kWave;
     a.n_qblocks = (a.q_len + kQPerWave * WAVES - 1) / (kQPerWave * WAVES);
     const int64_t blocks = bh * a.n_qblocks;
-    MIMIR_REQUIRE(ctx, dispatch_fits(blocks, kThreads), "attention: grid of %lld workgroups exceeds the limit",
+    MIMIR_REQUIRE(ctx, dispatch_fits(blocks * a.splits, kThreads), "attention: grid of %lld workgroups exceeds the limit",
                   (long long)blocks);
     a.total_blocks = static_cast<uint32_t>(blocks);
-    if (vec) attention_fwd_mfma<DP, WAVES, true><<<a.total_blocks, kThreads, 0, ctx->stream>>>(a);
-    else attention_fwd_mfma<DP, WAVES, false><<<a.total_blocks, kThreads, 0, ctx->stream>>>(a);
-    return launched(ctx, "attention_fwd_mfma");
+    const auto n = static_cast<unsigned>(blocks * a.splits);
+    if (a.stats) {
+        if (vec) attention_fwd_mfma<DP, WAVES, true, true><<<n, kThreads, 0, ctx->stream>>>(a);
+        else attention_fwd_mfma<DP, WAVES, false, true><<<n, kThreads, 0, ctx->stream>>>(a);
+    } else {
+        if (vec) attention_fwd_mfma<DP, WAVES, true, false><<<n, kThreads, 0, ctx->stream>>>(a);
+        else attention_fwd_mfma<DP, WAVES, false, false><<<n, kThreads, 0, ctx->stream>>>(a);
+    }
+    if (int st = launched(ctx, "attention_fwd_mfma")) return st;
+    if (!a.part) return MIMIR_OK;
+    const int64_t rows = bh * (a.stats ? a.stats_ld : a.q_len);
+    MIMIR_REQUIRE(ctx, dispatch_fits((rows + 3) / 4, 4 * kWave), "attention: grid exceeds the limit");
+    const auto m = static_cast<unsigned>((rows + 3) / 4);
+    if (a.stats) attention_fwd_combine<true><<<m, 4 * kWave, 0, ctx->stream>>>(a, kQPerWave * WAVES);
+    else attention_fwd_combine<false><<<m, 4 * kWave, 0, ctx->stream>>>(a, kQPerWave * WAVES);
+    return launched(ctx, "attention_fwd_combine");
+}
+
+// Splits of the keys: until the workgroups fill the GPU, with partial results
+// within `floats`.  Only for 24 tiles and more: below that the combine costs
+// what the shorter chains give.  Measured (1 / 2 / 4 splits, us): 16 heads x
+// 1024 x 128 causal 106 / 86 / 70, 32 heads 107 / 101 / 112, 48 heads x 333 x
+// 777 x 80 69 / 61 / 73, 8 heads x 40 x 1500 x 128 125 / 73 / 45 (8: 34); 64
+// heads x 512 x 128 59 / 75 / 93, 8 heads x 300 x 64 20 / 23 / 21.
+int64_t splits_for(const mimir_ctx* ctx, int64_t bh, int64_t q_len, int64_t kv_len, int64_t head_dim, int64_t floats) {
+    const int64_t blocks = bh * ((q_len + 8 * kQPerWave - 1) / (8 * kQPerWave));
+    const int64_t tiles = (kv_len + kKeyTile - 1) / kKeyTile;
+    int64_t s = tiles >= 24 ? std::min<int64_t>(kSplitTarget / blocks, tiles / 4) : 1;
+    if (ctx->tune.attn_splits > 0) s = ctx->tune.attn_splits;
+    s = std::min(s, floats / (bh * q_len * (head_dim + 2)));
+    return std::max<int64_t>(s, 1);
 }
 
 template <int DP>
@@ -470,12 +515,53 @@ int launch_mfma(mimir_ctx* ctx, const AttnArgs& a, int64_t bh, bool vec) {
     // 96 x 333 x 777 x 80 136 / 78.  Few queries (40 against 1500 keys): the
     // tile's way in is the work, 142 / 122.
     const int64_t blocks4 = bh * ((a.q_len + 4 * kQPerWave - 1) / (4 * kQPerWave));
-    int waves = blocks4 <= 256 && a.q_len > 64 ? 4 : 8;
+    int waves = a.splits == 1 && blocks4 <= 256 && a.q_len > 64 ? 4 : 8;
     if (ctx->tune.attn_waves == 4 || ctx->tune.attn_waves == 8) waves = ctx->tune.attn_waves;
     return waves == 4 ? launch<DP, 4>(ctx, a, bh, vec) : launch<DP, 8>(ctx, a, bh, vec);
 }
 
+// Whether heads and strides are what the matrix-core kernels take: the tiles'
+// buffer descriptors span 32 rows of ld floats, below 2^31 bytes.
+bool mfma_takes(int64_t head_dim, int64_t ld) { return head_dim <= 128 && ld < (int64_t{1} << 31) / (4 * kKeyTile); }
+
+int launch_any(mimir_ctx* ctx, const AttnArgs& a, int64_t bh, bool vec) {
+    if (a.head_dim <= 32) return launch_mfma<32>(ctx, a, bh, vec);
+    if (a.head_dim <= 64) return launch_mfma<64>(ctx, a, bh, vec);
+    if (a.head_dim <= 96) return launch_mfma<96>(ctx, a, bh, vec);
+    return launch_mfma<128>(ctx, a, bh, vec);
+}
+
 }  // namespace
+
+int64_t mimir::attention_stats_floats(const mimir_ctx* ctx, int64_t n_bh, int64_t q_len, int64_t kv_len, int64_t head_dim) {
+    const int64_t s = splits_for(ctx, n_bh, q_len, kv_len, head_dim, INT64_MAX);
+    return s > 1 ? s * n_bh * q_len * (head_dim + 2) : 0;
+}
+
+int mimir::attention_stats(mimir_ctx* ctx, const AttnStats& x, bool vec) {
+    AttnArgs a{};
+    a.q = x.q;
+    a.k = x.k;
+    a.v = x.v;
+    a.out = x.out;
+    a.ld_q = x.ld_q;
+    a.ld_kv = x.ld_kv;
+    a.ld_out = x.ld_out;
+    a.q_len = x.q_len;
+    a.kv_len = x.kv_len;
+    a.heads = x.heads;
+    a.head_dim = x.head_dim;
+    a.qscale = x.scale * kLog2e;
+    a.causal = x.causal;
+    a.dout = x.dout;
+    a.ld_dout = x.ld_dout;
+    a.stats = x.stats;
+    a.stats_ld = x.stats_ld;
+    a.bh0 = x.bh0;
+    a.splits = static_cast<int32_t>(splits_for(ctx, x.n_bh, x.q_len, x.kv_len, x.head_dim, INT64_MAX));
+    a.part = a.splits > 1 ? x.work : nullptr;
+    return launch_any(ctx, a, x.n_bh, vec);
+}
 
 extern "C" {
 
@@ -497,7 +583,7 @@ int mimir_attention_fwd(mimir_ctx* ctx, const float* q, int64_t ld_q, const floa
     if (batch == 0 || q_len == 0) return MIMIR_OK;
     MIMIR_REQUIRE(ctx, q && out && (kv_len == 0 || (k && v)), "attention: null pointer");
     if (int st = enter(ctx)) return st;
-    AttnArgs a;
+    AttnArgs a{};
     a.q = q;
     a.k = kv_len ? k : q;  // never read when kv_len == 0
     a.v = kv_len ? v : q;
@@ -509,8 +595,6 @@ int mimir_attention_fwd(mimir_ctx* ctx, const float* q, int64_t ld_q, const floa
     a.kv_len = static_cast<int32_t>(kv_len);
     a.heads = static_cast<int32_t>(heads);
     a.head_dim = static_cast<int32_t>(head_dim);
-    a.n_qblocks = 0;
-    a.total_blocks = 0;
     a.qscale = scale * kLog2e;
     a.causal = causal ? 1 : 0;
     const bool vec = head_dim % 4 == 0 && ld_q % 4 == 0 && ld_kv % 4 == 0 && ld_out % 4 == 0 && aligned16(q) &&
@@ -520,13 +604,10 @@ int mimir_attention_fwd(mimir_ctx* ctx, const float* q, int64_t ld_q, const floa
     if (attention_decode_applies(q_len, kv_len, head_dim, a.causal))
         return attention_decode_launch(ctx, q, ld_q, a.k, a.v, ld_kv, out, ld_out, batch, q_len, kv_len, heads, head_dim,
                                        a.qscale, vec);
-    // The tile's buffer descriptors span 32 rows of ld_kv floats: below 2^31
-    // bytes, or the wide-head kernel.
-    if (ld_kv < (int64_t{1} << 31) / (4 * kKeyTile)) {
-        if (head_dim <= 32) return launch_mfma<32>(ctx, a, batch * heads, vec);
-        if (head_dim <= 64) return launch_mfma<64>(ctx, a, batch * heads, vec);
-        if (head_dim <= 96) return launch_mfma<96>(ctx, a, batch * heads, vec);
-        if (head_dim <= 128) return launch_mfma<128>(ctx, a, batch * heads, vec);
+    if (mfma_takes(head_dim, ld_kv)) {
+        a.splits = static_cast<int32_t>(splits_for(ctx, batch * heads, q_len, kv_len, head_dim, kFixedWorkBytes / 4));
+        a.part = a.splits > 1 ? static_cast<float*>(ctx->fixed_work) : nullptr;
+        return launch_any(ctx, a, batch * heads, vec);
     }
     MIMIR_REQUIRE(ctx, dispatch_fits(batch * heads, kGenericWaves * kWave) && (q_len + kGenericWaves - 1) / kGenericWaves <= 65535,
                   "attention: grid exceeds the limit of the wide-head kernel");

@@ -10,8 +10,9 @@
 //   dQ = scale dS K,   dK = scale dS^T Q,
 // then the projections' gradients dW += X^T dG and dX = dG W^T.
 //
-// The reference recomputes P from the layer's input and keeps it whole
-// ([heads, q_len, kv_len]).  Here too: P and dS are materialised per group
+// Heads up to 128 go to attention_bwd_mfma.hip; what follows is the form for
+// wider ones.  The reference recomputes P from the layer's input and keeps it
+// whole ([heads, q_len, kv_len]).  Here too: P and dS are materialised per group
 // of heads in the context's scratch (capped at kWorkBytes, one head at
 // least), the five per-head products run as strided-batched library GEMMs
 // over the group's heads straight on the Q / K / V columns of the projection
@@ -299,28 +300,6 @@ int dsoftmax(mimir_ctx* ctx, const float* p, float* g, int64_t rows, int32_t q_l
     return launched(ctx, "attn_dsoftmax_kernel");
 }
 
-// One backward of the core.  att (optional): also write the attended heads
-// P V, which the layers' output-projection gradient reads.
-struct CoreBwd {
-    const float* q;
-    int64_t ld_q;
-    const float* k;
-    const float* v;
-    int64_t ld_kv;
-    const float* dout;
-    int64_t ld_dout;
-    float* dq;
-    int64_t ld_dq;
-    float* dk;
-    float* dv;
-    int64_t ld_dkv;
-    float* att;
-    int64_t ld_att;
-    int64_t batch, q_len, kv_len, heads, head_dim;
-    float scale;
-    int causal;
-};
-
 // Heads per group (a tuning override may lower it), and the scratch floats
 // of one group (P and dS).
 int64_t heads_per_group(const mimir_ctx* ctx, const CoreBwd& a) {
@@ -332,6 +311,7 @@ int64_t heads_per_group(const mimir_ctx* ctx, const CoreBwd& a) {
 // P and dS of a head group, then either the group's dQ / dK / dV in head-
 // major blocks (hipBLASLt) or K^T and V^T of a sequence (rocBLAS only).
 int64_t work_floats(mimir_ctx* ctx, const CoreBwd& a) {
+    if (attention_bwd_mfma_takes(a)) return attention_bwd_mfma_floats(ctx, a);
     const int64_t hc = heads_per_group(ctx, a);
     return 2 * hc * a.q_len * a.kv_len + (gemm_lt(ctx) ? hc * a.head_dim * (a.q_len + 2 * a.kv_len)
                                                        : 2 * a.heads * a.head_dim * a.kv_len);
@@ -348,6 +328,7 @@ int core_bwd(mimir_ctx* ctx, const CoreBwd& a, float* work) {
         }
         return MIMIR_OK;
     }
+    if (attention_bwd_mfma_takes(a)) return attention_bwd_mfma(ctx, a, work);
     const int64_t hc = heads_per_group(ctx, a);
     const int64_t width = a.heads * D;
     float* P = work;

@@ -1,0 +1,517 @@
+// attention_bwd_mfma.hip -- the gradient of the attention core for heads up to
+// 128, on the bf16 matrix cores with fp32 operands held as three bf16 terms
+// (split.hpp).
+//
+// Reference: the per-head part of backward_self_attention (Model.cpp:
+// 6892-7028) and backward_cross_attention (:7122-7246).  With s = scale q . k
+// (causal j > i masked), p = exp(s - max) / (sum + 1e-9), dp = dout . v:
+//   dV = P^T dO,  dS = P (dP - delta),  dQ = scale dS K,  dK = scale dS^T Q,
+// delta_i = sum_j p_ij dp_ij = out_i . dout_i.  Only visible 32 x 32 tiles are
+// computed, and P is never stored:
+// 1. attention_stats (attention.hip): the forward, leaving each query's max,
+//    1 / (sum + 1e-9) and delta (and the output, where the layer wants it).
+// 2. attention_bwd_kv: a workgroup owns 128 keys and streams tiles of 32
+//    queries.  Its eight waves are four pairs, a pair for 32 keys: one wave
+//    holds the K rows and computes S, then P, then dV += dO P; the other holds
+//    the V rows and computes dP, takes P from its partner through LDS, forms
+//    dS, and computes dK += Q dS.  So each holds one operand (96 registers at
+//    128 dimensions) and one result (64) where a single wave for both would
+//    need twice that and run alone on its SIMD; a pair shares a SIMD, and both
+//    do the same two products per tile, so the code is one.  S and dP come
+//    out with the queries as rows and the wave's keys as columns, the layout
+//    of the second product's operand.  dS goes to memory in blocks of 32 x 32,
+//    [key][query], for
+// 3. attention_bwd_q: dQ += K dS^T, a wave for 32 queries, streaming 32 keys.
+// dS is the only matrix in memory (the (sequence, head) pairs run in groups
+// whose blocks fit kDsBytes), written and read once.
+//
+// Bound by latency and the barriers as much as by the matrix cores: at 8 x 32
+// heads x 1024 x 128, causal, step 2 takes 1015 us with the matrix pipes busy
+// 41% of the cycles, step 1 465 us, step 3 245 us: 1.71 ms = 101 TFLOP/s of the
+// five products, against 3.30 ms for the same products as library fp32 GEMMs
+// with P and dS in memory; 64 heads x 512 x 64 120 / 964 us, 128 heads x 100 x 64
+// 42 / 1059 us (the GEMMs ran sequence by sequence).
+//
+// LDS of step 2: Q rows, dO rows, Q^T and dO^T of one tile in bf16 planes
+// (114 KB at 128 dimensions), the pairs' P (16 KB) and the tile's max / sum /
+// delta.  One buffer: the next tile waits in registers.
+#include "attention_tile.hpp"
+#include "internal.hpp"
+
+#include <math.h>
+
+#include <algorithm>
+
+using namespace mimir;
+
+namespace {
+
+constexpr int kWaves = 8;
+constexpr int kThreads = kWaves * kWave;
+constexpr int kKeysPerBlock = 128;
+constexpr int kXcds = 8;
+constexpr float kLog2e = 1.4426950408889634f;
+constexpr int kBlockFloats = kTileRows * kTileRows;
+
+struct BwdArgs {
+    CoreBwd c;
+    int32_t q_len, kv_len, heads, head_dim;
+    float qscale;              // scale * log2(e)
+    float* stats;              // attention_stats' planes
+    int64_t stats_ld;
+    float* ds;                 // [n_bh][key tile][query tile][32 keys][32 queries]
+    int32_t q_tiles, k_tiles;
+    uint32_t bh0, n_bh;
+    uint32_t blocks;           // blocks of keys (queries) per (sequence, head)
+    // The queries (attention_bwd_kv) or keys (attention_bwd_q) dealt to
+    // several workgroups: partial dV and dK, or dQ, [split][n_bh][rows]
+    // [head_dim] each; null: one workgroup.
+    int32_t splits, q_splits;
+    float* part[3];            // dV, dK, dQ
+};
+
+// Workgroup -> (sequence, head) and its block, the longest first; each XCD
+// keeps whole (sequence, head) pairs where they divide by the XCDs.
+__device__ __forceinline__ void coords(const BwdArgs& a, uint32_t bid, uint32_t* bh, uint32_t* block) {
+    uint32_t first = 0, owned = a.n_bh, idx = bid;
+    if (a.n_bh % kXcds == 0) {
+        owned = a.n_bh / kXcds;
+        first = bid % kXcds * owned;
+        idx = bid / kXcds;
+    }
+    *block = idx / owned;
+    *bh = first + idx % owned;
+}
+
+// The gradient of one key (row) in plain fp32 by a whole wave: dv (ROLE 0) or
+// dk (ROLE 1), for keys whose split result was not finite.
+template <int CH>
+__device__ __forceinline__ void one_key(const BwdArgs& a, int role, int key, int q0, int q1, const float* q, const float* k,
+                                        const float* v, const float* dout, const float* stats, int64_t plane, float* out) {
+    const int lane = threadIdx.x % kWave;
+    float kr[CH], vr[CH], acc[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const int d = lane + c * kWave;
+        kr[c] = d < a.head_dim ? k[key * a.c.ld_kv + d] : 0.f;
+        vr[c] = d < a.head_dim ? v[key * a.c.ld_kv + d] : 0.f;
+        acc[c] = 0.f;
+    }
+    for (int i = a.c.causal ? max(key, q0) : q0; i < min(q1, a.q_len); ++i) {
+        float s = 0.f, dp = 0.f;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            const int d = lane + c * kWave;
+            if (d >= a.head_dim) continue;
+            s += q[i * a.c.ld_q + d] * kr[c];
+            dp += dout[i * a.c.ld_dout + d] * vr[c];
+        }
+        s = wave_sum(s) * a.qscale;
+        float w = __builtin_amdgcn_exp2f(s - stats[i]) * stats[plane + i];
+        if (role) {
+            dp = wave_sum(dp);
+            w = (a.c.causal && i == 0) || a.kv_len == 1 ? 0.f : w * (dp - stats[2 * plane + i]);
+        }
+        const float* row = role ? q + i * a.c.ld_q : dout + i * a.c.ld_dout;
+#pragma unroll
+        for (int c = 0; c < CH; ++c)
+            if (lane + c * kWave < a.head_dim) acc[c] += w * row[lane + c * kWave];
+    }
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+        if (lane + c * kWave < a.head_dim) out[lane + c * kWave] = acc[c] * (role ? a.c.scale : 1.f);
+}
+
+template <int DP, bool VEC>
+__global__ __launch_bounds__(kThreads, 2) void attention_bwd_kv(BwdArgs a) {
+    using Rows = RowTile<DP, kThreads, VEC>;
+    using Cols = ColTile<DP, kThreads>;
+    constexpr int kC = DP / 16, kDb = DP / 32;
+    constexpr int kRole = Rows::kBytes + Cols::kBytes;  // the rows and columns one role reads
+    __shared__ __attribute__((aligned(16))) char lds[2 * kRole];
+    __shared__ __attribute__((aligned(16))) f4 pshare[kWaves / 2][4][kWave];
+    __shared__ __attribute__((aligned(16))) float tstats[3][kTileRows];
+
+    uint32_t bh, kblock;
+    const uint32_t split = blockIdx.x % static_cast<uint32_t>(a.splits);
+    coords(a, blockIdx.x / static_cast<uint32_t>(a.splits), &bh, &kblock);
+    const uint32_t head = a.bh0 + bh;
+    const int64_t b = head / static_cast<uint32_t>(a.heads);
+    const int64_t hd = static_cast<int64_t>(head % static_cast<uint32_t>(a.heads)) * a.head_dim;
+    const float* q = a.c.q + b * a.q_len * a.c.ld_q + hd;
+    const float* dout = a.c.dout + b * a.q_len * a.c.ld_dout + hd;
+    const float* k = a.c.k + b * a.kv_len * a.c.ld_kv + hd;
+    const float* v = a.c.v + b * a.kv_len * a.c.ld_kv + hd;
+    const float* stats = a.stats + bh * a.stats_ld;
+    const int64_t plane = a.n_bh * a.stats_ld;
+
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int li = lane % 32, hf = lane / 32;
+    const int pair = wave % 4, role = __builtin_amdgcn_readfirstlane(wave / 4);
+    const int k0 = static_cast<int>(kblock) * kKeysPerBlock + pair * kTileRows;
+    const int key = k0 + li;
+    const int ktile = k0 / kTileRows;
+    // Query tiles the workgroup streams, and the first that this pair sees.
+    const int first_t = a.c.causal ? min(static_cast<int>(kblock) * (kKeysPerBlock / kTileRows), a.q_tiles) : 0;
+    const int per = (a.q_tiles - first_t + a.splits - 1) / a.splits;
+    const int t0 = min(first_t + static_cast<int>(split) * per, a.q_tiles), t_end = min(t0 + per, a.q_tiles);
+    const int pair_t0 = a.c.causal ? ktile : 0;
+    const bool pair_in = k0 < a.kv_len;
+
+    Rows qrows, drows;
+    Cols qcols, dcols;
+    qrows.init(a.c.ld_q, a.head_dim);
+    qcols.init(a.c.ld_q, a.head_dim);
+    drows.init(a.c.ld_dout, a.head_dim);
+    dcols.init(a.c.ld_dout, a.head_dim);
+    float stat = 0.f;
+    auto load = [&](int t) {
+        qrows.load(q, t, a.c.ld_q, a.q_len, a.head_dim);
+        dcols.load(dout, t, a.c.ld_dout, a.q_len, a.head_dim);
+        drows.load(dout, t, a.c.ld_dout, a.q_len, a.head_dim);
+        qcols.load(q, t, a.c.ld_q, a.q_len, a.head_dim);
+        if (threadIdx.x < 3 * kTileRows) stat = stats[threadIdx.x / kTileRows * plane + t * kTileRows + threadIdx.x % kTileRows];
+    };
+    auto stash = [&]() {  // role 0 reads Q rows and dO columns, role 1 dO rows and Q columns
+        qrows.stash(lds);
+        dcols.stash(lds + Rows::kBytes);
+        drows.stash(lds + kRole);
+        qcols.stash(lds + kRole + Rows::kBytes);
+        if (threadIdx.x < 3 * kTileRows) tstats[threadIdx.x / kTileRows][threadIdx.x % kTileRows] = stat;
+    };
+    if (t0 < t_end) load(t0);
+    Split8 own[kC];
+    row_operand<DP, VEC>((role ? v : k) + static_cast<int64_t>(min(key, a.kv_len - 1)) * a.c.ld_kv, hf, a.head_dim, 1.0f, own);
+    f16v acc[kDb];
+#pragma unroll
+    for (int d = 0; d < kDb; ++d) acc[d] = f16v{};
+    const char* const rows = lds + role * kRole;
+    const char* const cols = rows + Rows::kBytes;
+
+    for (int t = t0; t < t_end; ++t) {
+        stash();
+        __syncthreads();
+        load(min(t + 1, t_end - 1));
+        const bool work = pair_in && t >= pair_t0;
+        f16v x = f16v{};
+        if (work) {
+#pragma unroll
+            for (int c = 0; c < kC; ++c) x = mfma_split(Rows::at(rows, li, hf, c), own[c], x);
+            if (role == 0) {
+                // A tile that the diagonal or the last key crosses.
+                const bool edge = k0 + kTileRows > a.kv_len || (a.c.causal && t == ktile);
+#pragma unroll
+                for (int r = 0; r < 16; r += 4) {
+                    const f4 m = *reinterpret_cast<const f4*>(&tstats[0][8 * (r / 4) + 4 * hf]);
+                    const f4 inv = *reinterpret_cast<const f4*>(&tstats[1][8 * (r / 4) + 4 * hf]);
+                    f4 p;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        p[e] = __builtin_amdgcn_exp2f(x[r + e] * a.qscale - m[e]) * inv[e];
+                        if (edge && (key >= a.kv_len || (a.c.causal && key > t * kTileRows + 8 * (r / 4) + 4 * hf + e)))
+                            p[e] = 0.f;
+                        x[r + e] = p[e];
+                    }
+                    pshare[pair][r / 4][lane] = p;
+                }
+            }
+        }
+        __syncthreads();
+        if (work) {
+            if (role == 1) {
+                float* block = a.ds + ((static_cast<int64_t>(bh) * a.k_tiles + ktile) * a.q_tiles + t) * kBlockFloats;
+#pragma unroll
+                for (int r = 0; r < 16; r += 4) {
+                    const f4 p = pshare[pair][r / 4][lane];
+                    const f4 delta = *reinterpret_cast<const f4*>(&tstats[2][8 * (r / 4) + 4 * hf]);
+                    f4 ds;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        // A query that sees one key has p = 1 and no gradient.
+                        const bool one = a.kv_len == 1 || (a.c.causal && t == 0 && r + e == 0 && hf == 0);
+                        ds[e] = one ? 0.f : p[e] * (x[r + e] - delta[e]);
+                        if (key >= a.kv_len) ds[e] = 0.f;
+                        x[r + e] = ds[e];
+                    }
+                    *reinterpret_cast<f4*>(block + li * kTileRows + 8 * (r / 4) + 4 * hf) = ds;
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                float w[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) w[e] = x[8 * c + e];
+                const Split8 s = split8(w);
+#pragma unroll
+                for (int d = 0; d < kDb; ++d) acc[d] = mfma_split(Cols::at(cols, li, hf, d, c), s, acc[d]);
+            }
+        }
+        __syncthreads();
+    }
+    const bool in = key < a.kv_len;
+    float* grad = (role ? a.c.dk : a.c.dv) + b * a.kv_len * a.c.ld_dkv + hd;
+    int64_t ld = a.c.ld_dkv;
+    if (a.part[role]) {
+        ld = a.head_dim;
+        grad = a.part[role] + (split * static_cast<int64_t>(a.n_bh) + bh) * a.kv_len * ld;
+    }
+    const float check = store_columns<DP, VEC>(acc, role ? a.c.scale : 1.0f, grad + min(key, a.kv_len - 1) * ld, in, hf,
+                                               a.head_dim);
+    for (uint32_t redo = bad_rows(check, in); redo; redo &= redo - 1) {
+        const int i = k0 + __builtin_ctz(redo);
+        one_key<(DP + kWave - 1) / kWave>(a, role, i, t0 * kTileRows, t_end * kTileRows, q, k, v, dout, stats, plane,
+                                          grad + i * ld);
+    }
+}
+
+// The splits' partial results added up, in order: grid.y chooses dV, dK or dQ.
+template <bool VEC>
+__global__ __launch_bounds__(256) void attention_bwd_sum(BwdArgs a) {
+    constexpr uint32_t kW = VEC ? 4 : 1;
+    const int which = blockIdx.y;
+    const float* part = a.part[which];
+    if (!part) return;
+    const uint32_t len = which == 2 ? a.q_len : a.kv_len, row = a.head_dim / kW;
+    const int splits = which == 2 ? a.q_splits : a.splits;
+    const int64_t ld = which == 2 ? a.c.ld_dq : a.c.ld_dkv, one = static_cast<int64_t>(a.n_bh) * len * a.head_dim;
+    float* out = which == 0 ? a.c.dv : which == 1 ? a.c.dk : a.c.dq;
+    const uint32_t x = blockIdx.x * 256 + threadIdx.x;
+    if (x >= a.n_bh * len * row) return;
+    const uint32_t at = x / row, d = x % row * kW, head = a.bh0 + at / len, i = at % len;
+    float* o = out + (static_cast<int64_t>(head / a.heads) * len + i) * ld + static_cast<int64_t>(head % a.heads) * a.head_dim + d;
+    const float* p = part + static_cast<int64_t>(x) * kW;
+    if constexpr (VEC) {
+        f4 sum = *reinterpret_cast<const f4*>(p);
+        for (int s = 1; s < splits; ++s) sum += *reinterpret_cast<const f4*>(p + s * one);
+        *reinterpret_cast<f4*>(o) = sum;
+    } else {
+        float sum = *p;
+        for (int s = 1; s < splits; ++s) sum += p[s * one];
+        *o = sum;
+    }
+}
+
+// dQ from dS: a wave for 32 queries; K^T tiles through LDS, dS blocks straight
+// to registers (lane = query).
+template <int DP, bool VEC>
+__global__ __launch_bounds__(kThreads, 2) void attention_bwd_q(BwdArgs a) {
+    using Cols = ColTile<DP, kThreads>;
+    constexpr int kDb = DP / 32;
+    __shared__ __attribute__((aligned(16))) char lds[2 * Cols::kBytes];
+
+    uint32_t bh, qblock;
+    const int split = static_cast<int>(blockIdx.x % static_cast<uint32_t>(a.q_splits));
+    coords(a, blockIdx.x / static_cast<uint32_t>(a.q_splits), &bh, &qblock);
+    if (a.c.causal) qblock = a.blocks - 1 - qblock;  // the last queries see the most keys
+    const uint32_t head = a.bh0 + bh;
+    const int64_t b = head / static_cast<uint32_t>(a.heads);
+    const int64_t hd = static_cast<int64_t>(head % static_cast<uint32_t>(a.heads)) * a.head_dim;
+    const float* k = a.c.k + b * a.kv_len * a.c.ld_kv + hd;
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int li = lane % 32, hf = lane / 32;
+    const int qt = static_cast<int>(qblock) * kWaves + wave;  // this wave's query tile
+    const int my_q = qt * kTileRows + li;
+    const int last_qt = min(static_cast<int>(qblock) * kWaves + kWaves, a.q_tiles) - 1;
+    const int all_tiles = a.c.causal ? min(a.k_tiles, last_qt + 1) : a.k_tiles;
+    const int per = (all_tiles + a.q_splits - 1) / a.q_splits;
+    const int t0 = min(split * per, all_tiles), n_tiles = min(t0 + per, all_tiles);
+    const int wave_tiles = qt >= a.q_tiles ? 0 : min(n_tiles, a.c.causal ? qt + 1 : a.k_tiles);
+    const float* ds = a.ds + (static_cast<int64_t>(bh) * a.k_tiles * a.q_tiles + min(qt, a.q_tiles - 1)) * kBlockFloats;
+
+    Cols kcols;
+    kcols.init(a.c.ld_kv, a.head_dim);
+    float w[16];
+    auto load_ds = [&](int t) {
+        const float* block = ds + static_cast<int64_t>(min(t, max(wave_tiles - 1, 0))) * a.q_tiles * kBlockFloats + li;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) w[r] = __builtin_nontemporal_load(block + (8 * (r / 4) + 4 * hf + r % 4) * kTileRows);
+    };
+    f16v acc[kDb];
+#pragma unroll
+    for (int d = 0; d < kDb; ++d) acc[d] = f16v{};
+    if (t0 < n_tiles) {
+        kcols.load(k, t0, a.c.ld_kv, a.kv_len, a.head_dim);
+        if (t0 < wave_tiles) load_ds(t0);
+        kcols.stash(lds);
+        kcols.load(k, min(t0 + 1, n_tiles - 1), a.c.ld_kv, a.kv_len, a.head_dim);
+    }
+    __syncthreads();
+    for (int t = t0; t < n_tiles; ++t) {
+        const char* cur = lds + ((t - t0) & 1) * Cols::kBytes;
+        if (t < wave_tiles) {
+            Split8 s[2];
+            s[0] = split8(w);
+            s[1] = split8(w + 8);
+            load_ds(t + 1);
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+#pragma unroll
+                for (int d = 0; d < kDb; ++d) acc[d] = mfma_split(Cols::at(cur, li, hf, d, c), s[c], acc[d]);
+        }
+        kcols.stash(lds + ((t - t0 + 1) & 1) * Cols::kBytes);
+        kcols.load(k, min(t + 2, n_tiles - 1), a.c.ld_kv, a.kv_len, a.head_dim);
+        __syncthreads();
+    }
+    const bool in = my_q < a.q_len;
+    float* dq = a.c.dq + b * a.q_len * a.c.ld_dq + hd;
+    int64_t ld = a.c.ld_dq;
+    if (a.part[2]) {
+        ld = a.head_dim;
+        dq = a.part[2] + (split * static_cast<int64_t>(a.n_bh) + bh) * a.q_len * ld;
+    }
+    const float check = store_columns<DP, VEC>(acc, a.c.scale, dq + min(my_q, a.q_len - 1) * ld, in, hf, a.head_dim);
+    // Queries whose result is not finite, in plain fp32 (split.hpp).
+    constexpr int kCh = (DP + kWave - 1) / kWave;
+    for (uint32_t redo = bad_rows(check, in); redo; redo &= redo - 1) {
+        const int i = qt * kTileRows + __builtin_ctz(redo);
+        const float* q = a.c.q + (b * a.q_len + i) * a.c.ld_q + hd;
+        const float* dout = a.c.dout + (b * a.q_len + i) * a.c.ld_dout + hd;
+        const float* v = a.c.v + b * a.kv_len * a.c.ld_kv + hd;
+        const float* stats = a.stats + bh * a.stats_ld + i;
+        const int64_t plane = a.n_bh * a.stats_ld;
+        const int keys = a.c.causal ? min(a.kv_len, i + 1) : a.kv_len;
+        float sum[kCh];
+#pragma unroll
+        for (int c = 0; c < kCh; ++c) sum[c] = 0.f;
+        for (int j = t0 * kTileRows; j < min(keys, n_tiles * kTileRows); ++j) {
+            float s = 0.f, dp = 0.f;
+#pragma unroll
+            for (int c = 0; c < kCh; ++c) {
+                const int d = lane + c * kWave;
+                if (d >= a.head_dim) continue;
+                s += q[d] * k[j * a.c.ld_kv + d];
+                dp += dout[d] * v[j * a.c.ld_kv + d];
+            }
+            s = wave_sum(s) * a.qscale;
+            dp = wave_sum(dp);
+            const float p = __builtin_amdgcn_exp2f(s - stats[0]) * stats[plane];
+            const float g = keys == 1 ? 0.f : p * (dp - stats[2 * plane]);
+#pragma unroll
+            for (int c = 0; c < kCh; ++c)
+                if (lane + c * kWave < a.head_dim) sum[c] += g * k[j * a.c.ld_kv + lane + c * kWave];
+        }
+#pragma unroll
+        for (int c = 0; c < kCh; ++c)
+            if (lane + c * kWave < a.head_dim) dq[i * ld + lane + c * kWave] = sum[c] * a.c.scale;
+    }
+}
+
+int64_t tiles(int64_t n) { return (n + kTileRows - 1) / kTileRows; }
+int64_t key_blocks(const CoreBwd& c) { return (c.kv_len + kKeysPerBlock - 1) / kKeysPerBlock; }
+int64_t query_blocks(const CoreBwd& c) { return (tiles(c.q_len) + kWaves - 1) / kWaves; }
+
+template <int DP>
+int launch(mimir_ctx* ctx, BwdArgs a, bool vec) {
+    a.blocks = static_cast<uint32_t>(key_blocks(a.c));
+    const int64_t n = static_cast<int64_t>(a.n_bh) * a.blocks * a.splits;
+    const int64_t m = static_cast<int64_t>(a.n_bh) * query_blocks(a.c) * a.q_splits;
+    MIMIR_REQUIRE(ctx, dispatch_fits(std::max(n, m), kThreads), "attention backward: grid too large");
+    if (vec) attention_bwd_kv<DP, true><<<static_cast<unsigned>(n), kThreads, 0, ctx->stream>>>(a);
+    else attention_bwd_kv<DP, false><<<static_cast<unsigned>(n), kThreads, 0, ctx->stream>>>(a);
+    if (int st = launched(ctx, "attention_bwd_kv")) return st;
+    a.blocks = static_cast<uint32_t>(query_blocks(a.c));
+    if (vec) attention_bwd_q<DP, true><<<static_cast<unsigned>(m), kThreads, 0, ctx->stream>>>(a);
+    else attention_bwd_q<DP, false><<<static_cast<unsigned>(m), kThreads, 0, ctx->stream>>>(a);
+    if (int st = launched(ctx, "attention_bwd_q")) return st;
+    if (!a.part[0] && !a.part[2]) return MIMIR_OK;
+    const int64_t rows = std::max(a.part[0] ? a.kv_len : 0, a.part[2] ? a.q_len : 0);
+    const int64_t items = a.n_bh * rows * (vec ? a.head_dim / 4 : a.head_dim);
+    MIMIR_REQUIRE(ctx, dispatch_fits((items + 255) / 256, 256), "attention backward: grid too large");
+    const dim3 grid(static_cast<unsigned>((items + 255) / 256), 3);
+    if (vec) attention_bwd_sum<true><<<grid, 256, 0, ctx->stream>>>(a);
+    else attention_bwd_sum<false><<<grid, 256, 0, ctx->stream>>>(a);
+    return launched(ctx, "attention_bwd_sum");
+}
+
+// (sequence, head) pairs per group: their dS blocks stay below kDsBytes.
+// Measured at 8 x 32 heads x 1024 x 128, causal (us): 128 MiB 2599, 256 MiB
+// 1998, 512 MiB 1703, 1 GiB 1710.
+constexpr int64_t kDsBytes = int64_t{1} << 29;
+int64_t group_of(const mimir_ctx* ctx, const CoreBwd& c) {
+    const int64_t one = tiles(c.q_len) * tiles(c.kv_len) * kBlockFloats * static_cast<int64_t>(sizeof(float));
+    int64_t n = std::min(c.batch * c.heads, std::max<int64_t>(1, kDsBytes / one));
+    if (n < c.batch * c.heads && n > kXcds) n -= n % kXcds;
+    if (ctx->tune.attn_bwd_heads > 0) n = std::min<int64_t>(n, ctx->tune.attn_bwd_heads);
+    return n;
+}
+
+// Workgroups per block of 128 keys or 256 queries: the other side is split
+// until the workgroups fill the GPU, four tiles each at least.  The target of
+// 512 against 256 / 1024 (us): 16 heads x 2048 x 64 causal 304 / 349 / 330, 16 x
+// 1024 x 128 218 / 210 / 267 (unsplit 364), 64 x 512 x 64 120 / 116 / 143.
+int64_t splits_of(int64_t blocks, int64_t steps) {
+    constexpr int64_t kTarget = 512;
+    return std::max<int64_t>(1, std::min<int64_t>(kTarget / blocks, steps / 4));
+}
+int64_t kv_splits(const CoreBwd& c, int64_t n_bh) { return splits_of(n_bh * key_blocks(c), tiles(c.q_len)); }
+int64_t q_splits(const CoreBwd& c, int64_t n_bh) { return splits_of(n_bh * query_blocks(c), tiles(c.kv_len)); }
+// Floats of one partial result (rounded so that the next is 16-byte aligned).
+int64_t part_floats(int64_t splits, int64_t n_bh, int64_t rows, int64_t head_dim) {
+    return splits > 1 ? (splits * n_bh * rows * head_dim + 3) / 4 * 4 : 0;
+}
+int64_t parts_floats(const mimir_ctx* ctx, const CoreBwd& c, int64_t n_bh) {
+    // The forward's partial results are gone before the others are written.
+    return std::max(2 * part_floats(kv_splits(c, n_bh), n_bh, c.kv_len, c.head_dim) +
+                        part_floats(q_splits(c, n_bh), n_bh, c.q_len, c.head_dim),
+                    attention_stats_floats(ctx, n_bh, c.q_len, c.kv_len, c.head_dim));
+}
+int64_t ds_floats(const CoreBwd& c, int64_t n_bh) { return n_bh * tiles(c.q_len) * tiles(c.kv_len) * kBlockFloats; }
+int64_t stats_floats(const CoreBwd& c, int64_t n_bh) { return 3 * n_bh * tiles(c.q_len) * kTileRows; }
+
+}  // namespace
+
+namespace mimir {
+
+bool attention_bwd_mfma_takes(const CoreBwd& c) {
+    const int64_t lim = (int64_t{1} << 31) / (4 * kTileRows);
+    return c.head_dim <= 128 && c.kv_len > 0 && c.q_len > 0 && c.ld_q < lim && c.ld_kv < lim && c.ld_dout < lim;
+}
+
+int64_t attention_bwd_mfma_floats(const mimir_ctx* ctx, const CoreBwd& c) {
+    const int64_t n = group_of(ctx, c), rest = c.batch * c.heads % n;  // the last group may be smaller and split more
+    return ds_floats(c, n) + stats_floats(c, n) + std::max(parts_floats(ctx, c, n), rest ? parts_floats(ctx, c, rest) : 0);
+}
+
+int attention_bwd_mfma(mimir_ctx* ctx, const CoreBwd& c, float* work) {
+    const int64_t group = group_of(ctx, c), total = c.batch * c.heads;
+    const int64_t stats_ld = tiles(c.q_len) * kTileRows;
+    auto vec4 = [](const float* p, int64_t ld) { return ld % 4 == 0 && aligned16(p); };
+    const bool vec = c.head_dim % 4 == 0 && vec4(c.q, c.ld_q) && vec4(c.k, c.ld_kv) && vec4(c.v, c.ld_kv) &&
+                     vec4(c.dout, c.ld_dout) && vec4(c.dq, c.ld_dq) && vec4(c.dk, c.ld_dkv) && vec4(c.dv, c.ld_dkv) &&
+                     (!c.att || vec4(c.att, c.ld_att));
+    BwdArgs a{};
+    a.c = c;
+    a.q_len = static_cast<int32_t>(c.q_len);
+    a.kv_len = static_cast<int32_t>(c.kv_len);
+    a.heads = static_cast<int32_t>(c.heads);
+    a.head_dim = static_cast<int32_t>(c.head_dim);
+    a.qscale = c.scale * kLog2e;
+    a.ds = work;  // 16-byte aligned blocks first
+    a.stats = work + ds_floats(c, group);
+    a.stats_ld = stats_ld;
+    a.q_tiles = static_cast<int32_t>(tiles(c.q_len));
+    a.k_tiles = static_cast<int32_t>(tiles(c.kv_len));
+    for (int64_t h0 = 0; h0 < total; h0 += group) {
+        a.bh0 = static_cast<uint32_t>(h0);
+        a.n_bh = static_cast<uint32_t>(std::min(group, total - h0));
+        float* const parts = a.stats + stats_floats(c, group);
+        const AttnStats st{c.q, c.ld_q, c.k, c.v, c.ld_kv, c.dout, c.ld_dout, c.att, c.ld_att, a.stats, stats_ld,
+                           a.q_len, a.kv_len, a.heads, a.head_dim, a.bh0, a.n_bh, c.scale, c.causal, parts};
+        if (int e = attention_stats(ctx, st, vec)) return e;
+        a.splits = static_cast<int32_t>(kv_splits(c, a.n_bh));
+        a.q_splits = static_cast<int32_t>(q_splits(c, a.n_bh));
+        const int64_t one = part_floats(a.splits, a.n_bh, c.kv_len, c.head_dim);
+        a.part[0] = a.splits > 1 ? parts : nullptr;
+        a.part[1] = a.splits > 1 ? parts + one : nullptr;
+        a.part[2] = a.q_splits > 1 ? parts + 2 * one : nullptr;
+        int e = MIMIR_OK;
+        if (c.head_dim <= 32) e = launch<32>(ctx, a, vec);
+        else if (c.head_dim <= 64) e = launch<64>(ctx, a, vec);
+        else if (c.head_dim <= 96) e = launch<96>(ctx, a, vec);
+        else e = launch<128>(ctx, a, vec);
+        if (e) return e;
+    }
+    return MIMIR_OK;
+}
+
+}  // namespace mimir

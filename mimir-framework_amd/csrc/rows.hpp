@@ -65,6 +65,7 @@ struct Tuning {
     int lnbwd_grid = 0;       // its persistent grid (workgroups)
     int chain_streamed = 0;   // chain=0: the runtime streams every layer's output (no kept outputs)
     int attn_waves = 0;       // attention forward: waves per workgroup (4, 8; 0: measured default)
+    int attn_splits = 0;      // attention forward: splits of the keys (0: measured default)
     int decode_splits = 0;    // attention_decode: workgroups per (sequence, head) (0: measured default)
     int attn_bwd_heads = 0;   // heads per group of the attention backward (0: what 1 GiB of P / dS holds)
     int attn_bwd_blocks = 0;  // causal attention backward: query / key blocks of the products (0: default)
@@ -118,6 +119,7 @@ inline Tuning read_tuning() {
         else if (!std::strcmp(k, "lnbwd_grid")) t.lnbwd_grid = std::atoi(v);
         else if (!std::strcmp(k, "chain")) t.chain_streamed = std::atoi(v) == 0;
         else if (!std::strcmp(k, "attnwaves")) t.attn_waves = std::atoi(v);
+        else if (!std::strcmp(k, "attnsplits")) t.attn_splits = std::atoi(v);
         else if (!std::strcmp(k, "decode")) t.decode_splits = std::atoi(v);
         else if (!std::strcmp(k, "attnbwd_heads")) t.attn_bwd_heads = std::atoi(v);
         else if (!std::strcmp(k, "attnbwd_blocks")) t.attn_bwd_blocks = std::atoi(v);

@@ -1,0 +1,59 @@
+"""The attention backward on split bf16 operands: the edges of its key blocks
+(128), query blocks (256), tiles (32) and splits, and values without a split,
+against float64."""
+import numpy as np
+import pytest
+
+import oracle as O
+from _attention import assert_bwd_close, attention_bwd64
+from test_gpu_attention_bwd import _tuned_context, check_core, gpu_core_bwd, rand_core
+
+pytestmark = pytest.mark.gpu
+
+# One tile and less, one key block and one key more, more than one query block,
+# few heads with long rows (both sides split) and heads that fill the GPU.
+SHAPES = [(1, 1, 33, 1, 4), (1, 32, 32, 2, 32), (2, 31, 129, 1, 36), (1, 257, 128, 2, 64), (1, 129, 257, 1, 72),
+          (1, 288, 288, 1, 96), (1, 1025, 200, 1, 32), (1, 200, 1030, 1, 128), (70, 33, 140, 8, 16), (1, 65, 65, 3, 7)]
+
+
+@pytest.mark.parametrize("b,lq,lk,heads,hd", SHAPES)
+@pytest.mark.parametrize("causal", [False, True])
+def test_split_backward(ctx, b, lq, lk, heads, hd, causal):
+    q, k, v, dout = rand_core(lq + lk + hd, b, lq, lk, heads * hd)
+    got = gpu_core_bwd(ctx, q, k, v, dout, heads, causal)
+    for i in range(0, b, max(1, b // 2)):
+        check_core([g[i:i + 1] for g in got], q[i:i + 1], k[i:i + 1], v[i:i + 1], dout[i:i + 1], heads, causal,
+                   f"split backward {b} {lq} {lk} {heads} {hd} {causal} [{i}]", oracle=False)
+
+
+def test_split_backward_groups():
+    """(sequence, head) pairs in groups with a smaller last one."""
+    c = _tuned_context("attnbwd_heads=3")
+    try:
+        q, k, v, dout = rand_core(8, 2, 300, 300, 4 * 32)
+        check_core(gpu_core_bwd(c, q, k, v, dout, 4, True), q, k, v, dout, 4, True, "groups of 3", oracle=False)
+    finally:
+        c.close()
+
+
+def test_split_backward_special_values(ctx):
+    """A NaN key reaches the gradients of the queries that see it and no
+    other; a query value that rounds to infinity in bf16 multiplies zeros."""
+    n, hd = 200, 32
+    q, k, v, dout = rand_core(4, 1, n, n, hd)
+    k[0, :, 3] = 0.0
+    q[0, 7, 3] = 3.4e38
+    (dq, dk, dv), tol = attention_bwd64(q[0], k[0], v[0], dout[0], 1, True, O.attention_scale(hd))
+    got = gpu_core_bwd(ctx, q, k, v, dout, 1, True)
+    keep = [d for d in range(hd) if d != 3]
+    for name, g, want, t, cols in (("dq", got[0][0], dq, tol[0], list(range(hd))), ("dk", got[1][0], dk, tol[1], keep),
+                                   ("dv", got[2][0], dv, tol[2], list(range(hd)))):
+        assert np.isfinite(g[:, cols]).all(), name
+        t = np.where(np.isfinite(t[:, cols]), np.minimum(t[:, cols], 1e-3), 1e-3)
+        np.testing.assert_array_less(np.abs(g[:, cols] - want[:, cols]), t + 1e-5, err_msg=name)
+    q, k, v, dout = rand_core(5, 1, n, n, hd)
+    (dq, _, _), tol = attention_bwd64(q[0], k[0], v[0], dout[0], 1, True, O.attention_scale(hd))
+    k[0, n - 1, 5] = np.nan
+    got = gpu_core_bwd(ctx, q, k, v, dout, 1, True)[0][0]
+    assert np.isnan(got[n - 1]).all()
+    assert_bwd_close(got[:n - 1], dq[:n - 1], tol[0][:n - 1], "queries that do not see the NaN key")
