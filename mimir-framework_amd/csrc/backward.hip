@@ -20,9 +20,10 @@
 //                            sums in registers over the rows it visits and
 //                            writes them once; sum_slots adds the slots in a
 //                            fixed order into grad_weights
-//   ln_bwd_scalar            the same with 4-byte columns: rows up to 4096
-//                            floats that are not 16-byte aligned or whose
-//                            width is not a multiple of 4
+//   ln_bwd_any               the same with vectors at 4-byte addresses: rows up
+//                            to 4096 floats that are not 16-byte aligned or
+//                            whose width is not a multiple of 4
+//   ln_bwd_scalar            rows of at most 64 floats, several per wave
 //   ln_stats_generic, ln_bwd_params_part, ln_bwd_generic  any other width /
 //                            alignment
 //   embed_sort_*, embed_bwd_* scatter-add of dy rows into the gradient table:
@@ -465,6 +466,7 @@ __global__ __launch_bounds__(1024) void sum_slots_tile(const float* part, int64_
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int64_t c = 4 * c4 + i;
+            if (c >= width) break;
             float* o = c < split ? out0 + c : out1 + (c - split);
             *o = acc ? *o + t[i] : t[i];
         }
@@ -489,14 +491,17 @@ __global__ __launch_bounds__(1024) void sum_total(const float* part, int64_t nsl
 int launch_sum_slots(mimir_ctx* ctx, const float* part, int64_t nslots, int64_t stride, int64_t width, float* out0,
                      float* out1, int64_t split, bool acc, float* tmp = nullptr) {
     unsigned blocks;
-    if (width % 4 == 0 && stride % 4 == 0 && split % 4 == 0 && aligned16(part)) {
+    if (stride % 4 == 0 && aligned16(part)) {
+        // Any width: a slot holds stride floats, a multiple of 4.
         if (nslots >= 4 * kGroups && nslots <= kTileMaxSlots) {
-            if (!grid_for(width / 4, kTileCols, 1024, &blocks))
+            if (!grid_for((width + 3) / 4, kTileCols, 1024, &blocks))
                 return fail(ctx, MIMIR_EINVAL, "sum_slots: width %lld exceeds the grid limit", (long long)width);
             sum_slots_tile<4><<<blocks, 1024, 0, ctx->stream>>>(part, nslots, stride, width, out0, out1, split,
                                                                acc ? 1 : 0);
             return launched(ctx, "sum_slots_tile");
         }
+    }
+    if (width % 4 == 0 && stride % 4 == 0 && split % 4 == 0 && aligned16(part)) {
         if (!grid_for(width / 4, kWave, kBlock, &blocks))
             return fail(ctx, MIMIR_EINVAL, "sum_slots: width %lld exceeds the grid limit", (long long)width);
         if (tmp && aligned16(tmp) && nslots >= 4 * kGroups) {
@@ -762,6 +767,9 @@ __device__ __forceinline__ void row_sum2(float& a, float& b, float* la, float* l
 
 __device__ __forceinline__ float hsum(f4 v) { return (v.x + v.y) + (v.z + v.w); }
 
+// Floats of one dgamma | dbeta slot of the persistent kernels: whole vectors.
+__host__ __device__ constexpr int64_t slot_floats(int64_t cols) { return (2 * cols + 3) / 4 * 4; }
+
 // A persistent grid (fewer blocks than row groups): sub-row `sub` of block b
 // visits rows sub + RPB*(b + k*grid) and keeps dgamma / dbeta for its
 // TPR*VPT*4 columns in registers; the block writes one slot of partial sums.
@@ -859,7 +867,7 @@ __global__ __launch_bounds__(BS) void ln_bwd_vec(LnBwdArgs a) {
     if (!a.part) return;
     // One slot per workgroup: the sub-rows' sums are added in sub-row order
     // through LDS, then written once.
-    float* p = a.part + static_cast<int64_t>(blockIdx.x) * 2 * a.cols;
+    float* p = a.part + static_cast<int64_t>(blockIdx.x) * slot_floats(a.cols);
     if constexpr (RPB > 1) {
         __shared__ f4 comb[2 * TPR * VPT];
         for (int r = 0; r < RPB; ++r) {
@@ -890,19 +898,13 @@ __global__ __launch_bounds__(BS) void ln_bwd_vec(LnBwdArgs a) {
     }
 }
 
-// Rows of up to 4096 floats whose 16-byte vectors do not line up (a width
-// that is not a multiple of 4, or an unaligned pointer), and rows of at most
-// 64 floats: ln_bwd_vec's scheme with 4-byte columns c = j*TPR + t, TPR
-// threads per row and kBlock/TPR rows per workgroup (one wave per row up to
-// 1024 floats: no barrier in the row sums, and four rows' loads in flight
-// per workgroup; 16 or 32 lanes per row up to 64 floats, so a wave holds two
-// or four rows and sums them with lane-group reductions).  Each row is read
-// once; a thread reads dy[c] before it writes dx[c], so dx may alias dy.
+// Rows of at most 64 floats: ln_bwd_vec's scheme with 4-byte columns
+// c = j*TPR + t, 16 or 32 lanes per row, so a wave holds two or four rows and
+// sums them with lane-group reductions.  Each row is read once; a thread reads
+// dy[c] before it writes dx[c], so dx may alias dy.
 template <int TPR, int VPT, bool KEEP>
 __global__ __launch_bounds__(kBlock) void ln_bwd_scalar(LnBwdArgs a) {
     constexpr int RPB = kBlock / TPR;
-    constexpr int NW = TPR / kWave;
-    __shared__ float lds[4][kBlock / kWave];
     const int t = threadIdx.x % TPR;
     const int sub = threadIdx.x / TPR;
     const float n = static_cast<float>(a.cols);
@@ -942,12 +944,8 @@ __global__ __launch_bounds__(kBlock) void ln_bwd_scalar(LnBwdArgs a) {
             s += xv[j];
             s1 += gv[j] * gm[j];
         }
-        if constexpr (TPR < kWave) {
-            s = group_sum<TPR>(s);
-            s1 = group_sum<TPR>(s1);
-        } else {
-            row_sum2<NW>(s, s1, lds[0], lds[1], sub);
-        }
+        s = group_sum<TPR>(s);
+        s1 = group_sum<TPR>(s1);
         const float mean = s / n;  // :7765-7768
         float q = 0.0f, p2 = 0.0f;
 #pragma unroll
@@ -958,12 +956,8 @@ __global__ __launch_bounds__(kBlock) void ln_bwd_scalar(LnBwdArgs a) {
                 p2 += gv[j] * gm[j] * d;
             }
         }
-        if constexpr (TPR < kWave) {
-            q = group_sum<TPR>(q);
-            p2 = group_sum<TPR>(p2);
-        } else {
-            row_sum2<NW>(q, p2, lds[2], lds[3], sub);
-        }
+        q = group_sum<TPR>(q);
+        p2 = group_sum<TPR>(p2);
         const float var = q / n;                          // :7770-7776
         const float inv_std = 1.0f / sqrtf(var + a.eps);  // :7777
         const float s2 = p2 * inv_std;
@@ -991,7 +985,7 @@ __global__ __launch_bounds__(kBlock) void ln_bwd_scalar(LnBwdArgs a) {
     if (!a.part) return;
     // One slot per workgroup: the sub-rows' sums are added in sub-row order
     // through LDS, then written once.
-    float* p = a.part + static_cast<int64_t>(blockIdx.x) * 2 * a.cols;
+    float* p = a.part + static_cast<int64_t>(blockIdx.x) * slot_floats(a.cols);
     if constexpr (RPB > 1) {
         __shared__ float comb[2 * TPR * VPT];
         for (int r = 0; r < RPB; ++r) {
@@ -1019,6 +1013,119 @@ __global__ __launch_bounds__(kBlock) void ln_bwd_scalar(LnBwdArgs a) {
             p[c] = dg[j];
             p[a.cols + c] = db[j];
         }
+    }
+}
+
+// Rows of more than 64 and up to 4096 floats whose 16-byte vectors do not line
+// up (a width that is not a multiple of 4, or an unaligned pointer): ln_bwd_vec's
+// scheme with vectors at 4-byte addresses, a wave per row up to 1024 floats (no
+// barrier in the row sums, four rows' loads in flight per workgroup).  Each row
+// is read once; a thread reads dy before it writes dx at the same columns, so dx
+// may alias dy.  Measured on MI355X at 8191 x 1001: 20-21 us against 24.0 in
+// 4-byte columns, and the slots' sum 4 us against 11 (their rows are padded to
+// whole vectors, so one launch of sum_slots_tile takes any width).
+template <int TPR, int VPT, bool KEEP>
+__global__ __launch_bounds__(kBlock) void ln_bwd_any(LnBwdArgs a) {
+    constexpr int RPB = kBlock / TPR;
+    constexpr int NW = TPR / kWave;
+    __shared__ float lds[4][kBlock / kWave];
+    const int t = threadIdx.x % TPR;
+    const int sub = threadIdx.x / TPR;
+    const RowSpan w(a.cols);
+    const float n = static_cast<float>(a.cols);
+    const float invF = 1.0f / n;  // Model.cpp:7799
+    f4 gm[VPT], dg[VPT], db[VPT];
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        gm[j] = a.g ? ld_slot<false>(a.g, j * TPR + t, w, 1.0f) : f4(1.0f);
+        dg[j] = f4(0.0f);
+        db[j] = f4(0.0f);
+    }
+    const int64_t step = static_cast<int64_t>(gridDim.x) * RPB;
+    auto load_rows = [&](int64_t b, f4* xo, f4* go) {
+        const int64_t r = b + sub;
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) {
+            xo[j] = r < a.rows ? ld_slot<true>(a.x + r * a.cols, j * TPR + t, w, 0.0f) : f4(0.0f);
+            go[j] = r < a.rows ? ld_slot<true>(a.dy + r * a.cols, j * TPR + t, w, 0.0f) : f4(0.0f);
+        }
+    };
+    f4 xv[VPT], gv[VPT];
+    load_rows(static_cast<int64_t>(blockIdx.x) * RPB, xv, gv);
+    for (int64_t base = static_cast<int64_t>(blockIdx.x) * RPB; base < a.rows; base += step) {
+        const int64_t row = base + sub;
+        f4 xn[VPT], gn[VPT];
+        load_rows(base + step, xn, gn);  // the next group's loads in flight during the reductions
+        float s = 0.0f, s1 = 0.0f;
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) {
+            s += hsum(xv[j]);
+            s1 += hsum(gv[j] * gm[j]);
+        }
+        row_sum2<NW>(s, s1, lds[0], lds[1], sub);
+        const float mean = s / n;  // :7765-7768
+        float q = 0.0f, p2 = 0.0f;
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) {
+            const int live = w.count(j * TPR + t);
+            f4 d = xv[j] - mean;
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                if (e >= live) d[e] = 0.0f;
+            q += (d.x * d.x + d.y * d.y) + (d.z * d.z + d.w * d.w);
+            p2 += hsum(gv[j] * gm[j] * d);
+        }
+        row_sum2<NW>(q, p2, lds[2], lds[3], sub);
+        const float var = q / n;                          // :7770-7776
+        const float inv_std = 1.0f / sqrtf(var + a.eps);  // :7777
+        const float s2 = p2 * inv_std;
+        const float k = inv_std * invF;
+        if (row < a.rows) {
+#pragma unroll
+            for (int j = 0; j < VPT; ++j) {  // :7783-7805
+                const int c4 = j * TPR + t;
+                const f4 xh = (xv[j] - mean) * inv_std;
+                const f4 dxh = gv[j] * gm[j];
+                dg[j] += gv[j] * xh;  // past the row's end gv is 0
+                db[j] += gv[j];
+                f4 o = k * ((n * dxh - s1) - xh * s2);
+                if (a.acc) o = ld_slot<true>(a.dx + row * a.cols, c4, w, 0.0f) + o;
+                st_slot<KEEP>(a.dx + row * a.cols, c4, w, o);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) {
+            xv[j] = xn[j];
+            gv[j] = gn[j];
+        }
+    }
+    if (!a.part) return;
+    // One slot per workgroup, as ln_bwd_vec.
+    float* p = a.part + static_cast<int64_t>(blockIdx.x) * slot_floats(a.cols);
+    if constexpr (RPB > 1) {
+        __shared__ f4 comb[2 * TPR * VPT];
+        for (int r = 0; r < RPB; ++r) {
+            if (sub == r) {
+#pragma unroll
+                for (int j = 0; j < VPT; ++j) {
+                    const int i = j * TPR + t;
+                    comb[i] = r == 0 ? dg[j] : comb[i] + dg[j];
+                    comb[TPR * VPT + i] = r == 0 ? db[j] : comb[TPR * VPT + i] + db[j];
+                }
+            }
+            __syncthreads();
+        }
+        if (sub != 0) return;
+#pragma unroll
+        for (int j = 0; j < VPT; ++j) {
+            dg[j] = comb[j * TPR + t];
+            db[j] = comb[TPR * VPT + j * TPR + t];
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        st_slot<true>(p, j * TPR + t, w, dg[j]);
+        st_slot<true>(p + a.cols, j * TPR + t, w, db[j]);
     }
 }
 
@@ -1108,17 +1215,17 @@ int ln_bwd_persistent(mimir_ctx* ctx, LnBwdArgs a, int64_t groups, float* dgamma
     float* tmp = nullptr;
     if (dgamma) {  // partial slots, then room for the second level of their sum
         void* s = nullptr;
-        const size_t bytes = sizeof(float) * static_cast<size_t>((nslots + kGroups) * 2 * a.cols);
+        const size_t bytes = sizeof(float) * static_cast<size_t>((nslots + kGroups) * slot_floats(a.cols));
         if (int st = get_scratch(ctx, fixed, bytes, &s)) return st;
         a.part = static_cast<float*>(s);
-        tmp = a.part + nslots * 2 * a.cols;
+        tmp = a.part + nslots * slot_floats(a.cols);
     }
     run(static_cast<unsigned>(grid), a);
     if (int st = launched(ctx, name)) return st;
     if (!dgamma) return MIMIR_OK;
     // dbeta null: sum only the dgamma half.
-    return launch_sum_slots(ctx, a.part, nslots, 2 * a.cols, dbeta ? 2 * a.cols : a.cols, dgamma, dbeta, a.cols,
-                            true, tmp);
+    return launch_sum_slots(ctx, a.part, nslots, slot_floats(a.cols), dbeta ? 2 * a.cols : a.cols, dgamma, dbeta,
+                            a.cols, true, tmp);
 }
 
 template <int TPR, int VPT, int BS>
@@ -1139,6 +1246,16 @@ int launch_ln_bwd_scalar(mimir_ctx* ctx, LnBwdArgs a, float* dgamma, float* dbet
                                  if (ctx->keep_outputs)
                                      ln_bwd_scalar<TPR, VPT, true><<<grid, kBlock, 0, ctx->stream>>>(la);
                                  else ln_bwd_scalar<TPR, VPT, false><<<grid, kBlock, 0, ctx->stream>>>(la);
+                             });
+}
+
+template <int TPR, int VPT>
+int launch_ln_bwd_any(mimir_ctx* ctx, LnBwdArgs a, float* dgamma, float* dbeta, const ScratchSpan* fixed) {
+    constexpr int RPB = kBlock / TPR;
+    return ln_bwd_persistent(ctx, a, (a.rows + RPB - 1) / RPB, dgamma, dbeta, "ln_bwd_any", fixed,
+                             [ctx](unsigned grid, const LnBwdArgs& la) {
+                                 if (ctx->keep_outputs) ln_bwd_any<TPR, VPT, true><<<grid, kBlock, 0, ctx->stream>>>(la);
+                                 else ln_bwd_any<TPR, VPT, false><<<grid, kBlock, 0, ctx->stream>>>(la);
                              });
 }
 
@@ -2169,10 +2286,13 @@ int layernorm_bwd(mimir_ctx* ctx, const float* x, const float* dy, const float* 
         MIMIR_ROW_SHAPES(MIMIR_LNBWD_CASE)
 #undef MIMIR_LNBWD_CASE
     }
-    if (!vec && n <= 256) return launch_ln_bwd_scalar<64, 4>(ctx, a, dgamma, dbeta, fixed);
-    if (!vec && n <= 1024) return launch_ln_bwd_scalar<64, 16>(ctx, a, dgamma, dbeta, fixed);
-    if (!vec && n <= 2048) return launch_ln_bwd_scalar<128, 16>(ctx, a, dgamma, dbeta, fixed);
-    if (!vec && n <= 4096) return launch_ln_bwd_scalar<256, 16>(ctx, a, dgamma, dbeta, fixed);
+    if (!vec) {
+        if (n <= 256) return launch_ln_bwd_any<64, 1>(ctx, a, dgamma, dbeta, fixed);
+        if (n <= 512) return launch_ln_bwd_any<64, 2>(ctx, a, dgamma, dbeta, fixed);
+        if (n <= 1024) return launch_ln_bwd_any<64, 4>(ctx, a, dgamma, dbeta, fixed);
+        if (n <= 2048) return launch_ln_bwd_any<128, 4>(ctx, a, dgamma, dbeta, fixed);
+        if (n <= 4096) return launch_ln_bwd_any<256, 4>(ctx, a, dgamma, dbeta, fixed);
+    }
     return ln_bwd_generic_run(ctx, a, dgamma, dbeta, fixed);
 }
 

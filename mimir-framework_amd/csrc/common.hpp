@@ -103,6 +103,57 @@ __device__ __forceinline__ void st_out(float* p, f4 v) {
 }
 
 // ---------------------------------------------------------------------------
+// Rows of any width and any 4-byte alignment in 16-byte vectors: gfx950 loads
+// and stores 16 bytes at any 4-byte address, so only the last vector of a row,
+// where fewer than four floats are left, goes in single ones.
+// ---------------------------------------------------------------------------
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+
+struct RowSpan {
+    int full, rem;  // whole vectors, floats left
+    __device__ __forceinline__ explicit RowSpan(int64_t cols)
+        : full(static_cast<int>(cols >> 2)), rem(static_cast<int>(cols & 3)) {}
+    // Floats of vector c4 inside the row.
+    __device__ __forceinline__ int count(int c4) const { return c4 < full ? 4 : c4 == full ? rem : 0; }
+};
+
+// Vector c4 of a row, `fill` past its end.
+template <bool NT>
+__device__ __forceinline__ f4 ld_slot(const float* row, int c4, const RowSpan& w, float fill) {
+    f4 v(fill);
+    if (c4 < w.full) {
+        const f4u* p = reinterpret_cast<const f4u*>(row + 4 * c4);
+        if constexpr (NT) v = __builtin_nontemporal_load(p);
+        else v = *p;
+    } else if (c4 == w.full) {
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+            if (e < w.rem) v[e] = row[4 * c4 + e];
+    }
+    return v;
+}
+
+template <bool KEEP>
+__device__ __forceinline__ void st_slot(float* row, int c4, const RowSpan& w, f4 v) {
+    if (c4 < w.full) {
+        gptr<f4u> g = (gptr<f4u>)(row + 4 * c4);
+        if constexpr (KEEP) {
+            *g = v;
+        } else {
+            asm volatile("" : "+v"(g));  // as in st_stream
+            __builtin_nontemporal_store(static_cast<f4u>(v), g);
+        }
+    } else if (c4 == w.full) {
+#pragma unroll
+        for (int e = 0; e < 3; ++e)
+            if (e < w.rem) {
+                if constexpr (KEEP) row[4 * c4 + e] = v[e];
+                else st_stream(row + 4 * c4 + e, v[e]);
+            }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // DPP wave reductions
 // ---------------------------------------------------------------------------
 enum : int {

@@ -5,8 +5,8 @@
 // the row max and the sum of exponentials are wave-uniform DPP reductions, so
 // each element is read from HBM once and written once.  Rows too wide for
 // the register budget are split over many workgroups (longrow.hip); rows of
-// a width that is not a multiple of 4, or unaligned, are held in registers
-// with 4-byte columns up to 4096 floats (softmax_rows_scalar); wider
+// a width that is not a multiple of 4, or unaligned, are held in registers in
+// vectors at 4-byte addresses up to 16384 floats (softmax_rows_any); wider
 // unaligned rows take one workgroup per row with three strided passes.
 //
 // Arithmetic (per row): m = max_j x[j]; e[j] = expf(x[j] - m); s = sum e[j];
@@ -125,53 +125,59 @@ __global__ __launch_bounds__(kBlock) void softmax_rows_generic(SoftmaxArgs a) {
     }
 }
 
-// Rows the vector kernel cannot take (a width that is not a multiple of 4,
-// or unaligned pointers), up to kBlock*VPT floats: the row held in registers
-// with 4-byte columns, one kBlock-thread workgroup per row -- one read of
-// the row, and the same max / sum / finish as softmax_rows_generic.
-template <int MODE, int VPT, bool KEEP>
-__global__ __launch_bounds__(kBlock) void softmax_rows_scalar(SoftmaxArgs a) {
-    constexpr int NW = kBlock / kWave;
-    __shared__ float lds[2][NW];
-    const int t = threadIdx.x;
-    const int64_t base = static_cast<int64_t>(blockIdx.x) * a.cols;
-    float v[VPT], e[VPT];
+// Rows the vector kernel cannot take (a width that is not a multiple of 4, or
+// unaligned pointers), up to 16384 floats: the row in registers as 16-byte
+// vectors at 4-byte addresses, TPR threads per row (a wave up to 2048 floats: no
+// barrier in its reductions; a workgroup above) -- one read of the row, and the
+// same max / sum / finish as softmax_rows_generic.  Measured on
+// MI355X at 8191 x 1001: 11.4-12.7 us against 19.5 in 4-byte columns, one
+// workgroup per row; 40000 x 1001 57 / 81 us.
+template <int MODE, int TPR, int VPT, bool KEEP>
+__global__ __launch_bounds__(kBlock) void softmax_rows_any(SoftmaxArgs a) {
+    constexpr int RPB = kBlock / TPR, NW = TPR / kWave;
+    __shared__ float lds[2][kBlock / kWave];
+    const int t = threadIdx.x % TPR, sub = threadIdx.x / TPR;
+    const int64_t row = static_cast<int64_t>(blockIdx.x) * RPB + sub;
+    if constexpr (NW == 1) {
+        if (row >= a.rows) return;  // whole waves; RPB == 1 otherwise
+    }
+    const int64_t base = row * a.cols;
+    const RowSpan w(a.cols);
+    f4 v[VPT], e[VPT];
     float m = -INFINITY;
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
-        const int64_t c = static_cast<int64_t>(j) * kBlock + t;
-        v[j] = c < a.cols ? __builtin_nontemporal_load(a.x + base + c) : 0.0f;
-        if (c < a.cols) m = fmaxf(m, v[j]);
+        v[j] = ld_slot<true>(a.x + base, j * TPR + t, w, -INFINITY);
+        m = fmaxf(m, fmaxf(fmaxf(v[j].x, v[j].y), fmaxf(v[j].z, v[j].w)));
     }
-    m = block_max<NW>(m, lds[0]);
+    m = row_max<NW>(m, lds[0], sub);
     float s = 0.0f;
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
-        e[j] = 0.0f;
-        if (static_cast<int64_t>(j) * kBlock + t < a.cols) {
-            e[j] = expf(v[j] - m);
-            s += e[j];
-        }
+        const int live = w.count(j * TPR + t);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) e[j][k] = k < live ? expf(v[j][k] - m) : 0.0f;
+        s += (e[j].x + e[j].y) + (e[j].z + e[j].w);
     }
     float sum, aux;
-    row_constants<MODE>(block_sum<NW>(s, lds[1]), &sum, &aux);
+    row_constants<MODE>(row_sum<NW>(s, lds[1], sub), &sum, &aux);
 #pragma unroll
     for (int j = 0; j < VPT; ++j) {
-        const int64_t c = static_cast<int64_t>(j) * kBlock + t;
-        if (c < a.cols) {
-            const float o = finish<MODE>(v[j], e[j], m, sum, aux);
-            if constexpr (KEEP) a.y[base + c] = o;
-            else st_stream(a.y + base + c, o);
-        }
+        f4 o;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) o[k] = finish<MODE>(v[j][k], e[j][k], m, sum, aux);
+        st_slot<KEEP>(a.y + base, j * TPR + t, w, o);
     }
 }
 
-template <int MODE, int VPT>
-int launch_scalar(mimir_ctx* ctx, const SoftmaxArgs& a) {
-    const unsigned grid = static_cast<unsigned>(a.rows);
-    if (ctx->keep_outputs) softmax_rows_scalar<MODE, VPT, true><<<grid, kBlock, 0, ctx->stream>>>(a);
-    else softmax_rows_scalar<MODE, VPT, false><<<grid, kBlock, 0, ctx->stream>>>(a);
-    return launched(ctx, "softmax_rows_scalar");
+template <int MODE, int TPR, int VPT>
+int launch_any(mimir_ctx* ctx, const SoftmaxArgs& a) {
+    unsigned grid;
+    if (!grid_for(a.rows, kBlock / TPR, kBlock, &grid))
+        return fail(ctx, MIMIR_EINVAL, "softmax: %lld rows exceed the grid limit", (long long)a.rows);
+    if (ctx->keep_outputs) softmax_rows_any<MODE, TPR, VPT, true><<<grid, kBlock, 0, ctx->stream>>>(a);
+    else softmax_rows_any<MODE, TPR, VPT, false><<<grid, kBlock, 0, ctx->stream>>>(a);
+    return launched(ctx, "softmax_rows_any");
 }
 
 template <int MODE, int TPR, int VPT, int BS>
@@ -198,9 +204,15 @@ int dispatch(mimir_ctx* ctx, const SoftmaxArgs& a) {
     }
     if (!dispatch_fits(a.rows, kBlock))
         return fail(ctx, MIMIR_EINVAL, "softmax: %lld rows exceed the grid limit", (long long)a.rows);
-    if (!vec && a.cols <= 4 * kBlock) return launch_scalar<MODE, 4>(ctx, a);
-    if (!vec && a.cols <= 8 * kBlock) return launch_scalar<MODE, 8>(ctx, a);
-    if (!vec && a.cols <= 16 * kBlock) return launch_scalar<MODE, 16>(ctx, a);
+    if (!vec) {
+        if (a.cols <= 256) return launch_any<MODE, 64, 1>(ctx, a);
+        if (a.cols <= 512) return launch_any<MODE, 64, 2>(ctx, a);
+        if (a.cols <= 1024) return launch_any<MODE, 64, 4>(ctx, a);
+        if (a.cols <= 2048) return launch_any<MODE, 64, 8>(ctx, a);
+        if (a.cols <= 4096) return launch_any<MODE, 256, 4>(ctx, a);
+        if (a.cols <= 8192) return launch_any<MODE, 256, 8>(ctx, a);
+        if (a.cols <= 16384) return launch_any<MODE, 256, 16>(ctx, a);
+    }
     softmax_rows_generic<MODE><<<static_cast<unsigned>(a.rows), kBlock, 0, ctx->stream>>>(a);
     return launched(ctx, "softmax_rows_generic");
 }
