@@ -26,15 +26,16 @@
 // whose blocks fit kDsBytes), written and read once.
 //
 // Bound by latency and the barriers as much as by the matrix cores: at 8 x 32
-// heads x 1024 x 128, causal, step 2 takes 1015 us with the matrix pipes busy
-// 41% of the cycles, step 1 465 us, step 3 245 us: 1.71 ms = 101 TFLOP/s of the
+// heads x 1024 x 128, causal, step 2 takes 925 us with the matrix pipes busy
+// 45% of the cycles (1020 us with its tile in one buffer and three barriers),
+// step 1 445 us, step 3 235 us: 1.53 ms = 112 TFLOP/s of the
 // five products, against 3.30 ms for the same products as library fp32 GEMMs
 // with P and dS in memory; 64 heads x 512 x 64 120 / 964 us, 128 heads x 100 x 64
 // 42 / 1059 us (the GEMMs ran sequence by sequence).
 //
 // LDS of step 2: Q rows, dO rows, Q^T and dO^T of one tile in bf16 planes
 // (114 KB at 128 dimensions), the pairs' P (16 KB) and the tile's max / sum /
-// delta.  One buffer: the next tile waits in registers.
+// delta.  One buffer, each half refilled while the other is read.
 #include "attention_tile.hpp"
 #include "internal.hpp"
 
@@ -130,7 +131,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_kv(BwdArgs a) {
     constexpr int kRole = Rows::kBytes + Cols::kBytes;  // the rows and columns one role reads
     __shared__ __attribute__((aligned(16))) char lds[2 * kRole];
     __shared__ __attribute__((aligned(16))) f4 pshare[kWaves / 2][4][kWave];
-    __shared__ __attribute__((aligned(16))) float tstats[3][kTileRows];
+    __shared__ __attribute__((aligned(16))) float tstats[2][3][kTileRows];
 
     uint32_t bh, kblock;
     const uint32_t split = blockIdx.x % static_cast<uint32_t>(a.splits);
@@ -165,21 +166,29 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_kv(BwdArgs a) {
     drows.init(a.c.ld_dout, a.head_dim);
     dcols.init(a.c.ld_dout, a.head_dim);
     float stat = 0.f;
-    auto load = [&](int t) {
+    // Role 0 reads Q rows and dO columns, role 1 dO rows and Q columns.
+    auto load_rows = [&](int t) {
         qrows.load(q, t, a.c.ld_q, a.q_len, a.head_dim);
-        dcols.load(dout, t, a.c.ld_dout, a.q_len, a.head_dim);
         drows.load(dout, t, a.c.ld_dout, a.q_len, a.head_dim);
-        qcols.load(q, t, a.c.ld_q, a.q_len, a.head_dim);
         if (threadIdx.x < 3 * kTileRows) stat = stats[threadIdx.x / kTileRows * plane + t * kTileRows + threadIdx.x % kTileRows];
     };
-    auto stash = [&]() {  // role 0 reads Q rows and dO columns, role 1 dO rows and Q columns
-        qrows.stash(lds);
-        dcols.stash(lds + Rows::kBytes);
-        drows.stash(lds + kRole);
-        qcols.stash(lds + kRole + Rows::kBytes);
-        if (threadIdx.x < 3 * kTileRows) tstats[threadIdx.x / kTileRows][threadIdx.x % kTileRows] = stat;
+    auto load_cols = [&](int t) {
+        dcols.load(dout, t, a.c.ld_dout, a.q_len, a.head_dim);
+        qcols.load(q, t, a.c.ld_q, a.q_len, a.head_dim);
     };
-    if (t0 < t_end) load(t0);
+    auto stash_rows = [&](int t) {
+        qrows.stash(lds);
+        drows.stash(lds + kRole);
+        if (threadIdx.x < 3 * kTileRows) tstats[t & 1][threadIdx.x / kTileRows][threadIdx.x % kTileRows] = stat;
+    };
+    auto stash_cols = [&]() {
+        dcols.stash(lds + Rows::kBytes);
+        qcols.stash(lds + kRole + Rows::kBytes);
+    };
+    if (t0 < t_end) {
+        load_rows(t0);
+        load_cols(t0);
+    }
     Split8 own[kC];
     row_operand<DP, VEC>((role ? v : k) + static_cast<int64_t>(min(key, a.kv_len - 1)) * a.c.ld_kv, hf, a.head_dim, 1.0f, own);
     f16v acc[kDb];
@@ -188,12 +197,24 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_kv(BwdArgs a) {
     const char* const rows = lds + role * kRole;
     const char* const cols = rows + Rows::kBytes;
 
+    if (t0 < t_end) {
+        stash_rows(t0);
+        load_rows(min(t0 + 1, t_end - 1));
+    }
+    __syncthreads();
+    // A tile has two phases, the first reading its rows and the second its
+    // columns, so each phase's half of LDS is refilled during the other.  Of the
+    // two waves of a SIMD one refills before its products and one after, so one's
+    // vector work runs beside the other's MFMAs.  Past the last tile the refills
+    // repeat it.
     for (int t = t0; t < t_end; ++t) {
-        stash();
-        __syncthreads();
-        load(min(t + 1, t_end - 1));
+        const float(*const ts)[kTileRows] = tstats[t & 1];
         const bool work = pair_in && t >= pair_t0;
         f16v x = f16v{};
+        if (role) {
+            stash_cols();
+            load_cols(min(t + 1, t_end - 1));
+        }
         if (work) {
 #pragma unroll
             for (int c = 0; c < kC; ++c) x = mfma_split(Rows::at(rows, li, hf, c), own[c], x);
@@ -202,8 +223,8 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_kv(BwdArgs a) {
                 const bool edge = k0 + kTileRows > a.kv_len || (a.c.causal && t == ktile);
 #pragma unroll
                 for (int r = 0; r < 16; r += 4) {
-                    const f4 m = *reinterpret_cast<const f4*>(&tstats[0][8 * (r / 4) + 4 * hf]);
-                    const f4 inv = *reinterpret_cast<const f4*>(&tstats[1][8 * (r / 4) + 4 * hf]);
+                    const f4 m = *reinterpret_cast<const f4*>(&ts[0][8 * (r / 4) + 4 * hf]);
+                    const f4 inv = *reinterpret_cast<const f4*>(&ts[1][8 * (r / 4) + 4 * hf]);
                     f4 p;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
@@ -216,14 +237,22 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_kv(BwdArgs a) {
                 }
             }
         }
+        if (!role) {
+            stash_cols();
+            load_cols(min(t + 1, t_end - 1));
+        }
         __syncthreads();
+        if (role) {
+            stash_rows(t + 1);
+            load_rows(min(t + 2, t_end - 1));
+        }
         if (work) {
             if (role == 1) {
                 float* block = a.ds + ((static_cast<int64_t>(bh) * a.k_tiles + ktile) * a.q_tiles + t) * kBlockFloats;
 #pragma unroll
                 for (int r = 0; r < 16; r += 4) {
                     const f4 p = pshare[pair][r / 4][lane];
-                    const f4 delta = *reinterpret_cast<const f4*>(&tstats[2][8 * (r / 4) + 4 * hf]);
+                    const f4 delta = *reinterpret_cast<const f4*>(&ts[2][8 * (r / 4) + 4 * hf]);
                     f4 ds;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
@@ -245,6 +274,10 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_kv(BwdArgs a) {
 #pragma unroll
                 for (int d = 0; d < kDb; ++d) acc[d] = mfma_split(Cols::at(cols, li, hf, d, c), s, acc[d]);
             }
+        }
+        if (!role) {
+            stash_rows(t + 1);
+            load_rows(min(t + 2, t_end - 1));
         }
         __syncthreads();
     }
