@@ -1,7 +1,8 @@
 // gemm.hip -- the plain fp32 matrix products around the attention core (the
 // QKV and output projections of the attention layers, and the per-head
-// products of the attention backward), through hipBLASLt on the context's
-// stream, with rocBLAS for any product hipBLASLt offers no algorithm for (or
+// products of wide heads' backward): the small and the very large ones in
+// gemm_split.hip, the others through hipBLASLt on the context's stream, with
+// rocBLAS for any product hipBLASLt offers no algorithm for (or
 // every product under MIMIR_TUNE blas=0).  These are library GEMMs: the
 // path's own kernels are the fused core between them (attention.hip) and the
 // backward's row passes (attention_bwd.hip).
@@ -195,6 +196,11 @@ int gemm_f32_ex(mimir_ctx* ctx, bool trans_a, bool trans_b, int64_t M, int64_t N
     const int64_t lim = INT32_MAX;
     if (M > lim || N > lim || K > lim || lda > lim || ldb > lim || ldc > lim || batch > lim)
         return fail(ctx, MIMIR_EINVAL, "matrix product: dimensions exceed the 32-bit library limit");
+    bool taken;
+    if (const int st = gemm_split(ctx, trans_a, trans_b, M, N, K, alpha, A, lda, stride_a, B, ldb, stride_b, beta, C,
+                                  ldc, stride_c, batch, &taken);
+        st != MIMIR_OK || taken)
+        return st;
     // Row-major C = op(A) op(B) is column-major C^T = op(B)^T op(A)^T: the
     // operands swap and each keeps its own transpose flag.  K == 0 with
     // beta == 0 gives C = 0 (an empty sum), which rocBLAS takes.

@@ -123,6 +123,11 @@ int gemm_f32_ex(mimir_ctx* ctx, bool trans_a, bool trans_b, int64_t M, int64_t N
                 const float* A, int64_t lda, int64_t stride_a, const float* B, int64_t ldb, int64_t stride_b,
                 float beta, float* C, int64_t ldc, int64_t stride_c, int64_t batch);
 void gemm_release(mimir_ctx* ctx);
+// The products that run on the bf16 matrix cores with split operands instead of
+// the library (gemm_split.hip); *taken says whether this one does.
+int gemm_split(mimir_ctx* ctx, bool trans_a, bool trans_b, int64_t M, int64_t N, int64_t K, float alpha, const float* A,
+               int64_t lda, int64_t stride_a, const float* B, int64_t ldb, int64_t stride_b, float beta, float* C,
+               int64_t ldc, int64_t stride_c, int64_t batch, bool* taken);
 // Whether products go to hipBLASLt (unless MIMIR_TUNE blas=0), where the
 // transposed-operand forms run as fast as the plain ones.
 bool gemm_lt(mimir_ctx* ctx);

@@ -76,6 +76,7 @@ struct Tuning {
     int embed_bwd_onepass = -1; // embedding backward: the counting sort in one launch where it applies (-1, 1) or
                                 // in three (0)
     int blas_lt = -1;           // library products: hipBLASLt first (-1, 1) or rocBLAS only (0)
+    int gemm = 0;               // matrix products: 128 (gemm_tile), 16 or 4 (waves of gemm_strip), 1 (library); 0: by size
     int lnbwd_narrow = -1;      // LayerNorm backward, rows <= 64 floats: several rows per wave (-1, 1) or not (0)
     int lr_cpw = 0;             // long rows: 4096-float chunks per workgroup of the first pass (1, 2, 4; 0: measured default)
     int ew_bs = 0;              // workgroup size of the one-float4-per-thread streaming kernels (64 .. 1024; 0: default)
@@ -128,6 +129,7 @@ inline Tuning read_tuning() {
         else if (!std::strcmp(k, "embruns")) t.embed_bwd_runs = std::atoi(v);
         else if (!std::strcmp(k, "emb1pass")) t.embed_bwd_onepass = std::atoi(v);
         else if (!std::strcmp(k, "blas")) t.blas_lt = std::atoi(v);
+        else if (!std::strcmp(k, "gemm")) t.gemm = std::atoi(v);
         else if (!std::strcmp(k, "lnbwd_narrow")) t.lnbwd_narrow = std::atoi(v);
         else if (!std::strcmp(k, "lrcpw")) t.lr_cpw = std::atoi(v);
         else if (!std::strcmp(k, "ewbs")) t.ew_bs = std::atoi(v);
