@@ -1330,15 +1330,15 @@ __device__ __forceinline__ int64_t run_end(const uint32_t* keys, int64_t i, int6
 
 // Runs of at least kLongRun tokens (a frequent id) are summed in two levels
 // instead of one token after another: the run's positions are cut at the
-// multiples of kLongRun, embed_bwd_seg_partial sums each segment's dy rows
+// multiples of kLongRun, embed_bwd_rows_seg sums each segment's dy rows
 // (token order) into a slot of partial rows, all segments at once, and
 // embed_bwd_seg_combine adds the run's slots onto the gradient row.  The
 // workgroup at a run's first segment also lists the run (id, head, end) for
 // the combine, whose grid then covers only the long runs.  The result is
 // deterministic; it is the reference's sequential sum regrouped, so it
 // agrees with it to the rounding of a float32 sum (the path's tolerance for
-// sums), not bit for bit.  Shorter runs stay with embed_bwd_rows_vec, which
-// adds in token order (bit-exact).
+// sums), not bit for bit.  Shorter runs are summed by embed_bwd_rows_seg
+// in token order (bit-exact).
 constexpr int kLongRun = 32;
 constexpr int kLongBatch = 16;
 
@@ -1419,47 +1419,6 @@ __device__ __forceinline__ LongRun long_run_at(const uint32_t* keys, int64_t p, 
     return r;
 }
 
-// First level: workgroup (m, o) of position p = m * kLongRun in a long run
-// sums the dy rows of its segment, positions p .. min(p + kLongRun, end) - 1
-// (and head .. p - 1 before them when p is the run's first multiple), in
-// token order, into partial slot m, for its o-th block of kSegCols 16-byte
-// columns (one per thread).  Each thread requests kSegRows tokens' rows
-// before adding the first.
-constexpr int kSegCols = 256;
-constexpr int kSegRows = 16;
-__global__ __launch_bounds__(kSegCols) void embed_bwd_seg_partial(const uint32_t* keys, const uint32_t* toks,
-                                                                  int64_t n, uint32_t vocab, const float* dy,
-                                                                  float* part, int64_t dim4, LongRunList list) {
-    const int64_t m = blockIdx.x;
-    const int64_t p = m * kLongRun;
-    if (p >= n) return;
-    const LongRun r = long_run_at(keys, p, n, vocab);
-    if (!r.is_long) return;
-    if (r.first && blockIdx.y == 0 && threadIdx.x == 0) list_long_run(list, r.id, r.head, r.end);
-    const int64_t c = static_cast<int64_t>(blockIdx.y) * kSegCols + threadIdx.x;
-    if (c >= dim4) return;  // after the ballots of long_run_at
-    const int64_t s0 = r.first ? r.head : p;
-    const int64_t s1 = p + kLongRun < r.end ? p + kLongRun : r.end;
-    const f4* src = reinterpret_cast<const f4*>(dy);
-    f4 acc;
-    bool started = false;
-    for (int64_t j = s0; j < s1; j += kSegRows) {
-        f4 v[kSegRows];
-#pragma unroll
-        for (int u = 0; u < kSegRows; ++u)
-            if (j + u < s1) v[u] = __builtin_nontemporal_load(src + static_cast<int64_t>(toks[j + u]) * dim4 + c);
-        __builtin_amdgcn_sched_barrier(0);  // the batch's loads are all issued before the first add
-#pragma unroll
-        for (int u = 0; u < kSegRows; ++u) {
-            if (j + u < s1) {
-                acc = started ? acc + v[u] : v[u];
-                started = true;
-            }
-        }
-    }
-    reinterpret_cast<f4*>(part)[m * dim4 + c] = acc;
-}
-
 // Second level: work item (run, column block) adds the run's partial slots
 // onto kCombineCols 16-byte columns of the id's gradient row.  Each of the
 // workgroup's kCombineGroups waves sums every kCombineGroups-th slot
@@ -1522,89 +1481,62 @@ __global__ __launch_bounds__(kWave * kCombineGroups) void embed_bwd_seg_combine(
     }
 }
 
-// One workgroup per sorted position.  The first position of each id's run
-// of fewer than kLongRun tokens (every run without `long_runs`) adds the
-// run's dy rows (token order, the sort is stable) onto the id's gradient row;
-// every other position leaves at once.  Each thread owns CPT 16-byte columns
-// TPT apart.  The first token's row and the gradient row are requested
-// before the run's end is known, so a run of one (the common case) waits for
-// two memory round trips; the rest of a run is loaded kRunBatch tokens at a
-// time, then added in token order.  Most workgroups leave at once, so the
-// kernel is kept small in registers: two 1024-thread workgroups fit a CU.
-constexpr int kRunBatch = 4;
+// The rows of a run, and of a long run's segments.  A workgroup of TPT threads
+// takes whole 16-byte columns, one per thread and column group.  Bound by memory
+// where ids are many and by latency where tokens are few: a run of up to 31 rows
+// is a serial chain, so the run's tokens are read at once, one per lane (each
+// wave gets its own copy, whichever columns it has), and kRowBatch rows are in
+// flight before the first is added, which keeps the kernel at 64 registers (two
+// 1024-thread workgroups a CU).  Rows are added in token order, the order of the
+// stable sort.  Measured on MI355X, Zipf ids, sort and sums: 8192 tokens of 5000
+// ids x 1024 75 -> 34 us against four rows in flight and a token read for each;
+// 16000 of 20000 x 500 83 -> 38; 4096 of 32000 x 4096 70 -> 53; 32768 of 32000 x 4096
+// 201 -> 185 (4.4 TB/s).
+constexpr int kRowBatch = 8;
 
-// The first token's row and the gradient row, for the CPT columns of this
-// thread that start at c0.
-template <int TPT, int CPT>
-__device__ __forceinline__ void embed_rows_load(const f4* g, const f4* src, uint32_t t0, int64_t c0, int64_t dim4,
-                                                f4 (&acc)[CPT], f4 (&v)[CPT]) {
+// acc += the dy rows of sorted positions j0 .. j1 - 1 in column c.  All lanes of
+// the wave; `c` may differ by lane, the positions not.
+__device__ __forceinline__ void embed_add_rows(f4& acc, const uint32_t* toks, int64_t j0, int64_t j1, const f4* src,
+                                               int64_t dim4, int64_t c) {
+    const int lane = threadIdx.x & (kWave - 1);
+    for (int64_t j = j0; j < j1; j += kWave) {
+        const int cnt = __builtin_amdgcn_readfirstlane(static_cast<int>(j1 - j < kWave ? j1 - j : kWave));
+        const int mine = lane < cnt ? static_cast<int>(toks[j + lane]) : 0;
+        for (int u0 = 0; u0 < cnt; u0 += kRowBatch) {
+            f4 v[kRowBatch];
 #pragma unroll
-    for (int k = 0; k < CPT; ++k) {
-        const int64_t c = c0 + static_cast<int64_t>(k) * TPT;
-        if (c < dim4) {
-            acc[k] = __builtin_nontemporal_load(g + c);
-            v[k] = __builtin_nontemporal_load(src + static_cast<int64_t>(t0) * dim4 + c);
-        }
-    }
-}
-
-// The run at sorted positions i .. end - 1 (first token t0, its row and the
-// gradient row already loaded for columns from threadIdx.x): adds the rows
-// in token order onto the gradient row, column group by column group.
-template <int TPT, int CPT>
-__device__ __forceinline__ void embed_rows_sum(int64_t i, int64_t end, uint32_t t0, const uint32_t* toks,
-                                               const f4* src, f4* g, int64_t dim4, f4 (&acc)[CPT], f4 (&v)[CPT]) {
-    int64_t c0 = threadIdx.x;
-    while (c0 < dim4) {
-#pragma unroll
-        for (int k = 0; k < CPT; ++k) acc[k] += v[k];
-        for (int64_t j = i + 1; j < end; j += kRunBatch) {
-            f4 w[kRunBatch][CPT];
-#pragma unroll
-            for (int u = 0; u < kRunBatch; ++u) {
-                if (j + u < end) {
-                    const int64_t row = static_cast<int64_t>(toks[j + u]) * dim4;
-#pragma unroll
-                    for (int k = 0; k < CPT; ++k) {
-                        const int64_t c = c0 + static_cast<int64_t>(k) * TPT;
-                        if (c < dim4) w[u][k] = __builtin_nontemporal_load(src + row + c);
-                    }
+            for (int u = 0; u < kRowBatch; ++u) {
+                if (u0 + u < cnt) {
+                    const uint32_t tok = static_cast<uint32_t>(__builtin_amdgcn_readlane(mine, u0 + u));
+                    v[u] = __builtin_nontemporal_load(src + static_cast<int64_t>(tok) * dim4 + c);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);  // the batch's loads are all issued before the first add
 #pragma unroll
-            for (int u = 0; u < kRunBatch; ++u) {
-                if (j + u < end) {
-#pragma unroll
-                    for (int k = 0; k < CPT; ++k) acc[k] += w[u][k];
-                }
-            }
+            for (int u = 0; u < kRowBatch; ++u)
+                if (u0 + u < cnt) acc += v[u];
         }
-#pragma unroll
-        for (int k = 0; k < CPT; ++k) {
-            const int64_t c = c0 + static_cast<int64_t>(k) * TPT;
-            if (c < dim4) st_stream(g + c, acc[k]);
-        }
-        c0 += static_cast<int64_t>(TPT) * CPT;
-        if (c0 < dim4) embed_rows_load<TPT, CPT>(g, src, t0, c0, dim4, acc, v);
     }
 }
 
-template <int TPT, int CPT>
-__device__ __forceinline__ void embed_rows_position(int64_t i, const uint32_t* keys, const uint32_t* toks, int64_t n,
-                                                    uint32_t vocab, const float* dy, float* grad, int64_t dim4,
-                                                    int long_runs) {
-    const uint32_t id = keys[i];
-    const uint32_t t0 = toks[i];
-    if (id >= vocab || (i > 0 && keys[i - 1] == id)) return;  // not a run's head
-    const f4* src = reinterpret_cast<const f4*>(dy);
-    f4* g = reinterpret_cast<f4*>(grad) + static_cast<int64_t>(id) * dim4;
-    f4 acc[CPT], v[CPT];
-    embed_rows_load<TPT, CPT>(g, src, t0, threadIdx.x, dim4, acc, v);
-    if (long_runs && i + kLongRun <= n && keys[i + kLongRun - 1] == id) return;  // a long run: segments
-    // Every lane of the wave takes part in the ballots of run_end.
-    const int64_t end = run_end(keys, i, n, id);
-    embed_rows_sum<TPT, CPT>(i, end, t0, toks, src, g, dim4, acc, v);
+// The run that starts at sorted position i with token tok: its dy rows added
+// onto the id's gradient row g.  The first token's row and the gradient row are
+// requested before end_of() tells the run's end (-1: a long run, left to the
+// segments), so a run of one, the common case, waits for two memory round trips.
+template <int TPT, class End>
+__device__ __forceinline__ void embed_run(int64_t i, uint32_t tok, End&& end_of, const uint32_t* toks, const f4* src,
+                                          f4* g, int64_t dim4) {
+    int64_t end = i;
+    for (int64_t c0 = threadIdx.x / kWave * kWave; c0 < dim4; c0 += TPT) {  // a wave past the last column leaves
+        const int64_t c = c0 + threadIdx.x % kWave, cc = c < dim4 ? c : dim4 - 1;
+        f4 acc = __builtin_nontemporal_load(g + cc);
+        const f4 v = __builtin_nontemporal_load(src + static_cast<int64_t>(tok) * dim4 + cc);
+        if (end == i) end = end_of();
+        if (end < 0) return;
+        acc += v;
+        embed_add_rows(acc, toks, i + 1, end, src, dim4, cc);
+        if (c < dim4) st_stream(g + c, acc);
+    }
 }
 
 // The runs of the counting sort, in ascending id order: (id, first sorted
@@ -1617,57 +1549,46 @@ struct RunList {
     const RunEntry* runs;
 };
 
-// Run j of the list (no workgroup when j is past the list's end), the same
-// sums as embed_rows_position at the run's head.
-template <int TPT, int CPT>
-__device__ __forceinline__ void embed_rows_run(int64_t j, const RunList& list, const uint32_t* toks,
-                                               const float* dy, float* grad, int64_t dim4, int long_runs) {
-    if (j >= *list.count) return;
-    const RunEntry e = list.runs[j];
-    if (long_runs && e.count >= static_cast<uint32_t>(kLongRun)) return;  // a long run: segments
-    const f4* src = reinterpret_cast<const f4*>(dy);
-    f4* g = reinterpret_cast<f4*>(grad) + static_cast<int64_t>(e.id) * dim4;
-    f4 acc[CPT], v[CPT];
-    embed_rows_load<TPT, CPT>(g, src, e.tok, threadIdx.x, dim4, acc, v);
-    embed_rows_sum<TPT, CPT>(e.start, static_cast<int64_t>(e.start) + e.count, e.tok, toks, src, g, dim4, acc, v);
-}
-
-// RUNS: workgroup j takes run j of the counting sort's list; otherwise
-// workgroup i takes sorted position i.  Separate instantiations, so each
-// form is compiled on its own.
-template <int TPT, int CPT, bool RUNS>
-__global__ __launch_bounds__(TPT) void embed_bwd_rows_vec(const uint32_t* keys, const uint32_t* toks, int64_t n,
-                                                          uint32_t vocab, const float* dy, float* grad, int64_t dim4,
-                                                          int long_runs, RunList runs) {
-    if constexpr (RUNS)
-        embed_rows_run<TPT, CPT>(blockIdx.x, runs, toks, dy, grad, dim4, long_runs);
-    else
-        embed_rows_position<TPT, CPT>(blockIdx.x, keys, toks, n, vocab, dy, grad, dim4, long_runs);
-}
-
 // The rows kernel and the long runs' first level in one launch, so the two
-// independent streams overlap: blocks [0, nslots) are the segments of
-// embed_bwd_seg_partial (dispatched first, so the long segments start before
-// the short rows), the blocks after them embed_bwd_rows_vec's (one per
-// listed run with RUNS, else one per sorted position), the segment blocks
-// each 1024 threads summing their segment's rows over whole 16-byte
-// columns with kMergedSegRows tokens' loads in flight.  The segment path is
-// kept small enough that the kernel stays at 64 registers, so two
-// 1024-thread workgroups still fit a CU (the rows path's turnover needs
-// them); its sums are embed_bwd_seg_partial's, in the same token order, bit
-// for bit.
-constexpr int kMergedSegRows = 8;
-template <bool RUNS>
-__global__ __launch_bounds__(1024, 8) void embed_bwd_rows_seg(const uint32_t* keys, const uint32_t* toks, int64_t n,
-                                                               uint32_t vocab, const float* dy, float* grad,
-                                                               float* part, int64_t dim4, LongRunList list,
-                                                               RunList runs) {
-    const int64_t nslots = (n + kLongRun - 1) / kLongRun;
+// independent streams overlap.  Blocks [0, nslots) (none without long runs) are
+// the segments, dispatched first: the one of position p = m * kLongRun in a long
+// run sums the dy rows of positions p .. min(p + kLongRun, end) - 1 (and head .. p
+// - 1 before them when p is the run's first multiple), in token order, into
+// partial slot m.  The blocks after them stride over the counting sort's list of
+// runs (RUNS), or over the sorted positions, where the first of each run does it
+// and the others leave.  At most kRowsGrid workgroups of 1024 threads: a workgroup
+// for each possible id is 6 us of empty ones at 32768 tokens of 8524 ids, and 4096
+// or fewer give up to 30 us of uneven ends.
+constexpr int64_t kRowsGrid = 8192;
+template <int TPT, bool RUNS>
+__global__ __launch_bounds__(TPT, 8) void embed_bwd_rows_seg(const uint32_t* keys, const uint32_t* toks, int64_t n,
+                                                             uint32_t vocab, const float* dy, float* grad, float* part,
+                                                             int64_t dim4, int64_t nslots, LongRunList list,
+                                                             RunList runs) {
+    const f4* src = reinterpret_cast<const f4*>(dy);
     if (blockIdx.x >= nslots) {
-        if constexpr (RUNS)
-            embed_rows_run<1024, 1>(blockIdx.x - nslots, runs, toks, dy, grad, dim4, 1);
-        else
-            embed_rows_position<1024, 1>(blockIdx.x - nslots, keys, toks, n, vocab, dy, grad, dim4, 1);
+        const int64_t step = gridDim.x - nslots;
+        const int64_t count = RUNS ? static_cast<int64_t>(*runs.count) : n;
+        for (int64_t j = blockIdx.x - nslots; j < count; j += step) {
+            if constexpr (RUNS) {
+                const RunEntry e = runs.runs[j];
+                if (nslots && e.count >= static_cast<uint32_t>(kLongRun)) continue;
+                embed_run<TPT>(
+                    e.start, e.tok, [&] { return static_cast<int64_t>(e.start) + e.count; }, toks, src,
+                    reinterpret_cast<f4*>(grad) + static_cast<int64_t>(e.id) * dim4, dim4);
+            } else {
+                const uint32_t id = keys[j];
+                const uint32_t tok = toks[j];
+                if (id >= vocab || (j > 0 && keys[j - 1] == id)) continue;  // not a run's head
+                embed_run<TPT>(
+                    j, tok,
+                    [&] {
+                        if (nslots && j + kLongRun <= n && keys[j + kLongRun - 1] == id) return int64_t{-1};
+                        return run_end(keys, j, n, id);
+                    },
+                    toks, src, reinterpret_cast<f4*>(grad) + static_cast<int64_t>(id) * dim4, dim4);
+            }
+        }
         return;
     }
     const int64_t m = blockIdx.x;
@@ -1678,25 +1599,11 @@ __global__ __launch_bounds__(1024, 8) void embed_bwd_rows_seg(const uint32_t* ke
     if (r.first && threadIdx.x == 0) list_long_run(list, r.id, r.head, r.end);
     const int64_t s0 = r.first ? r.head : p;
     const int64_t s1 = p + kLongRun < r.end ? p + kLongRun : r.end;
-    const f4* src = reinterpret_cast<const f4*>(dy);
-    for (int64_t c = threadIdx.x; c < dim4; c += 1024) {
-        f4 acc;
-        bool started = false;
-        for (int64_t j = s0; j < s1; j += kMergedSegRows) {
-            f4 v[kMergedSegRows];
-#pragma unroll
-            for (int u = 0; u < kMergedSegRows; ++u)
-                if (j + u < s1) v[u] = __builtin_nontemporal_load(src + static_cast<int64_t>(toks[j + u]) * dim4 + c);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int u = 0; u < kMergedSegRows; ++u) {
-                if (j + u < s1) {
-                    acc = started ? acc + v[u] : v[u];
-                    started = true;
-                }
-            }
-        }
-        reinterpret_cast<f4*>(part)[m * dim4 + c] = acc;
+    for (int64_t c0 = threadIdx.x / kWave * kWave; c0 < dim4; c0 += TPT) {
+        const int64_t c = c0 + threadIdx.x % kWave, cc = c < dim4 ? c : dim4 - 1;
+        f4 acc = f4{-0.0f, -0.0f, -0.0f, -0.0f};  // the sum starts from the first row as it is
+        embed_add_rows(acc, toks, s0, s1, src, dim4, cc);
+        if (c < dim4) reinterpret_cast<f4*>(part)[m * dim4 + c] = acc;
     }
 }
 
@@ -2179,55 +2086,28 @@ int embed_bwd(mimir_ctx* ctx, const void* ids, int64_t n_ids, const float* dy, f
     if (vec) {
         const uint32_t v = static_cast<uint32_t>(vocab);
         const int64_t dim4 = dim / 4;
-        const int lr = long_runs ? 1 : 0;
-        // Measured on MI355X at dim 4096 (MIMIR_TUNE gather=256/512/1024 picks a
-        // variant): one 16-byte column per thread in 1024-thread workgroups
-        // is fastest, 2-4 columns per thread in smaller ones ~2-4% slower.
-        const int tpt = ctx->tune.gather_tpt ? ctx->tune.gather_tpt : (dim4 >= 1024 ? 1024 : dim4 >= 512 ? 512 : 256);
-        // With the run list, a workgroup per run: at most min(n, vocab) of them.
-        const int64_t rows_grid = runs.count && vocab < n_ids ? vocab : n_ids;
-        const bool merged = long_runs && tpt == 1024 && dispatch_fits(rows_grid + nslots, 1024) &&
-                            ctx->tune.embed_bwd_merged != 0;
-        if (!dispatch_fits(rows_grid, tpt))
-            return fail(ctx, MIMIR_EINVAL, "Embedding backward: %lld rows of %d threads exceed the grid limit",
-                        (long long)rows_grid, tpt);
-        const unsigned rg = static_cast<unsigned>(rows_grid);
-        const bool by_run = runs.count != nullptr;
-        if (merged) {
-            const unsigned grid = static_cast<unsigned>(rows_grid + nslots);
-            if (by_run)
-                embed_bwd_rows_seg<true><<<grid, 1024, 0, ctx->stream>>>(skeys, stoks, n_ids, v, dy, grad, part, dim4,
-                                                                        list, runs);
+        const int64_t rows = runs.count && vocab < n_ids ? vocab : n_ids;  // at most this many runs
+        if (!dispatch_fits(rows, dim4 >= 1024 ? 1024 : dim4 >= 512 ? 512 : 256))
+            return fail(ctx, MIMIR_EINVAL, "Embedding backward: %lld rows of %lld floats exceed the grid limit",
+                        (long long)rows, (long long)dim);
+        // One 16-byte column per thread up to 1024 threads (MIMIR_TUNE
+        // gather=256/512/1024 picks a variant); more columns per thread were slower.
+        const int tpt = ctx->tune.gather_tpt ? ctx->tune.gather_tpt : (dim4 > 512 ? 1024 : dim4 > 256 ? 512 : 256);
+        const int64_t slots = long_runs ? nslots : 0;
+        const auto launch = [&](auto t) {
+            constexpr int T = decltype(t)::value;
+            const auto grid = static_cast<unsigned>(slots + std::min<int64_t>(rows, kRowsGrid * (1024 / T)));
+            if (runs.count)
+                embed_bwd_rows_seg<T, true><<<grid, T, 0, ctx->stream>>>(skeys, stoks, n_ids, v, dy, grad, part, dim4,
+                                                                         slots, list, runs);
             else
-                embed_bwd_rows_seg<false><<<grid, 1024, 0, ctx->stream>>>(skeys, stoks, n_ids, v, dy, grad, part,
-                                                                         dim4, list, runs);
-            if (int st = launched(ctx, "embed_bwd_rows_seg")) return st;
-        } else {
-            if (long_runs) {
-                const dim3 pgrid(static_cast<unsigned>(nslots),
-                                 static_cast<unsigned>((dim4 + kSegCols - 1) / kSegCols));
-                embed_bwd_seg_partial<<<pgrid, kSegCols, 0, ctx->stream>>>(skeys, stoks, n_ids, v, dy, part, dim4,
-                                                                           list);
-                if (int st = launched(ctx, "embed_bwd_seg_partial")) return st;
-            }
-#define MIMIR_EMB_ROWS(T, C)                                                                                  \
-    do {                                                                                                      \
-        if (by_run)                                                                                           \
-            embed_bwd_rows_vec<T, C, true><<<rg, T, 0, ctx->stream>>>(skeys, stoks, n_ids, v, dy, grad, dim4, lr, \
-                                                                      runs);                                  \
-        else                                                                                                  \
-            embed_bwd_rows_vec<T, C, false><<<rg, T, 0, ctx->stream>>>(skeys, stoks, n_ids, v, dy, grad, dim4,  \
-                                                                       lr, runs);                             \
-    } while (0)
-            if (tpt == 256)
-                MIMIR_EMB_ROWS(256, 4);
-            else if (tpt == 512)
-                MIMIR_EMB_ROWS(512, 2);
-            else
-                MIMIR_EMB_ROWS(1024, 1);
-#undef MIMIR_EMB_ROWS
-            if (int st = launched(ctx, "embed_bwd_rows_vec")) return st;
-        }
+                embed_bwd_rows_seg<T, false><<<grid, T, 0, ctx->stream>>>(skeys, stoks, n_ids, v, dy, grad, part, dim4,
+                                                                          slots, list, runs);
+        };
+        if (tpt == 256) launch(std::integral_constant<int, 256>{});
+        else if (tpt == 512) launch(std::integral_constant<int, 512>{});
+        else launch(std::integral_constant<int, 1024>{});
+        if (int st = launched(ctx, "embed_bwd_rows_seg")) return st;
         if (!long_runs) return MIMIR_OK;
         // The long runs' segment partials are complete and listed (stream
         // order): add them.  At most nslots runs of `blocks` items each.

@@ -49,7 +49,7 @@ struct RowShape {
 // Tuning override, read once per context from MIMIR_TUNE, e.g.
 //   MIMIR_TUNE="norm=1024x1x1024,layernorm=512x2x512,softmax=64x4x64,ew=1,gather=1024,rope=1,
 //               lnbwd=512x2x512,lnbwd_grid=512,chain=0,attnbwd_heads=4,attnbwd_blocks=2,
-//               embmerge=0,embsort=0,embruns=0,emb1pass=0,blas=0,lnbwd_narrow=0,lrcpw=2,ewbs=128,
+//               embsort=0,embruns=0,emb1pass=0,blas=0,lnbwd_narrow=0,lrcpw=2,ewbs=128,
 //               lrapply=256x4,lrpart=256"
 // Each entry selects among the compiled variants above; an entry that does
 // not fit a call (row too wide for it) is ignored for that call.  Unset, the
@@ -69,7 +69,6 @@ struct Tuning {
     int decode_splits = 0;    // attention_decode: workgroups per (sequence, head) (0: measured default)
     int attn_bwd_heads = 0;   // heads per group of the attention backward (0: what 1 GiB of P / dS holds)
     int attn_bwd_blocks = 0;  // causal attention backward: query / key blocks of the products (0: default)
-    int embed_bwd_merged = -1;  // embedding backward: rows + segment partials in one launch (1) or two (0)
     int embed_bwd_sort = -1;    // embedding backward: counting sort where it applies (-1, 1) or rocPRIM's (0)
     int embed_bwd_runs = -1;    // embedding backward: rows kernel over the counting sort's run list (-1, 1) or
                                 // over the sorted positions (0)
@@ -124,7 +123,6 @@ inline Tuning read_tuning() {
         else if (!std::strcmp(k, "decode")) t.decode_splits = std::atoi(v);
         else if (!std::strcmp(k, "attnbwd_heads")) t.attn_bwd_heads = std::atoi(v);
         else if (!std::strcmp(k, "attnbwd_blocks")) t.attn_bwd_blocks = std::atoi(v);
-        else if (!std::strcmp(k, "embmerge")) t.embed_bwd_merged = std::atoi(v);
         else if (!std::strcmp(k, "embsort")) t.embed_bwd_sort = std::atoi(v);
         else if (!std::strcmp(k, "embruns")) t.embed_bwd_runs = std::atoi(v);
         else if (!std::strcmp(k, "emb1pass")) t.embed_bwd_onepass = std::atoi(v);
