@@ -240,11 +240,11 @@ int mimir_rope_fwd(mimir_ctx* ctx, const float* q, float* q_out, int64_t q_heads
  * (ld = 3 * heads * head_dim).  Head h owns columns [h*head_dim,
  * (h+1)*head_dim).  The reference's scale is 1.0f / sqrtf(head_dim).
  * head_dim <= 2048 (above 128 a plain fp32 vector kernel runs instead of the
- * matrix-core one).  fp32 throughout (fp32 matrix-core products), no score
- * matrix in memory.  out must not overlap q, k or v.  kv_len == 0 gives zeros;
+ * matrix-core one).  fp32 precision (each fp32 operand three bf16 terms on the
+ * matrix cores, accumulated in fp32), no score matrix in memory.  out must not overlap q, k or v.  kv_len == 0 gives zeros;
  * batch == 0 or q_len == 0 is a no-op.  Device pointers, stream order.  Up to
- * 8 queries without a mask may use the context's fixed workspace (allocated
- * with the context). */
+ * 8 queries without a mask, and 737 keys or more where few workgroups have them,
+ * may use the context's fixed workspace (allocated with the context). */
 int mimir_attention_fwd(mimir_ctx* ctx, const float* q, int64_t ld_q, const float* k, const float* v,
                         int64_t ld_kv, float* out, int64_t ld_out, int64_t batch, int64_t q_len,
                         int64_t kv_len, int64_t heads, int64_t head_dim, float scale, int causal);
@@ -256,7 +256,7 @@ int mimir_attention_fwd(mimir_ctx* ctx, const float* q, int64_t ld_q, const floa
  * (embed_dim x embed_dim)], row-major as the reference's matmul reads them,
  * at least 4 embed_dim^2 floats (the reference reads past a shorter block; it
  * is refused here); out [seq_len x embed_dim].  The projections are fp32
- * library GEMMs, the core is mimir_attention_fwd with the reference's
+ * products (this library's own or library GEMMs), the core is mimir_attention_fwd with the reference's
  * scale 1/sqrtf(head_dim).  head_dim <= 2048.  Uses the context's scratch
  * (4 seq_len embed_dim floats).  out must not overlap input or weights. */
 int mimir_self_attention_fwd(mimir_ctx* ctx, const float* input, int64_t seq_len, int64_t embed_dim,

@@ -1,5 +1,5 @@
 // attention.hip -- the attention core softmax(Q K^T * scale) V with the
-// softmax fused between the two products, fp32 on the gfx950 matrix cores.
+// softmax fused between the two products, on the gfx950 matrix cores.
 //
 // Reference: the core of LayerOps::self_attention_forward (LayerOps.hpp:
 // 1045-1089) and cross_attention_forward (:1163-1209), which materialise one
@@ -516,6 +516,8 @@ int launch_mfma(mimir_ctx* ctx, const AttnArgs& a, int64_t bh, bool vec) {
     // tile's way in is the work, 142 / 122.
     const int64_t blocks4 = bh * ((a.q_len + 4 * kQPerWave - 1) / (4 * kQPerWave));
     int waves = a.splits == 1 && blocks4 <= 256 && a.q_len > 64 ? 4 : 8;
+    // A grid holds twice the workgroups of four waves.
+    if (!dispatch_fits(bh * ((a.q_len + 8 * kQPerWave - 1) / (8 * kQPerWave)) * a.splits, 8 * kWave)) waves = 4;
     if (ctx->tune.attn_waves == 4 || ctx->tune.attn_waves == 8) waves = ctx->tune.attn_waves;
     return waves == 4 ? launch<DP, 4>(ctx, a, bh, vec) : launch<DP, 8>(ctx, a, bh, vec);
 }
@@ -601,7 +603,7 @@ int mimir_attention_fwd(mimir_ctx* ctx, const float* q, int64_t ld_q, const floa
                      aligned16(a.k) && aligned16(a.v) && aligned16(out);
     // Few queries: each key row is read once by vector code, where the
     // matrix-core kernel would use one of its waves (attention_decode.hip).
-    if (attention_decode_applies(q_len, kv_len, head_dim, a.causal))
+    if (attention_decode_applies(batch * heads, q_len, kv_len, head_dim, a.causal))
         return attention_decode_launch(ctx, q, ld_q, a.k, a.v, ld_kv, out, ld_out, batch, q_len, kv_len, heads, head_dim,
                                        a.qscale, vec);
     if (mfma_takes(head_dim, ld_kv)) {
@@ -618,7 +620,7 @@ int mimir_attention_fwd(mimir_ctx* ctx, const float* q, int64_t ld_q, const floa
 }
 
 // The attention layers (Model.cpp:5904-5934, 5936-5990): the projections as
-// library GEMMs (gemm.hip), the fused core between them on the projection's
+// fp32 products (gemm.hip), the fused core between them on the projection's
 // output in place (no split copies).  Scratch: the projections' outputs and
 // the attended heads, reused in stream order.
 int mimir_self_attention_fwd(mimir_ctx* ctx, const float* input, int64_t seq_len, int64_t embed_dim,

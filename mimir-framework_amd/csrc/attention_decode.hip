@@ -253,8 +253,10 @@ void launch_nq(const DecodeArgs& a, unsigned grid, bool vec, hipStream_t s) {
 
 namespace mimir {
 
-bool attention_decode_applies(int64_t q_len, int64_t kv_len, int64_t head_dim, bool causal) {
-    return q_len <= kDecodeQueries && kv_len > 0 && head_dim <= kMaxDim && !causal;
+// More (sequence, head) pairs than the grid holds at a workgroup per query go to
+// the matrix-core kernel, which needs fewer workgroups.
+bool attention_decode_applies(int64_t bh, int64_t q_len, int64_t kv_len, int64_t head_dim, bool causal) {
+    return q_len <= kDecodeQueries && kv_len > 0 && head_dim <= kMaxDim && !causal && dispatch_fits(bh * q_len, kThreads);
 }
 
 int attention_decode_launch(mimir_ctx* ctx, const float* q, int64_t ld_q, const float* k, const float* v, int64_t ld_kv,

@@ -137,7 +137,7 @@ bool gemm_lt(mimir_ctx* ctx);
 // head_dim, the strides and the pointers are 16-byte multiples.
 constexpr int kDecodeQueries = 8;
 constexpr size_t kFixedWorkBytes = size_t(64) << 20;
-bool attention_decode_applies(int64_t q_len, int64_t kv_len, int64_t head_dim, bool causal);
+bool attention_decode_applies(int64_t bh, int64_t q_len, int64_t kv_len, int64_t head_dim, bool causal);
 int attention_decode_launch(mimir_ctx* ctx, const float* q, int64_t ld_q, const float* k, const float* v, int64_t ld_kv,
                             float* out, int64_t ld_out, int64_t batch, int64_t q_len, int64_t kv_len, int64_t heads,
                             int64_t head_dim, float qscale, bool vec);

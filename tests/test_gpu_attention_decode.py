@@ -44,3 +44,22 @@ def test_decode_special_values(ctx, lk):
     v64 = v[0].astype(np.float64)
     np.testing.assert_allclose(got[:, keep], p @ v64[:, keep], rtol=0, atol=1e-5)
     assert np.isposinf(got[:, 5]).all() and np.isnan(got[:, 9]).all()
+
+
+# 2^32 work-items bound a grid: 9 million sequences have fewer with four waves
+# per workgroup than with eight, or with a workgroup per few queries.  With one
+# key the output is its value, up to the 1e-9 beside the sum.
+@pytest.mark.parametrize("lq", [5, 9])
+def test_more_sequences_than_the_wider_grids_hold(ctx, lq):
+    n = 9_000_000
+    q = np.ones((n * lq, 1), np.float32)
+    kv = np.random.default_rng(3).standard_normal((n, 2)).astype(np.float32)
+    print(f"attention of {n} sequences, {lq} queries, one key", flush=True)
+    dq, dkv, out = ctx.to_device(q), ctx.to_device(kv), ctx.empty(q.shape)
+    try:
+        ctx.attention(dq, dkv, dkv.ptr + 4, out, n, lq, 1, 1, 1, ld_kv=2)
+        got = out.numpy()
+    finally:
+        for d in (dq, dkv, out):
+            d.free()
+    np.testing.assert_allclose(got.reshape(n, lq), np.repeat(kv[:, 1:], lq, 1), rtol=2e-7, atol=0)
