@@ -441,6 +441,19 @@ __global__ __launch_bounds__(1024) void sum_slots_tile(const float* part, int64_
     const int col = l & (kTileCols - 1);
     const int64_t q = (kWave / kTileCols) * w + (l / kTileCols);
     const int64_t c4 = static_cast<int64_t>(blockIdx.x) * kTileCols + col;
+    // The sums that the result is added to are on their way while the slots are:
+    // loaded at the end, one by one behind the width's checks, they made the backward
+    // of a residual block at 8192 x 4096 take 364.3 us instead of 362.5.
+    float* o[4];
+    f4 old = f4(0.0f);
+    if (threadIdx.x < kTileCols) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int64_t c = 4 * c4 + i;
+            o[i] = c < split ? out0 + c : out1 + (c - split);
+            if (acc && c < width) old[i] = *o[i];
+        }
+    }
     f4 s = f4(0.0f);
     if (4 * c4 < width) {
         const f4* p = reinterpret_cast<const f4*>(part) + c4;
@@ -464,12 +477,8 @@ __global__ __launch_bounds__(1024) void sum_slots_tile(const float* part, int64_
 #pragma unroll
         for (int i = 1; i < NW; ++i) t += lds[i][col];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int64_t c = 4 * c4 + i;
-            if (c >= width) break;
-            float* o = c < split ? out0 + c : out1 + (c - split);
-            *o = acc ? *o + t[i] : t[i];
-        }
+        for (int i = 0; i < 4; ++i)
+            if (4 * c4 + i < width) *o[i] = acc ? old[i] + t[i] : t[i];
     }
 }
 
