@@ -364,8 +364,8 @@ int launch_vec(mimir_ctx* ctx, const NormArgs& args) {
 
 // Rows the vector kernel cannot take (a width that is not a multiple of 4, or
 // unaligned pointers), up to 16384 floats: the row in registers as 16-byte
-// vectors at 4-byte addresses, TPR threads per row (a wave up to 2048 floats,
-// so its sums need no barrier; a workgroup above).  One read of the row (and of
+// vectors at 4-byte addresses, TPR threads per row (a wave up to 1536 floats,
+// so its sums need no barrier; a workgroup above, and where the rows are few).  One read of the row (and of
 // the residual for add + RMSNorm, whose sum is written once, after the
 // reduction's barrier: r_out may be r, and a row's last vector overlaps
 // nothing).  Bound by HBM like the vector kernel; measured at 8191 x 1001,
@@ -466,8 +466,10 @@ int dispatch(mimir_ctx* ctx, const NormArgs& a) {
     if (!vec) {
         if (a.cols <= 256) return launch_any<K, 64, 1>(ctx, a);
         if (a.cols <= 512) return launch_any<K, 64, 2>(ctx, a);
-        if (a.cols <= 1024) return launch_any<K, 64, 4>(ctx, a);
-        if (a.cols <= 2048) return launch_any<K, 64, 8>(ctx, a);
+        const bool wave = a.rows > kAnyWaveRows;
+        if (a.cols <= 1024) return wave ? launch_any<K, 64, 4>(ctx, a) : launch_any<K, 256, 1>(ctx, a);
+        if (a.cols <= 1536 && wave) return launch_any<K, 64, 6>(ctx, a);
+        if (a.cols <= 2048) return launch_any<K, 256, 2>(ctx, a);
         if (a.cols <= 4096) return launch_any<K, 256, 4>(ctx, a);
         if (a.cols <= 8192) return launch_any<K, 256, 8>(ctx, a);
         if (a.cols <= 16384) return launch_any<K, 256, 16>(ctx, a);

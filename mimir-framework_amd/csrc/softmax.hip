@@ -127,8 +127,8 @@ __global__ __launch_bounds__(kBlock) void softmax_rows_generic(SoftmaxArgs a) {
 
 // Rows the vector kernel cannot take (a width that is not a multiple of 4, or
 // unaligned pointers), up to 16384 floats: the row in registers as 16-byte
-// vectors at 4-byte addresses, TPR threads per row (a wave up to 2048 floats: no
-// barrier in its reductions; a workgroup above) -- one read of the row, and the
+// vectors at 4-byte addresses, TPR threads per row (a wave up to 1536 floats: no
+// barrier in its reductions; a workgroup above and where the rows are few) -- one read of the row, and the
 // same max / sum / finish as softmax_rows_generic.  Measured on
 // MI355X at 8191 x 1001: 11.4-12.7 us against 19.5 in 4-byte columns, one
 // workgroup per row; 40000 x 1001 57 / 81 us.
@@ -207,8 +207,10 @@ int dispatch(mimir_ctx* ctx, const SoftmaxArgs& a) {
     if (!vec) {
         if (a.cols <= 256) return launch_any<MODE, 64, 1>(ctx, a);
         if (a.cols <= 512) return launch_any<MODE, 64, 2>(ctx, a);
-        if (a.cols <= 1024) return launch_any<MODE, 64, 4>(ctx, a);
-        if (a.cols <= 2048) return launch_any<MODE, 64, 8>(ctx, a);
+        const bool wave = a.rows > kAnyWaveRows;
+        if (a.cols <= 1024) return wave ? launch_any<MODE, 64, 4>(ctx, a) : launch_any<MODE, 256, 1>(ctx, a);
+        if (a.cols <= 1536 && wave) return launch_any<MODE, 64, 6>(ctx, a);
+        if (a.cols <= 2048) return launch_any<MODE, 256, 2>(ctx, a);
         if (a.cols <= 4096) return launch_any<MODE, 256, 4>(ctx, a);
         if (a.cols <= 8192) return launch_any<MODE, 256, 8>(ctx, a);
         if (a.cols <= 16384) return launch_any<MODE, 256, 16>(ctx, a);

@@ -54,7 +54,8 @@ def ln64(x, eps):
 
 
 CASES = [(rows, cols, 0) for cols in WIDTHS for rows in (1, 5)] + [(131, 1001, 0), (2500, 67, 0), (7, 64, 1), (6, 1024, 3),
-                                                                  (3, 4096, 2), (600, 260, 1)]
+                                                                  (3, 4096, 2), (600, 260, 1), (2048, 515, 0), (2049, 515, 0),
+                                                                  (2048, 1535, 0), (2049, 1535, 0), (2049, 1537, 0)]
 
 
 @pytest.mark.parametrize("rows,cols,shift", CASES)
