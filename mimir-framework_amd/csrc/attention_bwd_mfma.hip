@@ -111,7 +111,8 @@ __device__ __forceinline__ void one_key(const BwdArgs& a, int role, int key, int
         float w = __builtin_amdgcn_exp2f(s - stats[i]) * stats[plane + i];
         if (role) {
             dp = wave_sum(dp);
-            w = (a.c.causal && i == 0) || a.kv_len == 1 ? 0.f : w * (dp - stats[2 * plane + i]);
+            // A query that sees one key: dS = p (dp - dp), 0 or NaN.
+            w *= (a.c.causal && i == 0) || a.kv_len == 1 ? dp - dp : dp - stats[2 * plane + i];
         }
         const float* row = role ? q + i * a.c.ld_q : dout + i * a.c.ld_dout;
 #pragma unroll
@@ -256,9 +257,10 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_kv(BwdArgs a) {
                     f4 ds;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        // A query that sees one key has p = 1 and no gradient.
+                        // A query that sees one key: its delta is that key's dP, so dS is 0, or
+                        // NaN where dP is not finite.
                         const bool one = a.kv_len == 1 || (a.c.causal && t == 0 && r + e == 0 && hf == 0);
-                        ds[e] = one ? 0.f : p[e] * (x[r + e] - delta[e]);
+                        ds[e] = p[e] * (x[r + e] - (one ? x[r + e] : delta[e]));
                         if (key >= a.kv_len) ds[e] = 0.f;
                         x[r + e] = ds[e];
                     }
@@ -418,7 +420,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_q(BwdArgs a) {
             s = wave_sum(s) * a.qscale;
             dp = wave_sum(dp);
             const float p = __builtin_amdgcn_exp2f(s - stats[0]) * stats[plane];
-            const float g = keys == 1 ? 0.f : p * (dp - stats[2 * plane]);
+            const float g = p * (keys == 1 ? dp - dp : dp - stats[2 * plane]);
 #pragma unroll
             for (int c = 0; c < kCh; ++c)
                 if (lane + c * kWave < a.head_dim) sum[c] += g * k[j * a.c.ld_kv + lane + c * kWave];

@@ -57,3 +57,33 @@ def test_split_backward_special_values(ctx):
     got = gpu_core_bwd(ctx, q, k, v, dout, 1, True)[0][0]
     assert np.isnan(got[n - 1]).all()
     assert_bwd_close(got[:n - 1], dq[:n - 1], tol[0][:n - 1], "queries that do not see the NaN key")
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf, -np.inf])
+@pytest.mark.parametrize("lk", [1, 40])
+def test_split_backward_one_visible_key(ctx, bad, lk):
+    """A query that sees a single key has dS = p (dP - dP): 0, but NaN where its
+    dP is not finite, as the formula has it.  lk == 1: every query; lk == 40,
+    causal: the first one."""
+    n, hd, at = 40, 32, 0
+    causal = lk > 1
+    q, k, v, dout = rand_core(11, 1, n, lk, hd)
+    if lk == 1:
+        at = 17
+    clean = dout.copy()
+    clean[0, at] = 0.0
+    (dq, dk, dv), tol = attention_bwd64(q[0], k[0], v[0], clean[0], 1, causal, O.attention_scale(hd))
+    dout[0, at, 3] = bad
+    got = [g[0] for g in gpu_core_bwd(ctx, q, k, v, dout, 1, causal)]
+    assert np.isnan(got[0][at]).all() and np.isnan(got[1][0]).all(), "dq of the query, dk of its key"
+    assert not np.isfinite(got[2][0, 3]), "dv of its key"
+    rest = np.arange(n) != at
+    if causal:  # no other gradient sees that query
+        assert_bwd_close(got[0][rest], dq[rest], tol[0][rest], "dq")
+        assert_bwd_close(got[1][1:], dk[1:], tol[1][1:], "dk")
+        assert_bwd_close(got[2][1:], dv[1:], tol[2][1:], "dv")
+    else:
+        assert (got[0][rest] == 0.0).all()
+    v[0, 0, 5] = bad  # the only visible value row of that query
+    got = gpu_core_bwd(ctx, q, k, v, clean if causal else dout, 1, causal)[0][0]
+    assert np.isnan(got[at]).all()
