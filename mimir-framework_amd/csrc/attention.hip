@@ -87,14 +87,6 @@ struct AttnArgs {
     uint32_t total_blocks;        // batch * heads * n_qblocks
     float qscale;                 // scale * log2(e), applied to Q
     int32_t causal;
-    // For the backward (STATS): the gradient of the output, and per query of
-    // each (sequence, head), in rows of stats_ld queries, the running max,
-    // 1 / (sum + 1e-9) and sum_d out_d dout_d.  out may be null then.
-    const float* dout;
-    int64_t ld_dout;
-    float* stats;
-    int64_t stats_ld;
-    uint32_t bh0;                 // first (sequence, head) of the launch
     // Keys dealt to several workgroups: partial results [split][n_bh][q_len]
     // [head_dim | max | sum], null: one workgroup per query block.
     int32_t splits;
@@ -170,19 +162,9 @@ struct OneQuery {
         for (int c = 0; c < CH; ++c)
             if (lane + c * kWave < head_dim) row[lane + c * kWave] = acc[c];
     }
-    __device__ __forceinline__ float dot(const float* row, int head_dim) const {
-        const int lane = threadIdx.x % kWave;
-        float part = 0.f;
-#pragma unroll
-        for (int c = 0; c < CH; ++c)
-            if (lane + c * kWave < head_dim) part += acc[c] * row[lane + c * kWave];
-        return wave_sum(part);
-    }
 };
 
-// STATS: for the backward, which needs every query's max, sum and
-// out . dout instead of (or beside) the output.
-template <int DP, int WAVES, bool VEC, bool STATS>
+template <int DP, int WAVES, bool VEC>
 __global__ __launch_bounds__(WAVES * kWave, WAVES > 4 ? 2 : 1) void attention_fwd_mfma(AttnArgs a) {
     using Keys = RowTile<DP, WAVES * kWave, VEC>;
     using Values = ColTile<DP, WAVES * kWave>;
@@ -195,9 +177,8 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES > 4 ? 2 : 1) void attention_fw
     int qb;
     const int split = static_cast<int>(blockIdx.x % static_cast<uint32_t>(a.splits));
     block_coords(a, blockIdx.x / static_cast<uint32_t>(a.splits), &bh, &qb);
-    const uint32_t head = a.bh0 + bh;
-    const int64_t b = head / static_cast<uint32_t>(a.heads);
-    const int64_t hd_off = static_cast<int64_t>(head % static_cast<uint32_t>(a.heads)) * a.head_dim;
+    const int64_t b = bh / static_cast<uint32_t>(a.heads);
+    const int64_t hd_off = static_cast<int64_t>(bh % static_cast<uint32_t>(a.heads)) * a.head_dim;
     const float* qbase = a.q + b * a.q_len * a.ld_q + hd_off;
     const float* kbase = a.k + b * a.kv_len * a.ld_kv + hd_off;
     const float* vbase = a.v + b * a.kv_len * a.ld_kv + hd_off;
@@ -314,8 +295,8 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES > 4 ? 2 : 1) void attention_fw
     const float inv = 1.0f / (l_tot + 1e-9f);
     const bool in = my_q < a.q_len;
     const int64_t row = min(my_q, a.q_len - 1);
-    const uint32_t n_bh = a.total_blocks / static_cast<uint32_t>(a.n_qblocks);
     if (a.part) {
+        const uint32_t n_bh = a.total_blocks / static_cast<uint32_t>(a.n_qblocks);
         float* p = a.part + ((split * static_cast<int64_t>(n_bh) + bh) * a.q_len + row) * (a.head_dim + 2);
         store_columns<DP, false>(o, 1.0f, p, in, hf, a.head_dim);
         if (in && hf == 0) {
@@ -324,28 +305,8 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES > 4 ? 2 : 1) void attention_fw
         }
         return;
     }
-    float check = store_columns<DP, VEC>(o, inv, a.out ? obase + row * a.ld_out : nullptr, in && a.out, hf, a.head_dim);
+    float check = store_columns<DP, VEC>(o, inv, obase + row * a.ld_out, in, hf, a.head_dim);
     check += l_tot - l_tot;
-    float* const stats = STATS ? a.stats + bh * a.stats_ld : nullptr;
-    const int64_t plane = n_bh * a.stats_ld;
-    const float* const dobase = STATS ? a.dout + b * a.q_len * a.ld_dout + hd_off : nullptr;
-    if constexpr (STATS) {
-        float dot = 0.f;
-#pragma unroll
-        for (int d = 0; d < kDb; ++d)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int dim = 32 * d + 8 * (r / 4) + 4 * hf + r % 4;
-                if (dim < a.head_dim) dot += o[d][r] * inv * dobase[row * a.ld_dout + dim];
-            }
-        dot += __shfl_xor(dot, 32);
-        // Rows past the sequence, up to the tile's end: no weight.
-        if (hf == 0 && my_q < a.stats_ld) {
-            stats[my_q] = in ? m_run : 0.f;
-            stats[plane + my_q] = in ? inv : 0.f;
-            stats[2 * plane + my_q] = in ? dot : 0.f;
-        }
-    }
     // Queries that came out NaN or infinite, again in fp32: their operands
     // may have had no bf16 split (split.hpp).
     for (uint32_t redo = bad_rows(check, in); redo; redo &= redo - 1) {
@@ -353,42 +314,24 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES > 4 ? 2 : 1) void attention_fw
         const OneQuery<(DP + kWave - 1) / kWave> one(qbase + i * a.ld_q, kbase, vbase, a.ld_kv,
                                                      a.causal ? min(static_cast<int64_t>(a.kv_len), i + 1) : a.kv_len,
                                                      a.head_dim, a.qscale);
-        if (a.out) one.store(obase + i * a.ld_out, a.head_dim);
-        if constexpr (STATS) {
-            const float dot = one.dot(dobase + i * a.ld_dout, a.head_dim);
-            if (lane == 0) {
-                stats[i] = one.m;
-                stats[plane + i] = one.inv;
-                stats[2 * plane + i] = dot;
-            }
-        }
+        one.store(obase + i * a.ld_out, a.head_dim);
     }
 }
 
 // The splits of one query, one wave per query: their sums brought to one max,
 // then what attention_fwd_mfma does with the whole.
-template <bool STATS>
 __global__ __launch_bounds__(4 * kWave) void attention_fwd_combine(AttnArgs a, int queries_per_block) {
     constexpr int kCh = 2;  // heads up to 128
     const uint32_t n_bh = a.total_blocks / static_cast<uint32_t>(a.n_qblocks);
-    const int64_t rows = STATS ? a.stats_ld : a.q_len;
     const int64_t at = static_cast<int64_t>(blockIdx.x) * 4 + threadIdx.x / kWave;
-    if (at >= n_bh * rows) return;  // whole waves
-    const int lane = threadIdx.x % kWave;
-    const uint32_t bh = static_cast<uint32_t>(at / rows);
-    const int64_t i = at % rows;
-    float* const stats = STATS ? a.stats + bh * a.stats_ld + i : nullptr;
-    const int64_t plane = n_bh * a.stats_ld;
-    if (i >= a.q_len) {  // up to the tile's end: no weight
-        if constexpr (STATS)
-            if (lane < 3) stats[lane * plane] = 0.f;
-        return;
-    }
-    const uint32_t head = a.bh0 + bh;
-    const int64_t b = head / static_cast<uint32_t>(a.heads);
-    const int64_t hd_off = static_cast<int64_t>(head % static_cast<uint32_t>(a.heads)) * a.head_dim;
+    if (at >= static_cast<int64_t>(n_bh) * a.q_len) return;  // whole waves
+    const int lane = threadIdx.x & (kWave - 1);
+    const uint32_t bh = static_cast<uint32_t>(at / a.q_len);
+    const int64_t i = at % a.q_len;
+    const int64_t b = bh / static_cast<uint32_t>(a.heads);
+    const int64_t hd_off = static_cast<int64_t>(bh % static_cast<uint32_t>(a.heads)) * a.head_dim;
     const int w = a.head_dim + 2;
-    const float* p = a.part + (static_cast<int64_t>(bh) * a.q_len + i) * w;
+    const float* p = a.part + at * w;
     const int64_t next = static_cast<int64_t>(n_bh) * a.q_len * w;
     const int all = tiles_of(a, static_cast<int>(i / queries_per_block) * queries_per_block, queries_per_block);
     const int per = (all + a.splits - 1) / a.splits, n = max(1, (all + per - 1) / max(per, 1));
@@ -402,38 +345,24 @@ __global__ __launch_bounds__(4 * kWave) void attention_fwd_combine(AttnArgs a, i
         for (int c = 0; c < kCh; ++c)
             if (lane + c * kWave < a.head_dim) acc[c] += x[lane + c * kWave] * f;
     }
-    float inv = 1.0f / (l + 1e-9f), check = l - l;
+    const float inv = 1.0f / (l + 1e-9f);
+    float check = l - l;
 #pragma unroll
     for (int c = 0; c < kCh; ++c) {
         acc[c] *= inv;
         check += acc[c] - acc[c];
     }
-    const float* dout = STATS ? a.dout + (b * a.q_len + i) * a.ld_dout + hd_off : nullptr;
+    float* const out = a.out + (b * a.q_len + i) * a.ld_out + hd_off;
     if (__any(check != check)) {
         const OneQuery<kCh> one(a.q + (b * a.q_len + i) * a.ld_q + hd_off, a.k + b * a.kv_len * a.ld_kv + hd_off,
                                 a.v + b * a.kv_len * a.ld_kv + hd_off, a.ld_kv,
                                 a.causal ? min(static_cast<int64_t>(a.kv_len), i + 1) : a.kv_len, a.head_dim, a.qscale);
-        m = one.m;
-        inv = one.inv;
+        one.store(out, a.head_dim);
+        return;
+    }
 #pragma unroll
-        for (int c = 0; c < kCh; ++c) acc[c] = one.acc[c];
-    }
-    float dot = 0.f;
-#pragma unroll
-    for (int c = 0; c < kCh; ++c) {
-        const int d = lane + c * kWave;
-        if (d >= a.head_dim) continue;
-        if (a.out) a.out[(b * a.q_len + i) * a.ld_out + hd_off + d] = acc[c];
-        if constexpr (STATS) dot += acc[c] * dout[d];
-    }
-    if constexpr (STATS) {
-        dot = wave_sum(dot);
-        if (lane == 0) {
-            stats[0] = m;
-            stats[plane] = inv;
-            stats[2 * plane] = dot;
-        }
-    }
+    for (int c = 0; c < kCh; ++c)
+        if (lane + c * kWave < a.head_dim) out[lane + c * kWave] = acc[c];
 }
 
 // Heads wider than 128 (up to 2048): one wave per query, the head's
@@ -474,20 +403,13 @@ int launch(mimir_ctx* ctx, AttnArgs a, int64_t bh, bool vec) {
                   (long long)blocks);
     a.total_blocks = static_cast<uint32_t>(blocks);
     const auto n = static_cast<unsigned>(blocks * a.splits);
-    if (a.stats) {
-        if (vec) attention_fwd_mfma<DP, WAVES, true, true><<<n, kThreads, 0, ctx->stream>>>(a);
-        else attention_fwd_mfma<DP, WAVES, false, true><<<n, kThreads, 0, ctx->stream>>>(a);
-    } else {
-        if (vec) attention_fwd_mfma<DP, WAVES, true, false><<<n, kThreads, 0, ctx->stream>>>(a);
-        else attention_fwd_mfma<DP, WAVES, false, false><<<n, kThreads, 0, ctx->stream>>>(a);
-    }
+    if (vec) attention_fwd_mfma<DP, WAVES, true><<<n, kThreads, 0, ctx->stream>>>(a);
+    else attention_fwd_mfma<DP, WAVES, false><<<n, kThreads, 0, ctx->stream>>>(a);
     if (int st = launched(ctx, "attention_fwd_mfma")) return st;
     if (!a.part) return MIMIR_OK;
-    const int64_t rows = bh * (a.stats ? a.stats_ld : a.q_len);
+    const int64_t rows = bh * a.q_len;
     MIMIR_REQUIRE(ctx, dispatch_fits((rows + 3) / 4, 4 * kWave), "attention: grid exceeds the limit");
-    const auto m = static_cast<unsigned>((rows + 3) / 4);
-    if (a.stats) attention_fwd_combine<true><<<m, 4 * kWave, 0, ctx->stream>>>(a, kQPerWave * WAVES);
-    else attention_fwd_combine<false><<<m, 4 * kWave, 0, ctx->stream>>>(a, kQPerWave * WAVES);
+    attention_fwd_combine<<<static_cast<unsigned>((rows + 3) / 4), 4 * kWave, 0, ctx->stream>>>(a, kQPerWave * WAVES);
     return launched(ctx, "attention_fwd_combine");
 }
 
@@ -534,36 +456,6 @@ int launch_any(mimir_ctx* ctx, const AttnArgs& a, int64_t bh, bool vec) {
 }
 
 }  // namespace
-
-int64_t mimir::attention_stats_floats(const mimir_ctx* ctx, int64_t n_bh, int64_t q_len, int64_t kv_len, int64_t head_dim) {
-    const int64_t s = splits_for(ctx, n_bh, q_len, kv_len, head_dim, INT64_MAX);
-    return s > 1 ? s * n_bh * q_len * (head_dim + 2) : 0;
-}
-
-int mimir::attention_stats(mimir_ctx* ctx, const AttnStats& x, bool vec) {
-    AttnArgs a{};
-    a.q = x.q;
-    a.k = x.k;
-    a.v = x.v;
-    a.out = x.out;
-    a.ld_q = x.ld_q;
-    a.ld_kv = x.ld_kv;
-    a.ld_out = x.ld_out;
-    a.q_len = x.q_len;
-    a.kv_len = x.kv_len;
-    a.heads = x.heads;
-    a.head_dim = x.head_dim;
-    a.qscale = x.scale * kLog2e;
-    a.causal = x.causal;
-    a.dout = x.dout;
-    a.ld_dout = x.ld_dout;
-    a.stats = x.stats;
-    a.stats_ld = x.stats_ld;
-    a.bh0 = x.bh0;
-    a.splits = static_cast<int32_t>(splits_for(ctx, x.n_bh, x.q_len, x.kv_len, x.head_dim, INT64_MAX));
-    a.part = a.splits > 1 ? x.work : nullptr;
-    return launch_any(ctx, a, x.n_bh, vec);
-}
 
 extern "C" {
 

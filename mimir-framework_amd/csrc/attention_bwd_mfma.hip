@@ -6,10 +6,14 @@
 // 6892-7028) and backward_cross_attention (:7122-7246).  With s = scale q . k
 // (causal j > i masked), p = exp(s - max) / (sum + 1e-9), dp = dout . v:
 //   dV = P^T dO,  dS = P (dP - delta),  dQ = scale dS K,  dK = scale dS^T Q,
-// delta_i = sum_j p_ij dp_ij = out_i . dout_i.  Only visible 32 x 32 tiles are
-// computed, and P is never stored:
-// 1. attention_stats (attention.hip): the forward, leaving each query's max,
-//    1 / (sum + 1e-9) and delta (and the output, where the layer wants it).
+// delta_i = sum_j p_ij dp_ij.  Only visible 32 x 32 tiles are computed, and P is
+// never stored:
+// 1. attention_bwd_stats: each query's max, 1 / (sum + 1e-9) and delta, from the
+//    scores and dP, both with the bits that step 2 computes again: where one key
+//    has all the weight, dP - delta cancels to what the other keys leave, and to 0
+//    where there is no other.  (out . dout, from the forward's output, is the
+//    same number with another rounding: it left 1e-7 of dP there, up to a
+//    hundred times dQ itself.)
 // 2. attention_bwd_kv: a workgroup owns 128 keys and streams tiles of 32
 //    queries.  Its eight waves are four pairs, a pair for 32 keys: one wave
 //    holds the K rows and computes S, then P, then dV += dO P; the other holds
@@ -58,12 +62,19 @@ struct BwdArgs {
     CoreBwd c;
     int32_t q_len, kv_len, heads, head_dim;
     float qscale;              // scale * log2(e)
-    float* stats;              // attention_stats' planes
+    // Per query of each (sequence, head), in rows of stats_ld queries: the max of
+    // its scores (base-2 units), 1 / (sum + 1e-9) and delta, three planes
+    // [n_bh][stats_ld] (rows past q_len zero).
+    float* stats;
     int64_t stats_ld;
+    // The keys of attention_bwd_stats dealt to several workgroups: max, sum and
+    // sum_j e_j dp_j of each, [split][3][n_bh][stats_ld]; null: one workgroup.
+    float* stats_part;
+    int32_t stats_splits;
     float* ds;                 // [n_bh][key tile][query tile][32 keys][32 queries]
     int32_t q_tiles, k_tiles;
     uint32_t bh0, n_bh;
-    uint32_t blocks;           // blocks of keys (queries) per (sequence, head)
+    uint32_t blocks;           // blocks of queries (keys) per (sequence, head)
     // The queries (attention_bwd_kv) or keys (attention_bwd_q) dealt to
     // several workgroups: partial dV and dK, or dQ, [split][n_bh][rows]
     // [head_dim] each; null: one workgroup.
@@ -82,6 +93,169 @@ __device__ __forceinline__ void coords(const BwdArgs& a, uint32_t bid, uint32_t*
     }
     *block = idx / owned;
     *bh = first + idx % owned;
+}
+
+// A score in base-2 units, rounded before a max is taken off it: the largest of a
+// row then gives exactly 1 wherever it is computed.
+__device__ __forceinline__ float base2(float s, float qscale) {
+#pragma clang fp contract(off)
+    return s * qscale;
+}
+
+// Running max, sum and sum of e dP of a query; a lane half holds its own share of
+// the sums.
+struct RowStats {
+    float m, l, d;
+    // One tile: scores s (base-2 units) and dP; -inf and 0 where the query does not
+    // see the key.
+    __device__ __forceinline__ void add(const f16v& s, const f16v& dp) {
+        float top = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
+        top = fmaxf(top, fmaxf(fmaxf(fmaxf(s[8], s[9]), fmaxf(s[10], s[11])),
+                               fmaxf(fmaxf(s[12], s[13]), fmaxf(s[14], s[15]))));
+        top = fmaxf(m, fmaxf(top, __shfl_xor(top, 32)));
+        const float alpha = __builtin_amdgcn_exp2f(m - top);
+        m = top;
+        float sum = 0.f, dot = 0.f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const float e = __builtin_amdgcn_exp2f(s[r] - top);
+            sum += e;
+            dot += e * dp[r];
+        }
+        l = l * alpha + sum;
+        d = d * alpha + dot;
+    }
+};
+
+// Step 1: a wave for 32 queries (their rows of Q and dO in registers), streaming 32
+// keys and values.  The scores come out as S^T = K Q^T, dP as V dO^T, the products
+// of step 2 transposed.
+template <int DP, bool VEC>
+__global__ __launch_bounds__(kThreads, 2) void attention_bwd_stats(BwdArgs a) {
+    using Rows = RowTile<DP, kThreads, VEC>;
+    constexpr int kC = DP / 16;
+    __shared__ __attribute__((aligned(16))) char lds[4 * Rows::kBytes];  // K and V rows of two tiles
+
+    uint32_t bh, qblock;
+    const int split = static_cast<int>(blockIdx.x % static_cast<uint32_t>(a.stats_splits));
+    coords(a, blockIdx.x / static_cast<uint32_t>(a.stats_splits), &bh, &qblock);
+    if (a.c.causal) qblock = a.blocks - 1 - qblock;  // the last queries see the most keys
+    const uint32_t head = a.bh0 + bh;
+    const int64_t b = head / static_cast<uint32_t>(a.heads);
+    const int64_t hd = static_cast<int64_t>(head % static_cast<uint32_t>(a.heads)) * a.head_dim;
+    const float* k = a.c.k + b * a.kv_len * a.c.ld_kv + hd;
+    const float* v = a.c.v + b * a.kv_len * a.c.ld_kv + hd;
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    const int li = lane % 32, hf = lane / 32;
+    const int qt = static_cast<int>(qblock) * kWaves + wave;  // this wave's query tile
+    const int my_q = qt * kTileRows + li;
+    const int last_qt = min(static_cast<int>(qblock) * kWaves + kWaves, a.q_tiles) - 1;
+    const int all_tiles = a.c.causal ? min(a.k_tiles, last_qt + 1) : a.k_tiles;
+    const int per = (all_tiles + a.stats_splits - 1) / a.stats_splits;
+    const int t0 = min(split * per, all_tiles), n_tiles = min(t0 + per, all_tiles);
+    const int wave_tiles = qt >= a.q_tiles ? 0 : min(n_tiles, a.c.causal ? qt + 1 : a.k_tiles);
+    const int end = a.c.causal ? min(a.kv_len, my_q + 1) : a.kv_len;  // this lane's keys
+    const int64_t row = min(my_q, a.q_len - 1);
+    const float* q = a.c.q + (b * a.q_len + row) * a.c.ld_q + hd;
+    const float* dout = a.c.dout + (b * a.q_len + row) * a.c.ld_dout + hd;
+
+    Rows keys, values;
+    keys.init(a.c.ld_kv, a.head_dim);
+    values.init(a.c.ld_kv, a.head_dim);
+    auto load = [&](int t) {
+        keys.load(k, t, a.c.ld_kv, a.kv_len, a.head_dim);
+        values.load(v, t, a.c.ld_kv, a.kv_len, a.head_dim);
+    };
+    if (t0 < n_tiles) load(t0);
+    Split8 qx[kC], ox[kC];
+    row_operand<DP, VEC>(q, hf, a.head_dim, 1.0f, qx);
+    row_operand<DP, VEC>(dout, hf, a.head_dim, 1.0f, ox);
+    // A masked key counts in the max with its score of -1e9 (Model.cpp:6906-6920).
+    const RowStats none{end < a.kv_len ? -1e9f * kLog2e : -1e30f, 0.f, 0.f};
+    RowStats st = none;
+    auto add = [&](RowStats& to, f16v& s, f16v& dp, int t) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = base2(s[r], a.qscale);
+        if ((t + 1) * kTileRows > a.kv_len || (a.c.causal && t == qt)) {
+            const int lim = end - t * kTileRows - 4 * hf;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const bool sees = 8 * (r / 4) + r % 4 < lim;
+                s[r] = sees ? s[r] : -INFINITY;
+                dp[r] = sees ? dp[r] : 0.f;
+            }
+        }
+        to.add(s, dp);
+    };
+    if (t0 < n_tiles) {
+        keys.stash(lds);
+        values.stash(lds + Rows::kBytes);
+        load(min(t0 + 1, n_tiles - 1));
+    }
+    __syncthreads();
+    for (int t = t0; t < n_tiles; ++t) {
+        const char* cur = lds + ((t - t0) & 1) * 2 * Rows::kBytes;
+        char* const next = lds + ((t - t0 + 1) & 1) * 2 * Rows::kBytes;
+        f16v s = f16v{}, dp = f16v{};
+        if (t < wave_tiles) {
+#pragma unroll
+            for (int c = 0; c < kC; ++c) s = mfma_split_mirror(Rows::at(cur, li, hf, c), qx[c], s);
+        }
+        // Past the last tile the stash rewrites a buffer that is not read again,
+        // and the load repeats the last tile.
+        keys.stash(next);
+        values.stash(next + Rows::kBytes);
+        load(min(t + 2, n_tiles - 1));
+        if (t < wave_tiles) {
+#pragma unroll
+            for (int c = 0; c < kC; ++c) dp = mfma_split_mirror(Rows::at(cur + Rows::kBytes, li, hf, c), ox[c], dp);
+            add(st, s, dp, t);
+        }
+        __syncthreads();
+    }
+    const bool in = my_q < a.q_len;
+    // Queries whose sums are not finite: again on the fp32 matrix cores (split.hpp).
+    // The others keep theirs, whose rounding is that of step 2.
+    if (const uint32_t bad = bad_rows((st.l - st.l) + (st.d - st.d), in)) {
+        RowStats redo = none;
+#pragma unroll 1
+        for (int t = t0; t < wave_tiles; ++t) {
+            f16v s = f32_scores(k, a.c.ld_kv, t * kTileRows, a.kv_len, a.head_dim, q, 1.0f);
+            f16v dp = f32_scores(v, a.c.ld_kv, t * kTileRows, a.kv_len, a.head_dim, dout, 1.0f);
+            add(redo, s, dp, t);
+        }
+        if (bad >> li & 1) st = redo;
+    }
+    st.l += __shfl_xor(st.l, 32);
+    st.d += __shfl_xor(st.d, 32);
+    if (hf || my_q >= a.stats_ld) return;
+    const int64_t plane = a.n_bh * a.stats_ld;
+    const float inv = 1.0f / (st.l + 1e-9f);
+    float* out = a.stats + bh * a.stats_ld + my_q;
+    if (a.stats_part) out = a.stats_part + (split * 3ll * a.n_bh + bh) * a.stats_ld + my_q;
+    // Rows past the sequence, up to the tile's end: no weight.
+    out[0] = in ? st.m : 0.f;
+    out[plane] = in ? (a.stats_part ? st.l : inv) : 0.f;
+    out[2 * plane] = in ? (a.stats_part ? st.d : st.d * inv) : 0.f;
+}
+
+// The splits' results of one query each, brought to one max.
+__global__ __launch_bounds__(256) void attention_bwd_stats_sum(BwdArgs a) {
+    const int64_t plane = a.n_bh * a.stats_ld, at = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    if (at >= plane) return;
+    const float* p = a.stats_part + at;
+    float m = p[0], l = 0.f, d = 0.f;
+    for (int s = 1; s < a.stats_splits; ++s) m = fmaxf(m, p[3 * s * plane]);
+    for (int s = 0; s < a.stats_splits; ++s, p += 3 * plane) {
+        const float f = __builtin_amdgcn_exp2f(p[0] - m);
+        l += p[plane] * f;
+        d += p[2 * plane] * f;
+    }
+    const bool in = at % a.stats_ld < a.q_len;
+    const float inv = 1.0f / (l + 1e-9f);
+    a.stats[at] = in ? m : 0.f;
+    a.stats[plane + at] = in ? inv : 0.f;
+    a.stats[2 * plane + at] = in ? d * inv : 0.f;
 }
 
 // The gradient of one key (row) in plain fp32 by a whole wave: dv (ROLE 0) or
@@ -107,12 +281,11 @@ __device__ __forceinline__ void one_key(const BwdArgs& a, int role, int key, int
             s += q[i * a.c.ld_q + d] * kr[c];
             dp += dout[i * a.c.ld_dout + d] * vr[c];
         }
-        s = wave_sum(s) * a.qscale;
+        s = base2(wave_sum(s), a.qscale);
         float w = __builtin_amdgcn_exp2f(s - stats[i]) * stats[plane + i];
         if (role) {
             dp = wave_sum(dp);
-            // A query that sees one key: dS = p (dp - dp), 0 or NaN.
-            w *= (a.c.causal && i == 0) || a.kv_len == 1 ? dp - dp : dp - stats[2 * plane + i];
+            w *= dp - stats[2 * plane + i];
         }
         const float* row = role ? q + i * a.c.ld_q : dout + i * a.c.ld_dout;
 #pragma unroll
@@ -229,7 +402,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_kv(BwdArgs a) {
                     f4 p;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        p[e] = __builtin_amdgcn_exp2f(x[r + e] * a.qscale - m[e]) * inv[e];
+                        p[e] = __builtin_amdgcn_exp2f(base2(x[r + e], a.qscale) - m[e]) * inv[e];
                         if (edge && (key >= a.kv_len || (a.c.causal && key > t * kTileRows + 8 * (r / 4) + 4 * hf + e)))
                             p[e] = 0.f;
                         x[r + e] = p[e];
@@ -257,10 +430,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_kv(BwdArgs a) {
                     f4 ds;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        // A query that sees one key: its delta is that key's dP, so dS is 0, or
-                        // NaN where dP is not finite.
-                        const bool one = a.kv_len == 1 || (a.c.causal && t == 0 && r + e == 0 && hf == 0);
-                        ds[e] = p[e] * (x[r + e] - (one ? x[r + e] : delta[e]));
+                        ds[e] = p[e] * (x[r + e] - delta[e]);
                         if (key >= a.kv_len) ds[e] = 0.f;
                         x[r + e] = ds[e];
                     }
@@ -417,10 +587,10 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_q(BwdArgs a) {
                 s += q[d] * k[j * a.c.ld_kv + d];
                 dp += dout[d] * v[j * a.c.ld_kv + d];
             }
-            s = wave_sum(s) * a.qscale;
+            s = base2(wave_sum(s), a.qscale);
             dp = wave_sum(dp);
             const float p = __builtin_amdgcn_exp2f(s - stats[0]) * stats[plane];
-            const float g = p * (keys == 1 ? dp - dp : dp - stats[2 * plane]);
+            const float g = p * (dp - stats[2 * plane]);
 #pragma unroll
             for (int c = 0; c < kCh; ++c)
                 if (lane + c * kWave < a.head_dim) sum[c] += g * k[j * a.c.ld_kv + lane + c * kWave];
@@ -437,6 +607,17 @@ int64_t query_blocks(const CoreBwd& c) { return (tiles(c.q_len) + kWaves - 1) / 
 
 template <int DP>
 int launch(mimir_ctx* ctx, BwdArgs a, bool vec) {
+    a.blocks = static_cast<uint32_t>(query_blocks(a.c));
+    const int64_t w = static_cast<int64_t>(a.n_bh) * a.blocks * a.stats_splits;
+    const int64_t rows_blocks = (a.n_bh * a.stats_ld + 255) / 256;
+    MIMIR_REQUIRE(ctx, dispatch_fits(w, kThreads) && dispatch_fits(rows_blocks, 256), "attention backward: grid too large");
+    if (vec) attention_bwd_stats<DP, true><<<static_cast<unsigned>(w), kThreads, 0, ctx->stream>>>(a);
+    else attention_bwd_stats<DP, false><<<static_cast<unsigned>(w), kThreads, 0, ctx->stream>>>(a);
+    if (int st = launched(ctx, "attention_bwd_stats")) return st;
+    if (a.stats_part) {
+        attention_bwd_stats_sum<<<static_cast<unsigned>(rows_blocks), 256, 0, ctx->stream>>>(a);
+        if (int st = launched(ctx, "attention_bwd_stats_sum")) return st;
+    }
     a.blocks = static_cast<uint32_t>(key_blocks(a.c));
     const int64_t n = static_cast<int64_t>(a.n_bh) * a.blocks * a.splits;
     const int64_t m = static_cast<int64_t>(a.n_bh) * query_blocks(a.c) * a.q_splits;
@@ -484,14 +665,14 @@ int64_t q_splits(const CoreBwd& c, int64_t n_bh) { return splits_of(n_bh * query
 int64_t part_floats(int64_t splits, int64_t n_bh, int64_t rows, int64_t head_dim) {
     return splits > 1 ? (splits * n_bh * rows * head_dim + 3) / 4 * 4 : 0;
 }
-int64_t parts_floats(const mimir_ctx* ctx, const CoreBwd& c, int64_t n_bh) {
-    // The forward's partial results are gone before the others are written.
-    return std::max(2 * part_floats(kv_splits(c, n_bh), n_bh, c.kv_len, c.head_dim) +
-                        part_floats(q_splits(c, n_bh), n_bh, c.q_len, c.head_dim),
-                    attention_stats_floats(ctx, n_bh, c.q_len, c.kv_len, c.head_dim));
-}
 int64_t ds_floats(const CoreBwd& c, int64_t n_bh) { return n_bh * tiles(c.q_len) * tiles(c.kv_len) * kBlockFloats; }
 int64_t stats_floats(const CoreBwd& c, int64_t n_bh) { return 3 * n_bh * tiles(c.q_len) * kTileRows; }
+int64_t parts_floats(const CoreBwd& c, int64_t n_bh) {
+    // The statistics' partial results are gone before the others are written.
+    const int64_t s = q_splits(c, n_bh);
+    return std::max(2 * part_floats(kv_splits(c, n_bh), n_bh, c.kv_len, c.head_dim) + part_floats(s, n_bh, c.q_len, c.head_dim),
+                    s > 1 ? s * stats_floats(c, n_bh) : 0);
+}
 
 }  // namespace
 
@@ -504,7 +685,7 @@ bool attention_bwd_mfma_takes(const CoreBwd& c) {
 
 int64_t attention_bwd_mfma_floats(const mimir_ctx* ctx, const CoreBwd& c) {
     const int64_t n = group_of(ctx, c), rest = c.batch * c.heads % n;  // the last group may be smaller and split more
-    return ds_floats(c, n) + stats_floats(c, n) + std::max(parts_floats(ctx, c, n), rest ? parts_floats(ctx, c, rest) : 0);
+    return ds_floats(c, n) + stats_floats(c, n) + std::max(parts_floats(c, n), rest ? parts_floats(c, rest) : 0);
 }
 
 int attention_bwd_mfma(mimir_ctx* ctx, const CoreBwd& c, float* work) {
@@ -512,8 +693,11 @@ int attention_bwd_mfma(mimir_ctx* ctx, const CoreBwd& c, float* work) {
     const int64_t stats_ld = tiles(c.q_len) * kTileRows;
     auto vec4 = [](const float* p, int64_t ld) { return ld % 4 == 0 && aligned16(p); };
     const bool vec = c.head_dim % 4 == 0 && vec4(c.q, c.ld_q) && vec4(c.k, c.ld_kv) && vec4(c.v, c.ld_kv) &&
-                     vec4(c.dout, c.ld_dout) && vec4(c.dq, c.ld_dq) && vec4(c.dk, c.ld_dkv) && vec4(c.dv, c.ld_dkv) &&
-                     (!c.att || vec4(c.att, c.ld_att));
+                     vec4(c.dout, c.ld_dout) && vec4(c.dq, c.ld_dq) && vec4(c.dk, c.ld_dkv) && vec4(c.dv, c.ld_dkv);
+    if (c.att)
+        if (int st = mimir_attention_fwd(ctx, c.q, c.ld_q, c.k, c.v, c.ld_kv, c.att, c.ld_att, c.batch, c.q_len, c.kv_len,
+                                         c.heads, c.head_dim, c.scale, c.causal))
+            return st;
     BwdArgs a{};
     a.c = c;
     a.q_len = static_cast<int32_t>(c.q_len);
@@ -530,11 +714,10 @@ int attention_bwd_mfma(mimir_ctx* ctx, const CoreBwd& c, float* work) {
         a.bh0 = static_cast<uint32_t>(h0);
         a.n_bh = static_cast<uint32_t>(std::min(group, total - h0));
         float* const parts = a.stats + stats_floats(c, group);
-        const AttnStats st{c.q, c.ld_q, c.k, c.v, c.ld_kv, c.dout, c.ld_dout, c.att, c.ld_att, a.stats, stats_ld,
-                           a.q_len, a.kv_len, a.heads, a.head_dim, a.bh0, a.n_bh, c.scale, c.causal, parts};
-        if (int e = attention_stats(ctx, st, vec)) return e;
         a.splits = static_cast<int32_t>(kv_splits(c, a.n_bh));
         a.q_splits = static_cast<int32_t>(q_splits(c, a.n_bh));
+        a.stats_splits = a.q_splits;
+        a.stats_part = a.stats_splits > 1 ? parts : nullptr;
         const int64_t one = part_floats(a.splits, a.n_bh, c.kv_len, c.head_dim);
         a.part[0] = a.splits > 1 ? parts : nullptr;
         a.part[1] = a.splits > 1 ? parts + one : nullptr;

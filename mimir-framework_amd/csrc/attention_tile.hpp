@@ -205,4 +205,32 @@ __device__ __forceinline__ uint32_t bad_rows(float check, bool in) {
     return static_cast<uint32_t>(b | b >> 32);
 }
 
+// For blocks whose split products are not finite (split.hpp), fp32 matrix cores:
+// D[row0 + 8 (r / 4) + 4 hf + r % 4][lane's row] in register r: the products of
+// 32 rows of a matrix with one row per lane (li; both halves the same), times
+// `scale`.  Rows at and past len: the last one's, for the caller to mask.  Few
+// registers, so that the kernels around it keep theirs.
+__device__ __forceinline__ f16v f32_scores(const float* base, int64_t ld, int row0, int len, int head_dim, const float* mine,
+                                           float scale) {
+    const int li = threadIdx.x % 32, hf = threadIdx.x % kWave / 32;
+    const float* row = base + min(row0 + li, len - 1) * ld;
+    f16v s = f16v{};
+#pragma unroll 1
+    for (int j = hf; j < head_dim + hf; j += 16) {  // the halves take turns: dimensions 2 i + hf
+        float x[8], y[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int d = min(j + 2 * i, head_dim - 1);
+            x[i] = row[d];
+            y[i] = mine[d];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const bool in = j + 2 * i < head_dim;
+            s = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? x[i] : 0.f, in ? y[i] * scale : 0.f, s, 0, 0, 0);
+        }
+    }
+    return s;
+}
+
 }  // namespace mimir

@@ -142,32 +142,6 @@ int attention_decode_launch(mimir_ctx* ctx, const float* q, int64_t ld_q, const 
                             float* out, int64_t ld_out, int64_t batch, int64_t q_len, int64_t kv_len, int64_t heads,
                             int64_t head_dim, float qscale, bool vec);
 
-// The forward core for the backward (attention.hip), heads up to 128: for the
-// (sequence, head) pairs bh0 .. bh0 + n_bh, per query the running max (base-2
-// units of the scaled scores), 1 / (sum + 1e-9) and out . dout, in three planes
-// [n_bh][stats_ld] of stats (stats_ld: q_len rounded up to 32; the rows past
-// q_len get zeros), and the output itself when out is set.
-struct AttnStats {
-    const float* q;
-    int64_t ld_q;
-    const float* k;
-    const float* v;
-    int64_t ld_kv;
-    const float* dout;
-    int64_t ld_dout;
-    float* out;
-    int64_t ld_out;
-    float* stats;
-    int64_t stats_ld;
-    int32_t q_len, kv_len, heads, head_dim;
-    uint32_t bh0, n_bh;
-    float scale;
-    int causal;
-    float* work;  // attention_stats_floats
-};
-int64_t attention_stats_floats(const mimir_ctx* ctx, int64_t n_bh, int64_t q_len, int64_t kv_len, int64_t head_dim);
-int attention_stats(mimir_ctx* ctx, const AttnStats& x, bool vec);
-
 // One backward of the core.  att (optional): also write the attended heads
 // P V, which the layers' output-projection gradient reads.
 struct CoreBwd {

@@ -86,6 +86,17 @@ __device__ __forceinline__ f16v mfma_split(const Split8& a, const Split8& b, f16
     return mfma_bf16(a.h, b.h, c);
 }
 
+// The same products in the order that mfma_split(b, a, c) takes them, so that the
+// transposed result has the same bits.
+__device__ __forceinline__ f16v mfma_split_mirror(const Split8& a, const Split8& b, f16v c) {
+    c = mfma_bf16(a.h, b.l, c);
+    c = mfma_bf16(a.l, b.h, c);
+    c = mfma_bf16(a.m, b.m, c);
+    c = mfma_bf16(a.h, b.m, c);
+    c = mfma_bf16(a.m, b.h, c);
+    return mfma_bf16(a.h, b.h, c);
+}
+
 // Word 3 of a raw (stride 0) buffer descriptor on gfx9-family GPUs: 32-bit
 // data format, no swizzle; out-of-range offsets return zeros.
 constexpr int kBufferWord3 = 0x00020000;

@@ -87,3 +87,31 @@ def test_split_backward_one_visible_key(ctx, bad, lk):
     v[0, 0, 5] = bad  # the only visible value row of that query
     got = gpu_core_bwd(ctx, q, k, v, clean if causal else dout, 1, causal)[0][0]
     assert np.isnan(got[at]).all()
+
+
+@pytest.mark.parametrize("n,hd,causal", [(200, 32, False), (512, 64, True), (333, 80, False), (1100, 128, True)])
+def test_split_backward_saturated_rows(ctx, n, hd, causal):
+    """Rows where one key has all but 1e-8 of the weight (scores of about +-40): dP
+    of that key and delta cancel, so both must have the same rounding.  There l
+    = 1 and delta = dP (1 + u) + at most 1e-8 of another dP, so dS, whose exact
+    value is below 2e-8 max |dP|, is within 2 u max |dP| of it, and dq within that
+    times scale max |k|."""
+    q, k, v, dout = rand_core(n + hd, 1, n, n, hd)
+    amp = np.float32(np.sqrt(40.0 / np.sqrt(hd)) * hd ** 0.25)
+    q *= amp
+    k *= amp
+    scale = float(np.float32(O.attention_scale(hd)))
+    q64, k64, v64, do64 = (a[0].astype(np.float64) for a in (q, k, v, dout))
+    (dq, _, dv), _ = attention_bwd64(q64, k64, v64, do64, 1, causal, scale)
+    s = scale * (q64 @ k64.T)
+    if causal:
+        s[np.triu(np.ones(s.shape, bool), 1)] = -np.inf
+    p = np.exp(s - s.max(1, keepdims=True))
+    rows = np.flatnonzero(p.sum(1) - 1 < 1e-8)
+    assert rows.size > n // 10
+    got = gpu_core_bwd(ctx, q, k, v, dout, 1, causal)
+    g = np.abs(do64 @ v64.T).max(1)
+    tol = 2 * O.U32 * scale * np.outer(g, np.abs(k64).max(0))
+    err = np.abs(got[0][0] - dq)
+    print(f"saturated n={n} hd={hd}: worst error {(err / tol)[rows].max():.3g} of the bound, {err[rows].max():.3g}", flush=True)
+    assert (err <= tol)[rows].all()
