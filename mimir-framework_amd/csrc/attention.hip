@@ -113,59 +113,44 @@ __device__ __forceinline__ void block_coords(const AttnArgs& a, uint32_t bid, ui
     *bh = first + idx % owned;
 }
 
-// One query by one wave in plain fp32, the head's dimensions spread over the
-// lanes (CH per lane, lane + 64 c): each score a DPP wave sum, the same online
-// softmax and the same division by (sum + 1e-9).
-template <int CH>
-struct OneQuery {
-    float acc[CH], m, inv;
-    __device__ __forceinline__ OneQuery(const float* qrow, const float* kb, const float* vb, int64_t ld_kv, int64_t keys,
-                                        int head_dim, float qscale) {
-        const int lane = threadIdx.x % kWave;
-        float q[CH];
+// A wave's 32 queries on the fp32 matrix cores (attention_tile.hpp), over key
+// tiles t0 .. t1 - 1, for 32 NB dimensions of the output (vbase and head_dim from
+// the first of them on): the same online softmax.  `end`: where the lane's keys end.
+template <int NB>
+__device__ __forceinline__ void queries_f32(const AttnArgs& a, const float* qrow, const float* kbase, const float* vbase,
+                                            int head_dim, int t0, int t1, int end, float* m, float* l, f16v* o) {
+    const int hf = threadIdx.x % kWave / 32;
 #pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            const int d = lane + c * kWave;
-            q[c] = d < head_dim ? qrow[d] * qscale : 0.f;
-            acc[c] = 0.f;
+    for (int d = 0; d < NB; ++d) o[d] = f16v{};
+    float m_run = -1e30f, l_run = 0.f;
+#pragma unroll 1
+    for (int t = t0; t < t1; ++t) {
+        f16v s = f32_scores(kbase, a.ld_kv, t * kKeyTile, a.kv_len, a.head_dim, qrow, a.qscale);
+        float m_new = m_run;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            s[r] = t * kKeyTile + 8 * (r / 4) + 4 * hf + r % 4 < end ? s[r] : -INFINITY;
+            m_new = fmaxf(m_new, s[r]);
         }
-        float l = 0.f;
-        m = -1e30f;
-        for (int64_t j = 0; j < keys; ++j) {
-            const float* krow = kb + j * ld_kv;
-            const float* vrow = vb + j * ld_kv;
-            float part = 0.f;
+        m_new = fmaxf(m_new, __shfl_xor(m_new, 32));
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        m_run = m_new;
+        l_run *= alpha;
 #pragma unroll
-            for (int c = 0; c < CH; ++c) {
-                const int d = lane + c * kWave;
-                if (d < head_dim) part += q[c] * krow[d];
-            }
-            const float s = wave_sum(part);  // wave-uniform
-            const float m_new = fmaxf(m, s);
-            const float alpha = __builtin_amdgcn_exp2f(m - m_new);
-            const float p = __builtin_amdgcn_exp2f(s - m_new);
-            m = m_new;
-            l = l * alpha + p;
+        for (int d = 0; d < NB; ++d) o[d] *= alpha;
 #pragma unroll
-            for (int c = 0; c < CH; ++c) {
-                const int d = lane + c * kWave;
-                acc[c] = acc[c] * alpha + (d < head_dim ? p * vrow[d] : 0.f);
-            }
+        for (int r = 0; r < 16; ++r) {
+            s[r] = __builtin_amdgcn_exp2f(s[r] - m_run);
+            l_run += s[r];
         }
-        inv = 1.0f / (l + 1e-9f);
-#pragma unroll
-        for (int c = 0; c < CH; ++c) acc[c] *= inv;
+        f32_accumulate<NB>(vbase, a.ld_kv, t * kKeyTile, a.kv_len, head_dim, s, 0, end, o);
     }
-    __device__ __forceinline__ void store(float* row, int head_dim) const {
-        const int lane = threadIdx.x % kWave;
-#pragma unroll
-        for (int c = 0; c < CH; ++c)
-            if (lane + c * kWave < head_dim) row[lane + c * kWave] = acc[c];
-    }
-};
+    *m = m_run;
+    *l = l_run + __shfl_xor(l_run, 32);
+}
 
 template <int DP, int WAVES, bool VEC>
-__global__ __launch_bounds__(WAVES * kWave, WAVES > 4 ? 2 : 1) void attention_fwd_mfma(AttnArgs a) {
+__global__ __launch_bounds__(WAVES * kWave, WAVES == 4 ? 1 : DP == 32 && VEC ? 4 : 2) void attention_fwd_mfma(AttnArgs a) {
     using Keys = RowTile<DP, WAVES * kWave, VEC>;
     using Values = ColTile<DP, WAVES * kWave>;
     constexpr int kBuf = Keys::kBytes + Values::kBytes;
@@ -225,6 +210,7 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES > 4 ? 2 : 1) void attention_fw
 #pragma unroll
     for (int d = 0; d < kDb; ++d) o[d] = f16v{};
     float m_run = -1e30f;  // running max (base-2 units); the reference starts at -1e30 (LayerOps.hpp:1052)
+    float m_top = -1e30f;  // the max itself: m_run lags behind it by up to kMaxSlack
     float l_run = 0.f;     // this half's share of the running sum
 
     if (n_tiles > t0) {
@@ -244,7 +230,6 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES > 4 ? 2 : 1) void attention_fw
             // Past the last tile the stash rewrites a buffer that is not read
             // again, and the load repeats the last tile.
             stash(next);
-            
             __builtin_amdgcn_s_setprio(0);
             load(min(t + 2, n_tiles - 1));
             if ((t + 1) * kKeyTile > a.kv_len || (a.causal && (t + 1) * kKeyTile - 1 > qw0)) {
@@ -256,6 +241,7 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES > 4 ? 2 : 1) void attention_fw
             tmax = fmaxf(tmax, fmaxf(fmaxf(fmaxf(s[8], s[9]), fmaxf(s[10], s[11])),
                                      fmaxf(fmaxf(s[12], s[13]), fmaxf(s[14], s[15]))));
             tmax = fmaxf(tmax, __shfl_xor(tmax, 32));
+            m_top = fmaxf(m_top, tmax);
             if (__any(tmax > m_run + kMaxSlack)) {
                 const float m_new = fmaxf(m_run, tmax);
                 const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
@@ -281,7 +267,6 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES > 4 ? 2 : 1) void attention_fw
 #pragma unroll
                 for (int d = 0; d < kDb; ++d) o[d] = mfma_split(Values::at(cur + Keys::kBytes, li, hf, d, c), p, o[d]);
             }
-            
             __builtin_amdgcn_s_setprio(0);
         } else {
             stash(next);
@@ -290,31 +275,47 @@ __global__ __launch_bounds__(WAVES * kWave, WAVES > 4 ? 2 : 1) void attention_fw
         __syncthreads();
     }
 
-    // out = O / (sum + 1e-9) (LayerOps.hpp:1076-1079).
+    // out = O / (sum + 1e-9) (LayerOps.hpp:1076-1079); a split's share in units of
+    // the true max, so that the shares' sum stays below what one workgroup without
+    // lag would hold.
+    const float lag = __builtin_amdgcn_exp2f(m_run - m_top);
     const float l_tot = l_run + __shfl_xor(l_run, 32);
     const float inv = 1.0f / (l_tot + 1e-9f);
     const bool in = my_q < a.q_len;
     const int64_t row = min(my_q, a.q_len - 1);
-    if (a.part) {
-        const uint32_t n_bh = a.total_blocks / static_cast<uint32_t>(a.n_qblocks);
-        float* p = a.part + ((split * static_cast<int64_t>(n_bh) + bh) * a.q_len + row) * (a.head_dim + 2);
-        store_columns<DP, false>(o, 1.0f, p, in, hf, a.head_dim);
+    const int64_t n_bh = a.total_blocks / static_cast<uint32_t>(a.n_qblocks);
+    float* const part = a.part ? a.part + ((split * n_bh + bh) * a.q_len + row) * (a.head_dim + 2) : nullptr;
+    float* const out = obase + row * a.ld_out;
+    float check;
+    if (part) {
+        check = store_columns<DP, false>(o, lag, part, in, hf, a.head_dim);
         if (in && hf == 0) {
-            p[a.head_dim] = m_run;
-            p[a.head_dim + 1] = l_tot;
+            part[a.head_dim] = m_top;
+            part[a.head_dim + 1] = l_tot * lag;
         }
-        return;
+    } else {
+        check = store_columns<DP, VEC>(o, inv, out, in, hf, a.head_dim);
     }
-    float check = store_columns<DP, VEC>(o, inv, obase + row * a.ld_out, in, hf, a.head_dim);
-    check += l_tot - l_tot;
-    // Queries that came out NaN or infinite, again in fp32: their operands
-    // may have had no bf16 split (split.hpp).
-    for (uint32_t redo = bad_rows(check, in); redo; redo &= redo - 1) {
-        const int64_t i = qw0 + __builtin_ctz(redo);
-        const OneQuery<(DP + kWave - 1) / kWave> one(qbase + i * a.ld_q, kbase, vbase, a.ld_kv,
-                                                     a.causal ? min(static_cast<int64_t>(a.kv_len), i + 1) : a.kv_len,
-                                                     a.head_dim, a.qscale);
-        one.store(obase + i * a.ld_out, a.head_dim);
+    // Queries that came out NaN or infinite, again in fp32: their operands may have
+    // had no bf16 split (split.hpp), or the lag of the max an overflow.
+    if (const uint32_t bad = bad_rows(check + (l_tot - l_tot), in)) {
+        constexpr int kNb = kRedoBlocks<DP>;
+        const bool mine = in && (bad >> li & 1);
+#pragma unroll 1
+        for (int d0 = 0; d0 < a.head_dim; d0 += 32 * kNb) {
+            f16v x[kNb];
+            float m, l;
+            queries_f32<kNb>(a, qbase + row * a.ld_q, kbase, vbase + d0, a.head_dim - d0, t0, wave_tiles, lane_key_end, &m, &l, x);
+            if (part) {
+                store_columns<32 * kNb, false>(x, 1.0f, part + d0, mine, hf, a.head_dim - d0);
+                if (mine && hf == 0) {
+                    part[a.head_dim] = m;
+                    part[a.head_dim + 1] = l;
+                }
+            } else {
+                store_columns<32 * kNb, VEC>(x, 1.0f / (l + 1e-9f), out + d0, mine, hf, a.head_dim - d0);
+            }
+        }
     }
 }
 
@@ -346,23 +347,10 @@ __global__ __launch_bounds__(4 * kWave) void attention_fwd_combine(AttnArgs a, i
             if (lane + c * kWave < a.head_dim) acc[c] += x[lane + c * kWave] * f;
     }
     const float inv = 1.0f / (l + 1e-9f);
-    float check = l - l;
-#pragma unroll
-    for (int c = 0; c < kCh; ++c) {
-        acc[c] *= inv;
-        check += acc[c] - acc[c];
-    }
     float* const out = a.out + (b * a.q_len + i) * a.ld_out + hd_off;
-    if (__any(check != check)) {
-        const OneQuery<kCh> one(a.q + (b * a.q_len + i) * a.ld_q + hd_off, a.k + b * a.kv_len * a.ld_kv + hd_off,
-                                a.v + b * a.kv_len * a.ld_kv + hd_off, a.ld_kv,
-                                a.causal ? min(static_cast<int64_t>(a.kv_len), i + 1) : a.kv_len, a.head_dim, a.qscale);
-        one.store(out, a.head_dim);
-        return;
-    }
 #pragma unroll
     for (int c = 0; c < kCh; ++c)
-        if (lane + c * kWave < a.head_dim) out[lane + c * kWave] = acc[c];
+        if (lane + c * kWave < a.head_dim) out[lane + c * kWave] = acc[c] * inv;
 }
 
 // Heads wider than 128 (up to 2048): one wave per query, the head's
@@ -375,15 +363,52 @@ __global__ __launch_bounds__(4 * kWave) void attention_fwd_combine(AttnArgs a, i
 constexpr int kGenericWaves = 4;
 template <int CH>
 __global__ __launch_bounds__(kGenericWaves * kWave) void attention_fwd_generic(AttnArgs a) {
+    const int lane = threadIdx.x % kWave;
     const int64_t qi = static_cast<int64_t>(blockIdx.y) * kGenericWaves + threadIdx.x / kWave;
     if (qi >= a.q_len) return;  // whole waves leave: no barrier below
     const uint32_t bh = blockIdx.x;
     const int64_t b = bh / static_cast<uint32_t>(a.heads);
     const int64_t hd_off = static_cast<int64_t>(bh % static_cast<uint32_t>(a.heads)) * a.head_dim;
-    const OneQuery<CH> one(a.q + (b * a.q_len + qi) * a.ld_q + hd_off, a.k + b * a.kv_len * a.ld_kv + hd_off,
-                           a.v + b * a.kv_len * a.ld_kv + hd_off, a.ld_kv,
-                           a.causal ? (qi + 1 < a.kv_len ? qi + 1 : a.kv_len) : a.kv_len, a.head_dim, a.qscale);
-    one.store(a.out + (b * a.q_len + qi) * a.ld_out + hd_off, a.head_dim);
+    const float* qrow = a.q + (b * a.q_len + qi) * a.ld_q + hd_off;
+    const float* kb = a.k + b * a.kv_len * a.ld_kv + hd_off;
+    const float* vb = a.v + b * a.kv_len * a.ld_kv + hd_off;
+    float q[CH], acc[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const int d = lane + c * kWave;
+        q[c] = d < a.head_dim ? qrow[d] * a.qscale : 0.f;
+        acc[c] = 0.f;
+    }
+    const int64_t key_end = a.causal ? (qi + 1 < a.kv_len ? qi + 1 : a.kv_len) : a.kv_len;
+    float m_run = -1e30f, l_run = 0.f;
+    for (int64_t j = 0; j < key_end; ++j) {
+        const float* krow = kb + j * a.ld_kv;
+        const float* vrow = vb + j * a.ld_kv;
+        float part = 0.f;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            const int d = lane + c * kWave;
+            if (d < a.head_dim) part += q[c] * krow[d];
+        }
+        const float s = wave_sum(part);  // wave-uniform
+        const float m_new = fmaxf(m_run, s);
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+        const float p = __builtin_amdgcn_exp2f(s - m_new);
+        m_run = m_new;
+        l_run = l_run * alpha + p;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+            const int d = lane + c * kWave;
+            acc[c] = acc[c] * alpha + (d < a.head_dim ? p * vrow[d] : 0.f);
+        }
+    }
+    const float inv = 1.0f / (l_run + 1e-9f);
+    float* orow = a.out + (b * a.q_len + qi) * a.ld_out + hd_off;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const int d = lane + c * kWave;
+        if (d < a.head_dim) orow[d] = acc[c] * inv;
+    }
 }
 
 template <int CH>

@@ -258,43 +258,54 @@ __global__ __launch_bounds__(256) void attention_bwd_stats_sum(BwdArgs a) {
     a.stats[2 * plane + at] = in ? d * inv : 0.f;
 }
 
-// The gradient of one key (row) in plain fp32 by a whole wave: dv (ROLE 0) or
-// dk (ROLE 1), for keys whose split result was not finite.
-template <int CH>
-__device__ __forceinline__ void one_key(const BwdArgs& a, int role, int key, int q0, int q1, const float* q, const float* k,
-                                        const float* v, const float* dout, const float* stats, int64_t plane, float* out) {
-    const int lane = threadIdx.x % kWave;
-    float kr[CH], vr[CH], acc[CH];
+// The gradient of a wave's 32 keys on the fp32 matrix cores (attention_tile.hpp),
+// over query tiles t0 .. t1 - 1, for 32 NB dimensions from d0 on: dV (role 0) or dK /
+// scale (role 1).
+template <int NB>
+__device__ __forceinline__ void keys_f32(const BwdArgs& a, int role, int key, int t0, int t1, int d0, const float* q,
+                                         const float* k, const float* v, const float* dout, const float* stats, int64_t plane,
+                                         f16v* acc) {
+    const int hf = threadIdx.x % kWave / 32;
+    const int lo = a.c.causal ? key : 0;
+    const float* const rows = role ? q : dout;
+    const int64_t ld = role ? a.c.ld_q : a.c.ld_dout;
 #pragma unroll
-    for (int c = 0; c < CH; ++c) {
-        const int d = lane + c * kWave;
-        kr[c] = d < a.head_dim ? k[key * a.c.ld_kv + d] : 0.f;
-        vr[c] = d < a.head_dim ? v[key * a.c.ld_kv + d] : 0.f;
-        acc[c] = 0.f;
-    }
-    for (int i = a.c.causal ? max(key, q0) : q0; i < min(q1, a.q_len); ++i) {
-        float s = 0.f, dp = 0.f;
+    for (int d = 0; d < NB; ++d) acc[d] = f16v{};
+#pragma unroll 1
+    for (int t = t0; t < t1; ++t) {
+        const int row0 = t * kTileRows;
+        f16v w = f32_scores(q, a.c.ld_q, row0, a.q_len, a.head_dim, k + key * a.c.ld_kv, 1.0f), dp = f16v{};
+        if (role) dp = f32_scores(dout, a.c.ld_dout, row0, a.q_len, a.head_dim, v + key * a.c.ld_kv, 1.0f);
 #pragma unroll
-        for (int c = 0; c < CH; ++c) {
-            const int d = lane + c * kWave;
-            if (d >= a.head_dim) continue;
-            s += q[i * a.c.ld_q + d] * kr[c];
-            dp += dout[i * a.c.ld_dout + d] * vr[c];
+        for (int r = 0; r < 16; ++r) {
+            const int i = row0 + 8 * (r / 4) + 4 * hf + r % 4;  // below stats_ld
+            float p = __builtin_amdgcn_exp2f(base2(w[r], a.qscale) - stats[i]) * stats[plane + i];
+            if (role) p *= dp[r] - stats[2 * plane + i];
+            w[r] = i >= lo && i < a.q_len ? p : 0.f;
         }
-        s = base2(wave_sum(s), a.qscale);
-        float w = __builtin_amdgcn_exp2f(s - stats[i]) * stats[plane + i];
-        if (role) {
-            dp = wave_sum(dp);
-            w *= dp - stats[2 * plane + i];
-        }
-        const float* row = role ? q + i * a.c.ld_q : dout + i * a.c.ld_dout;
-#pragma unroll
-        for (int c = 0; c < CH; ++c)
-            if (lane + c * kWave < a.head_dim) acc[c] += w * row[lane + c * kWave];
+        f32_accumulate<NB>(rows + d0, ld, row0, a.q_len, a.head_dim - d0, w, lo, a.q_len, acc);
     }
+}
+
+// The same for a wave's 32 queries, over key tiles t0 .. t1 - 1, for 32
+// dimensions: dQ / scale.  stats: the lane's query's.
+__device__ __forceinline__ void queries_f32(const BwdArgs& a, int end, int t0, int t1, int d0, const float* q, const float* k,
+                                            const float* v, const float* dout, const float* stats, int64_t plane, f16v& acc) {
+    const int hf = threadIdx.x % kWave / 32;
+    const float m = stats[0], inv = stats[plane], delta = stats[2 * plane];
+    acc = f16v{};
+#pragma unroll 1
+    for (int t = t0; t < t1; ++t) {
+        const int row0 = t * kTileRows;
+        f16v w = f32_scores(k, a.c.ld_kv, row0, a.kv_len, a.head_dim, q, 1.0f);
+        const f16v dp = f32_scores(v, a.c.ld_kv, row0, a.kv_len, a.head_dim, dout, 1.0f);
 #pragma unroll
-    for (int c = 0; c < CH; ++c)
-        if (lane + c * kWave < a.head_dim) out[lane + c * kWave] = acc[c] * (role ? a.c.scale : 1.f);
+        for (int r = 0; r < 16; ++r) {
+            const float ds = __builtin_amdgcn_exp2f(base2(w[r], a.qscale) - m) * inv * (dp[r] - delta);
+            w[r] = row0 + 8 * (r / 4) + 4 * hf + r % 4 < end ? ds : 0.f;
+        }
+        f32_accumulate<1>(k + d0, a.c.ld_kv, row0, a.kv_len, a.head_dim - d0, w, 0, end, &acc);
+    }
 }
 
 template <int DP, bool VEC>
@@ -460,12 +471,19 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_kv(BwdArgs a) {
         ld = a.head_dim;
         grad = a.part[role] + (split * static_cast<int64_t>(a.n_bh) + bh) * a.kv_len * ld;
     }
-    const float check = store_columns<DP, VEC>(acc, role ? a.c.scale : 1.0f, grad + min(key, a.kv_len - 1) * ld, in, hf,
-                                               a.head_dim);
-    for (uint32_t redo = bad_rows(check, in); redo; redo &= redo - 1) {
-        const int i = k0 + __builtin_ctz(redo);
-        one_key<(DP + kWave - 1) / kWave>(a, role, i, t0 * kTileRows, t_end * kTileRows, q, k, v, dout, stats, plane,
-                                          grad + i * ld);
+    const int own_key = min(key, a.kv_len - 1);
+    const float scale = role ? a.c.scale : 1.0f;
+    grad += own_key * ld;
+    const float check = store_columns<DP, VEC>(acc, scale, grad, in, hf, a.head_dim);
+    // Keys whose result is not finite, in fp32 (split.hpp).
+    if (const uint32_t bad = bad_rows(check, in)) {
+        constexpr int kNb = kRedoBlocks<DP>;
+#pragma unroll 1
+        for (int d0 = 0; d0 < a.head_dim; d0 += 32 * kNb) {
+            f16v x[kNb];
+            keys_f32<kNb>(a, role, own_key, max(t0, pair_t0), t_end, d0, q, k, v, dout, stats, plane, x);
+            store_columns<32 * kNb, VEC>(x, scale, grad + d0, in && (bad >> li & 1), hf, a.head_dim - d0);
+        }
     }
 }
 
@@ -564,40 +582,21 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_q(BwdArgs a) {
         ld = a.head_dim;
         dq = a.part[2] + (split * static_cast<int64_t>(a.n_bh) + bh) * a.q_len * ld;
     }
-    const float check = store_columns<DP, VEC>(acc, a.c.scale, dq + min(my_q, a.q_len - 1) * ld, in, hf, a.head_dim);
-    // Queries whose result is not finite, in plain fp32 (split.hpp).
-    constexpr int kCh = (DP + kWave - 1) / kWave;
-    for (uint32_t redo = bad_rows(check, in); redo; redo &= redo - 1) {
-        const int i = qt * kTileRows + __builtin_ctz(redo);
-        const float* q = a.c.q + (b * a.q_len + i) * a.c.ld_q + hd;
-        const float* dout = a.c.dout + (b * a.q_len + i) * a.c.ld_dout + hd;
-        const float* v = a.c.v + b * a.kv_len * a.c.ld_kv + hd;
-        const float* stats = a.stats + bh * a.stats_ld + i;
-        const int64_t plane = a.n_bh * a.stats_ld;
-        const int keys = a.c.causal ? min(a.kv_len, i + 1) : a.kv_len;
-        float sum[kCh];
-#pragma unroll
-        for (int c = 0; c < kCh; ++c) sum[c] = 0.f;
-        for (int j = t0 * kTileRows; j < min(keys, n_tiles * kTileRows); ++j) {
-            float s = 0.f, dp = 0.f;
-#pragma unroll
-            for (int c = 0; c < kCh; ++c) {
-                const int d = lane + c * kWave;
-                if (d >= a.head_dim) continue;
-                s += q[d] * k[j * a.c.ld_kv + d];
-                dp += dout[d] * v[j * a.c.ld_kv + d];
-            }
-            s = base2(wave_sum(s), a.qscale);
-            dp = wave_sum(dp);
-            const float p = __builtin_amdgcn_exp2f(s - stats[0]) * stats[plane];
-            const float g = p * (dp - stats[2 * plane]);
-#pragma unroll
-            for (int c = 0; c < kCh; ++c)
-                if (lane + c * kWave < a.head_dim) sum[c] += g * k[j * a.c.ld_kv + lane + c * kWave];
+    const int64_t row = min(my_q, a.q_len - 1);
+    dq += row * ld;
+    const float check = store_columns<DP, VEC>(acc, a.c.scale, dq, in, hf, a.head_dim);
+    // Queries whose result is not finite, in fp32 (split.hpp); 32 dimensions a pass,
+    // so that the kernel stays at 128 registers and two workgroups a CU.
+    if (const uint32_t bad = bad_rows(check, in)) {
+#pragma unroll 1
+        for (int d0 = 0; d0 < a.head_dim; d0 += 32) {
+            f16v x;
+            queries_f32(a, a.c.causal ? min(a.kv_len, static_cast<int>(row) + 1) : a.kv_len, t0, wave_tiles, d0,
+                        a.c.q + (b * a.q_len + row) * a.c.ld_q + hd, k, a.c.v + b * a.kv_len * a.c.ld_kv + hd,
+                        a.c.dout + (b * a.q_len + row) * a.c.ld_dout + hd, a.stats + bh * a.stats_ld + row,
+                        a.n_bh * a.stats_ld, x);
+            store_columns<32, VEC>(&x, a.c.scale, dq + d0, in && (bad >> li & 1), hf, a.head_dim - d0);
         }
-#pragma unroll
-        for (int c = 0; c < kCh; ++c)
-            if (lane + c * kWave < a.head_dim) dq[i * ld + lane + c * kWave] = sum[c] * a.c.scale;
     }
 }
 

@@ -1,7 +1,8 @@
 // attention_tile.hpp -- the streamed tiles of the attention kernels
 // (attention.hip, attention_bwd.hip): 32 rows of a head on their way from
 // memory to LDS as three bf16 planes (split.hpp), in one of two layouts, and
-// the MFMA operands read from them.
+// the MFMA operands read from them; and the same products on the fp32 matrix
+// cores, for rows whose split result is not finite.
 #pragma once
 
 #include "split.hpp"
@@ -205,7 +206,16 @@ __device__ __forceinline__ uint32_t bad_rows(float check, bool in) {
     return static_cast<uint32_t>(b | b >> 32);
 }
 
-// For blocks whose split products are not finite (split.hpp), fp32 matrix cores:
+// ---------------------------------------------------------------------------
+// Blocks without a split.  A wave whose split result for its 32 rows holds a NaN
+// or an infinity computes them again with v_mfma_f32_32x32x2_f32, which gives what
+// fp32 arithmetic gives.  Operands come straight from memory, few at a time, and
+// kRedoBlocks x 32 dimensions of the result per pass (the scores again for each),
+// so that the kernels around it keep their registers.
+// ---------------------------------------------------------------------------
+template <int DP>
+constexpr int kRedoBlocks = DP >= 64 ? 2 : 1;
+
 // D[row0 + 8 (r / 4) + 4 hf + r % 4][lane's row] in register r: the products of
 // 32 rows of a matrix with one row per lane (li; both halves the same), times
 // `scale`.  Rows at and past len: the last one's, for the caller to mask.  Few
@@ -231,6 +241,55 @@ __device__ __forceinline__ f16v f32_scores(const float* base, int64_t ld, int ro
         }
     }
     return s;
+}
+
+// acc += rows^T w for 32 NB dimensions: rows row0 .. row0 + 31 of a matrix, w as
+// f32_scores lays it out (zero for rows a lane does not see), acc as store_columns
+// takes it.  A lane sees rows lo .. hi - 1; where some lane does not see a row that
+// others see, the row's values, which may not be finite, reach only those that do.
+// head_dim: dimensions from `base` on.
+template <int NB>
+__device__ __forceinline__ void f32_accumulate(const float* base, int64_t ld, int row0, int len, int head_dim, const f16v& w,
+                                               int lo, int hi, f16v* acc) {
+    const int li = threadIdx.x % 32, hf = threadIdx.x % kWave / 32;
+    const int end = min(row0 + kTileRows, len);
+    if (__all(lo <= row0 && hi >= end)) {
+        int first = row0 + 4 * hf;
+        asm volatile("" : "+v"(first));
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int row = first + 8 * (r / 4) + r % 4;
+            const float* p = base + min(row, len - 1) * ld;
+#pragma unroll
+            for (int d = 0; d < NB; ++d) {
+                const float v = p[min(32 * d + li, head_dim - 1)];
+                acc[d] = __builtin_amdgcn_mfma_f32_32x32x2f32(row < len && 32 * d + li < head_dim ? v : 0.f, w[r], acc[d], 0, 0, 0);
+            }
+            if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // no more than four rows in flight
+        }
+        return;
+    }
+#pragma unroll 1
+    for (int row = row0; row < end; ++row) {
+        const int at = row - row0;
+        float own = 0.f;  // this row's weight, in one of the lane halves
+#pragma unroll
+        for (int r = 0; r < 16; ++r) own = r == at % 4 + 4 * (at / 8) ? w[r] : own;
+        const float weight = __shfl(own, li + 32 * (at / 4 % 2));
+        const bool sees = lo <= row && row < hi;
+        const float* p = base + row * ld;
+        int last = head_dim - 1;
+        asm volatile("" : "+v"(last));  // the offsets are computed where they are used, not kept for the loop
+#pragma unroll
+        for (int d = 0; d < NB; ++d) {
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float v = p[min(32 * d + 8 * (r / 4) + 4 * hf + r % 4, last)];
+                acc[d][r] = sees ? acc[d][r] + weight * v : acc[d][r];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
 }
 
 }  // namespace mimir

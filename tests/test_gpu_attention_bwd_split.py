@@ -36,10 +36,12 @@ def test_split_backward_groups():
         c.close()
 
 
-def test_split_backward_special_values(ctx):
+# 1000 x 1000: keys and queries dealt to several workgroups.
+@pytest.mark.parametrize("n", [200, 1000])
+def test_split_backward_special_values(ctx, n):
     """A NaN key reaches the gradients of the queries that see it and no
     other; a query value that rounds to infinity in bf16 multiplies zeros."""
-    n, hd = 200, 32
+    hd = 32
     q, k, v, dout = rand_core(4, 1, n, n, hd)
     k[0, :, 3] = 0.0
     q[0, 7, 3] = 3.4e38
