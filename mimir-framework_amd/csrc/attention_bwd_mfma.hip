@@ -43,9 +43,11 @@
 #include "attention_tile.hpp"
 #include "internal.hpp"
 
+#include <float.h>
 #include <math.h>
 
 #include <algorithm>
+#include <cmath>
 
 using namespace mimir;
 
@@ -61,9 +63,11 @@ constexpr int kBlockFloats = kTileRows * kTileRows;
 struct BwdArgs {
     CoreBwd c;
     int32_t q_len, kv_len, heads, head_dim;
-    float qscale;              // scale * log2(e)
+    // A product q . k times `sign` (of the scale) orders like the scores, and qscale
+    // = |scale| log2(e) takes a difference of two to base-2 units.
+    float qscale, sign;
     // Per query of each (sequence, head), in rows of stats_ld queries: the max of
-    // its scores (base-2 units), 1 / (sum + 1e-9) and delta, three planes
+    // its signed products, 1 / (sum + 1e-9) and delta, three planes
     // [n_bh][stats_ld] (rows past q_len zero).
     float* stats;
     int64_t stats_ld;
@@ -95,32 +99,35 @@ __device__ __forceinline__ void coords(const BwdArgs& a, uint32_t bid, uint32_t*
     *bh = first + idx % owned;
 }
 
-// A score in base-2 units, rounded before a max is taken off it: the largest of a
-// row then gives exactly 1 wherever it is computed.
-__device__ __forceinline__ float base2(float s, float qscale) {
-#pragma clang fp contract(off)
-    return s * qscale;
+// exp(score - max) of a product with its query's max: the difference is taken before
+// it is scaled, so its error is relative to it and not to the two scores, and the
+// largest of a row gives exactly 1.
+__device__ __forceinline__ float weight(const BwdArgs& a, float product, float max) {
+    return __builtin_amdgcn_exp2f((product * a.sign - max) * a.qscale);
 }
 
 // Running max, sum and sum of e dP of a query; a lane half holds its own share of
 // the sums.
 struct RowStats {
     float m, l, d;
-    // One tile: scores s (base-2 units) and dP; -inf and 0 where the query does not
-    // see the key.
-    __device__ __forceinline__ void add(const f16v& s, const f16v& dp) {
-        float top = fmaxf(fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3])), fmaxf(fmaxf(s[4], s[5]), fmaxf(s[6], s[7])));
-        top = fmaxf(top, fmaxf(fmaxf(fmaxf(s[8], s[9]), fmaxf(s[10], s[11])),
-                               fmaxf(fmaxf(s[12], s[13]), fmaxf(s[14], s[15]))));
+    // One tile: products s and dP, of which the first `lim` of the lane's half count.
+    __device__ __forceinline__ void add(const BwdArgs& a, const f16v& s, const f16v& dp, int lim) {
+        f16v x;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) x[r] = 8 * (r / 4) + r % 4 < lim ? s[r] * a.sign : -INFINITY;
+        float top = fmaxf(fmaxf(fmaxf(x[0], x[1]), fmaxf(x[2], x[3])), fmaxf(fmaxf(x[4], x[5]), fmaxf(x[6], x[7])));
+        top = fmaxf(top, fmaxf(fmaxf(fmaxf(x[8], x[9]), fmaxf(x[10], x[11])),
+                               fmaxf(fmaxf(x[12], x[13]), fmaxf(x[14], x[15]))));
         top = fmaxf(m, fmaxf(top, __shfl_xor(top, 32)));
-        const float alpha = __builtin_amdgcn_exp2f(m - top);
+        const float alpha = __builtin_amdgcn_exp2f((m - top) * a.qscale);
         m = top;
         float sum = 0.f, dot = 0.f;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const float e = __builtin_amdgcn_exp2f(s[r] - top);
-            sum += e;
-            dot += e * dp[r];
+            const bool sees = 8 * (r / 4) + r % 4 < lim;
+            const float e = weight(a, s[r], top);
+            sum += sees ? e : 0.f;
+            dot += sees ? e * dp[r] : 0.f;
         }
         l = l * alpha + sum;
         d = d * alpha + dot;
@@ -170,22 +177,13 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_stats(BwdArgs a) {
     Split8 qx[kC], ox[kC];
     row_operand<DP, VEC>(q, hf, a.head_dim, 1.0f, qx);
     row_operand<DP, VEC>(dout, hf, a.head_dim, 1.0f, ox);
-    // A masked key counts in the max with its score of -1e9 (Model.cpp:6906-6920).
-    const RowStats none{end < a.kv_len ? -1e9f * kLog2e : -1e30f, 0.f, 0.f};
+    // A masked key counts in the max with its score of -1e9 (Model.cpp:6906-6920);
+    // the max starts at -1e30 (LayerOps.hpp:1052).
+    const RowStats none{fmaxf((end < a.kv_len ? -1e9f : -1e30f) * kLog2e / a.qscale, -FLT_MAX), 0.f, 0.f};
     RowStats st = none;
-    auto add = [&](RowStats& to, f16v& s, f16v& dp, int t) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[r] = base2(s[r], a.qscale);
-        if ((t + 1) * kTileRows > a.kv_len || (a.c.causal && t == qt)) {
-            const int lim = end - t * kTileRows - 4 * hf;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const bool sees = 8 * (r / 4) + r % 4 < lim;
-                s[r] = sees ? s[r] : -INFINITY;
-                dp[r] = sees ? dp[r] : 0.f;
-            }
-        }
-        to.add(s, dp);
+    auto add = [&](RowStats& to, const f16v& s, const f16v& dp, int t) {
+        if ((t + 1) * kTileRows > a.kv_len || (a.c.causal && t == qt)) to.add(a, s, dp, end - t * kTileRows - 4 * hf);
+        else to.add(a, s, dp, kTileRows);
     };
     if (t0 < n_tiles) {
         keys.stash(lds);
@@ -220,8 +218,8 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_stats(BwdArgs a) {
         RowStats redo = none;
 #pragma unroll 1
         for (int t = t0; t < wave_tiles; ++t) {
-            f16v s = f32_scores(k, a.c.ld_kv, t * kTileRows, a.kv_len, a.head_dim, q, 1.0f);
-            f16v dp = f32_scores(v, a.c.ld_kv, t * kTileRows, a.kv_len, a.head_dim, dout, 1.0f);
+            const f16v s = f32_scores(k, a.c.ld_kv, t * kTileRows, a.kv_len, a.head_dim, q, 1.0f);
+            const f16v dp = f32_scores(v, a.c.ld_kv, t * kTileRows, a.kv_len, a.head_dim, dout, 1.0f);
             add(redo, s, dp, t);
         }
         if (bad >> li & 1) st = redo;
@@ -247,7 +245,7 @@ __global__ __launch_bounds__(256) void attention_bwd_stats_sum(BwdArgs a) {
     float m = p[0], l = 0.f, d = 0.f;
     for (int s = 1; s < a.stats_splits; ++s) m = fmaxf(m, p[3 * s * plane]);
     for (int s = 0; s < a.stats_splits; ++s, p += 3 * plane) {
-        const float f = __builtin_amdgcn_exp2f(p[0] - m);
+        const float f = __builtin_amdgcn_exp2f((p[0] - m) * a.qscale);
         l += p[plane] * f;
         d += p[2 * plane] * f;
     }
@@ -279,7 +277,7 @@ __device__ __forceinline__ void keys_f32(const BwdArgs& a, int role, int key, in
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int i = row0 + 8 * (r / 4) + 4 * hf + r % 4;  // below stats_ld
-            float p = __builtin_amdgcn_exp2f(base2(w[r], a.qscale) - stats[i]) * stats[plane + i];
+            float p = weight(a, w[r], stats[i]) * stats[plane + i];
             if (role) p *= dp[r] - stats[2 * plane + i];
             w[r] = i >= lo && i < a.q_len ? p : 0.f;
         }
@@ -301,7 +299,7 @@ __device__ __forceinline__ void queries_f32(const BwdArgs& a, int end, int t0, i
         const f16v dp = f32_scores(v, a.c.ld_kv, row0, a.kv_len, a.head_dim, dout, 1.0f);
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-            const float ds = __builtin_amdgcn_exp2f(base2(w[r], a.qscale) - m) * inv * (dp[r] - delta);
+            const float ds = weight(a, w[r], m) * inv * (dp[r] - delta);
             w[r] = row0 + 8 * (r / 4) + 4 * hf + r % 4 < end ? ds : 0.f;
         }
         f32_accumulate<1>(k + d0, a.c.ld_kv, row0, a.kv_len, a.head_dim - d0, w, 0, end, &acc);
@@ -413,7 +411,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_kv(BwdArgs a) {
                     f4 p;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        p[e] = __builtin_amdgcn_exp2f(base2(x[r + e], a.qscale) - m[e]) * inv[e];
+                        p[e] = weight(a, x[r + e], m[e]) * inv[e];
                         if (edge && (key >= a.kv_len || (a.c.causal && key > t * kTileRows + 8 * (r / 4) + 4 * hf + e)))
                             p[e] = 0.f;
                         x[r + e] = p[e];
@@ -703,7 +701,8 @@ int attention_bwd_mfma(mimir_ctx* ctx, const CoreBwd& c, float* work) {
     a.kv_len = static_cast<int32_t>(c.kv_len);
     a.heads = static_cast<int32_t>(c.heads);
     a.head_dim = static_cast<int32_t>(c.head_dim);
-    a.qscale = c.scale * kLog2e;
+    a.qscale = std::max(std::fabs(c.scale) * kLog2e, FLT_MIN);  // a scale of 0: all weights the same
+    a.sign = c.scale < 0 ? -1.0f : 1.0f;
     a.ds = work;  // 16-byte aligned blocks first
     a.stats = work + ds_floats(c, group);
     a.stats_ld = stats_ld;

@@ -117,3 +117,33 @@ def test_split_backward_saturated_rows(ctx, n, hd, causal):
     err = np.abs(got[0][0] - dq)
     print(f"saturated n={n} hd={hd}: worst error {(err / tol)[rows].max():.3g} of the bound, {err[rows].max():.3g}", flush=True)
     assert (err <= tol)[rows].all()
+
+
+@pytest.mark.parametrize("scale", [0.125, -0.125])
+@pytest.mark.parametrize("causal", [False, True])
+def test_split_backward_large_scores(ctx, causal, scale):
+    """Integer q and k, so q . k is exact, with scores of about 256 that differ by a
+    few units: the weights' error is that of exp at the difference (up to 16 in
+    base-2 units where a weight matters: 16 x 2 u x ln 2, and 4 u for exp, the sum
+    and its reciprocal), not of the scores."""
+    r = np.random.default_rng(2)
+    n, hd = 200, 64
+    q, k = (r.integers(-2, 3, (1, n, hd)).astype(np.float32) for _ in range(2))
+    q[..., 0], k[..., 0] = 64.0, np.copysign(32.0, scale)
+    v, dout = (r.standard_normal((1, n, hd)).astype(np.float32) for _ in range(2))
+    got = gpu_core_bwd(ctx, q, k, v, dout, 1, causal, scale=scale)
+    want, _ = attention_bwd64(q[0], k[0], v[0], dout[0], 1, causal, scale)
+    s = scale * (q[0].astype(np.float64) @ k[0].astype(np.float64).T)
+    if causal:
+        s[np.triu(np.ones(s.shape, bool), 1)] = -np.inf
+    p = np.exp(s - s.max(1, keepdims=True))
+    p /= p.sum(1, keepdims=True)
+    rel = (32 * np.log(2) + 4) * O.U32
+    tol = (rel + 1e-6) * (p.T @ np.abs(dout[0])) + 1e-9  # 1e-6: the sum over 200 queries, sqrt(n) u and its splits
+    err = np.abs(got[2][0] - want[2])
+    print(f"large scores: dv {(err / tol).max():.3g} of the bound", flush=True)
+    assert (err <= tol).all()
+    for g, w, name in zip(got[:2], want[:2], ("dq", "dk")):
+        e = np.linalg.norm(g[0] - w) / np.linalg.norm(w)
+        print(f"  {name} {e:.3g}", flush=True)
+        assert e <= 2 * rel, name
