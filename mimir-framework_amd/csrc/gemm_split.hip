@@ -360,6 +360,10 @@ namespace mimir {
 // 177; 100 x 1024 x 1024 7.9 / 6.9 / 8.7; 777 x 768 x 256 7.5 / 7.3 / 9.0; 2048 x 768 x
 // 256 14.1 / 10.8 / 16.7; 257 x 129 x 511, B transposed 11.6 / 5.4 / 9.1; 2048 x 3072 x
 // 1024 87 / 95 / 92; 4096^3 747 / 919 / 920; 32 x 512 x 1024 x 128 35 / 45 / 45.
+// Fewer terms than kLeastK go to the library: six of the nine products of two
+// splits leave a single product 8.7e-8 off where fp32 rounds it to 5.9e-8; from four
+// terms on, the split's sum is the closer one.
+constexpr int64_t kLeastK = 4;
 constexpr int64_t kLargeTiles = 1024, kSmallTiles = 256, kSmallK = 896, kShortTiles = 640, kShortK = 256;
 
 static int64_t tile_count(int64_t M, int64_t N, int64_t batch, int64_t t) {
@@ -375,7 +379,7 @@ static int pick(const mimir_ctx* ctx, bool ak, bool bk, bool vec, int64_t M, int
                 int64_t ldb, int64_t batch) {
     constexpr int64_t kMost = int64_t{1} << 30;
     const int force = ctx->tune.gemm;  // one of the above, or 1 for the library
-    if (force == 1 || ctx->tune.blas_lt == 0 || K == 0 || M > kMost || N > kMost || K > kMost) return 0;
+    if (force == 1 || ctx->tune.blas_lt == 0 || K < kLeastK || M > kMost || N > kMost || K > kMost) return 0;
     const auto below = [](int64_t floats) { return floats < (int64_t{1} << 29); };  // byte offsets within a tile
     if (force == 128 || (!force && tile_count(M, N, batch, 128) >= kLargeTiles))
         return below((ak ? 128 : kStep) * lda) && below((bk ? 128 : kStep) * ldb) ? 128 : 0;

@@ -70,3 +70,19 @@ def test_products_special_values(tile):
         for b in bufs:
             b.free()
         c.close()
+
+
+def test_products_of_one_term_are_rounded_once(ctx):
+    """One token of width 1: the layer is x wv wout, two products of one term, each
+    the float32 product."""
+    r = np.random.default_rng(7)
+    x, w = r.standard_normal(200).astype(np.float32), r.standard_normal((200, 4)).astype(np.float32)
+    bufs = [_dev(ctx, x), _dev(ctx, w), _dev(ctx, np.zeros_like(x))]
+    xb, wb, yb = bufs
+    try:
+        for i in range(x.size):
+            ctx.self_attention(xb.offset(i, (1,)), 1, 1, 1, True, wb.offset(4 * i, (4,)), 4, yb.offset(i, (1,)))
+        np.testing.assert_array_equal(yb.numpy().ravel(), x * w[:, 2] * w[:, 3])
+    finally:
+        for b in bufs:
+            b.free()
