@@ -95,6 +95,7 @@ using LtKey = std::tuple<int, int, int64_t, int64_t, int64_t, int64_t, int64_t, 
 constexpr size_t kMaxPlans = 1024;
 struct LtState {
     hipblasLtHandle_t handle = nullptr;
+    int version = 0;      // 100000 major + 100 minor + patch
     bool failed = false;  // the handle could not be created: rocBLAS only
     std::map<LtKey, LtPlan> plans;
 };
@@ -114,6 +115,8 @@ LtState* lt_of(mimir_ctx* ctx) {
         if (hipblasLtCreate(&s->handle) != HIPBLAS_STATUS_SUCCESS) {
             s->handle = nullptr;
             s->failed = true;
+        } else if (hipblasLtGetVersion(s->handle, &s->version) != HIPBLAS_STATUS_SUCCESS) {
+            s->version = 0;
         }
         ctx->blaslt = s;
     }
@@ -188,6 +191,11 @@ int gemm_f32(mimir_ctx* ctx, int64_t M, int64_t N, int64_t K, const float* A, in
 }
 
 bool gemm_lt(mimir_ctx* ctx) { return lt_of(ctx) != nullptr; }
+
+int gemm_lt_version(mimir_ctx* ctx) {
+    const LtState* s = lt_of(ctx);
+    return s ? s->version : 0;
+}
 
 int gemm_f32_ex(mimir_ctx* ctx, bool trans_a, bool trans_b, int64_t M, int64_t N, int64_t K, float alpha,
                 const float* A, int64_t lda, int64_t stride_a, const float* B, int64_t ldb, int64_t stride_b,

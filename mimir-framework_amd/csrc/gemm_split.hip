@@ -356,15 +356,27 @@ namespace mimir {
 // 256.  The rest goes to the library: as fast up to the large ones, and a layer's
 // products run 10% faster there than with this file's tiles.  Measured on MI355X, us
 // (gemm_strip or gemm_tile / library / the library in a PyTorch process): 300 x 512 x
-// 512 5.5 / 6.3 / 9.0; 512^3 5.8 / 6.5 / 8.7; 256 x 256 x 777, A transposed 7.4 / 6.0 /
-// 177; 100 x 1024 x 1024 7.9 / 6.9 / 8.7; 777 x 768 x 256 7.5 / 7.3 / 9.0; 2048 x 768 x
-// 256 14.1 / 10.8 / 16.7; 257 x 129 x 511, B transposed 11.6 / 5.4 / 9.1; 2048 x 3072 x
-// 1024 87 / 95 / 92; 4096^3 747 / 919 / 920; 32 x 512 x 1024 x 128 35 / 45 / 45.
+// 512 5.5 / 6.3 / 9.0; 512^3 5.8 / 6.5 / 8.7; 100 x 1024 x 1024 7.9 / 6.9 / 8.7; 2048 x
+// 768 x 256 14.1 / 10.8 / 16.7; 257 x 129 x 511, B transposed 11.6 / 5.4 / 9.1; 2048 x
+// 3072 x 1024 87 / 95 / 92; 4096^3 747 / 919 / 920; 32 x 512 x 1024 x 128 35 / 45 / 45.
+//
+// Those limits are for the hipBLASLt that PyTorch brings (1.0), which takes 33 to 178
+// us for many small products (256 x 256 x 777 117, 128 x 768 x 256 33).  From
+// kGoodLibrary on (1.2, a program without PyTorch) the library is good at them, and
+// the limits lie where a call here is no slower.  Calls in a row, us (here /
+// library), and the kernels alone: 128 x 768 x 256 4.8 / 7.7 (5.0 / 4.9), 512^3 5.5 /
+// 7.4 (5.9 / 6.8), 256 x 256 x 777, A transposed 7.5 / 7.3 (7.7 / 6.4): up to 512.  Both
+// operands contiguous along the contraction (B transposed): 256 x 768 x 128 4.3 / 7.6
+// (4.4 / 4.3), 512 x 512 x 768 9.1 / 7.4 (8.8 / 7.3): up to 128, and none of more than
+// 256 tiles (777 x 768 x 256 8.5 / 7.4).  More than 256 tiles otherwise: 700 x 700 x 256
+// kernels 6.0 / 6.4, x 128 5.8 / 5.3: only above 128.
 // Fewer terms than kLeastK go to the library: six of the nine products of two
 // splits leave a single product 8.7e-8 off where fp32 rounds it to 5.9e-8; from four
 // terms on, the split's sum is the closer one.
 constexpr int64_t kLeastK = 4;
 constexpr int64_t kLargeTiles = 1024, kSmallTiles = 256, kSmallK = 896, kShortTiles = 640, kShortK = 256;
+constexpr int kGoodLibrary = 100200;
+constexpr int64_t kGoodLibraryK = 512, kGoodLibraryShortK = 128;
 
 static int64_t tile_count(int64_t M, int64_t N, int64_t batch, int64_t t) {
     return (M + t - 1) / t * ((N + t - 1) / t) * batch;
@@ -375,7 +387,7 @@ static bool vectors(bool ak, bool bk, int64_t K, const float* A, int64_t lda, in
            (!bk || (ldb % 4 == 0 && stride_b % 4 == 0 && aligned16(B)));
 }
 // 0: the library; 128: gemm_tile; 16, 4: gemm_strip with so many waves.
-static int pick(const mimir_ctx* ctx, bool ak, bool bk, bool vec, int64_t M, int64_t N, int64_t K, int64_t lda,
+static int pick(mimir_ctx* ctx, bool ak, bool bk, bool vec, int64_t M, int64_t N, int64_t K, int64_t lda,
                 int64_t ldb, int64_t batch) {
     constexpr int64_t kMost = int64_t{1} << 30;
     const int force = ctx->tune.gemm;  // one of the above, or 1 for the library
@@ -386,8 +398,13 @@ static int pick(const mimir_ctx* ctx, bool ak, bool bk, bool vec, int64_t M, int
     if (!below(ak ? 32 * lda + K : K * lda + 32) || !below(bk ? 32 * ldb + K : K * ldb + 32)) return 0;
     if (force) return force;
     const int64_t tiles = tile_count(M, N, batch, 32);
-    if (tiles <= kSmallTiles) return K <= (vec || (!ak && !bk) ? kSmallK : kShortK) ? 16 : 0;
-    return tiles <= kShortTiles && K <= kShortK ? 4 : 0;
+    if (tiles > kShortTiles) return 0;
+    int64_t least = 0, most = tiles > kSmallTiles || !(vec || (!ak && !bk)) ? kShortK : kSmallK;
+    if (gemm_lt_version(ctx) >= kGoodLibrary) {
+        if (tiles > kSmallTiles) least = ak && bk ? most : kGoodLibraryShortK;
+        else most = std::min(most, ak && bk ? kGoodLibraryShortK : kGoodLibraryK);
+    }
+    return K <= least || K > most ? 0 : tiles <= kSmallTiles ? 16 : 4;
 }
 
 int gemm_split(mimir_ctx* ctx, bool trans_a, bool trans_b, int64_t M, int64_t N, int64_t K, float alpha, const float* A,

@@ -112,8 +112,8 @@ int retire_or_free(mimir_ctx* ctx, void* p);
 void graph_pin(mimir_ctx* ctx);
 int graph_unpin(mimir_ctx* ctx);
 
-// Row-major fp32 C[M x N] = A[M x K] * B[K x N] on the context's stream
-// (rocBLAS; gemm.hip), and the release of its handle at context teardown.
+// Row-major fp32 C[M x N] = A[M x K] * B[K x N] on the context's stream (gemm.hip),
+// and the release of the libraries' handles at context teardown.
 int gemm_f32(mimir_ctx* ctx, int64_t M, int64_t N, int64_t K, const float* A, int64_t lda, const float* B,
              int64_t ldb, float* C, int64_t ldc);
 // The general form: row-major C = alpha op(A) op(B) + beta C over `batch`
@@ -131,6 +131,9 @@ int gemm_split(mimir_ctx* ctx, bool trans_a, bool trans_b, int64_t M, int64_t N,
 // Whether products go to hipBLASLt (unless MIMIR_TUNE blas=0), where the
 // transposed-operand forms run as fast as the plain ones.
 bool gemm_lt(mimir_ctx* ctx);
+// hipBLASLt's version (100000 major + 100 minor + patch) as the process has loaded
+// it; 0 without it.
+int gemm_lt_version(mimir_ctx* ctx);
 
 // The attention core, not causal, for at most kDecodeQueries queries per sequence
 // (attention_decode.hip), of heads up to 128; qscale = scale * log2(e).  vec:
