@@ -241,10 +241,14 @@ int mimir_rope_fwd(mimir_ctx* ctx, const float* q, float* q_out, int64_t q_heads
  * (h+1)*head_dim).  The reference's scale is 1.0f / sqrtf(head_dim).
  * head_dim <= 2048 (above 128 a plain fp32 vector kernel runs instead of the
  * matrix-core one).  fp32 precision (each fp32 operand three bf16 terms on the
- * matrix cores, accumulated in fp32), no score matrix in memory.  out must not overlap q, k or v.  kv_len == 0 gives zeros;
+ * matrix cores, accumulated in fp32; a value below 2^-110 keeps an absolute
+ * precision of 2^-134, so fewer than 24 bits), no score matrix in memory.
+ * out must not overlap q, k or v.  kv_len == 0 gives zeros;
  * batch == 0 or q_len == 0 is a no-op.  Device pointers, stream order.  Up to
  * 8 queries without a mask, and 737 keys or more where few workgroups have them,
- * may use the context's fixed workspace (allocated with the context). */
+ * use 33 MiB of device memory that the first such call of a context allocates
+ * (also under capture) and the context keeps; where there is none the call runs
+ * without, slower. */
 int mimir_attention_fwd(mimir_ctx* ctx, const float* q, int64_t ld_q, const float* k, const float* v,
                         int64_t ld_kv, float* out, int64_t ld_out, int64_t batch, int64_t q_len,
                         int64_t kv_len, int64_t heads, int64_t head_dim, float scale, int causal);

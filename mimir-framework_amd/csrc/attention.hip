@@ -525,7 +525,8 @@ int mimir_attention_fwd(mimir_ctx* ctx, const float* q, int64_t ld_q, const floa
                                        a.qscale, vec);
     if (mfma_takes(head_dim, ld_kv)) {
         a.splits = static_cast<int32_t>(splits_for(ctx, batch * heads, q_len, kv_len, head_dim, kFixedWorkBytes / 4));
-        a.part = a.splits > 1 ? static_cast<float*>(ctx->fixed_work) : nullptr;
+        a.part = a.splits > 1 ? fixed_work(ctx) : nullptr;
+        if (!a.part) a.splits = 1;
         return launch_any(ctx, a, batch * heads, vec);
     }
     MIMIR_REQUIRE(ctx, dispatch_fits(batch * heads, kGenericWaves * kWave) && (q_len + kGenericWaves - 1) / kGenericWaves <= 65535,

@@ -273,12 +273,13 @@ int attention_decode_launch(mimir_ctx* ctx, const float* q, int64_t ld_q, const 
     const int tuned = ctx->tune.decode_splits;
     if (tuned > 0) splits = std::min<int64_t>(tuned, kv_len);
     const int64_t floats = batch * heads * q_len * splits * (head_dim + 2);
-    if (splits > 1 && floats * 4 > static_cast<int64_t>(kFixedWorkBytes)) splits = 1;
+    float* part = splits > 1 && floats * 4 <= static_cast<int64_t>(kFixedWorkBytes) ? fixed_work(ctx) : nullptr;
+    if (!part) splits = 1;
     int64_t span = (kv_len + splits - 1) / splits;
     splits = (kv_len + span - 1) / span;
     MIMIR_REQUIRE(ctx, dispatch_fits(rows * splits, kThreads) && dispatch_fits(batch * heads * q_len, kWave),
                   "attention: grid of %lld workgroups exceeds the limit", (long long)(rows * splits));
-    DecodeArgs a{q, k, v, out, splits > 1 ? static_cast<float*>(ctx->fixed_work) : nullptr, ld_q, ld_kv, ld_out,
+    DecodeArgs a{q, k, v, out, splits > 1 ? part : nullptr, ld_q, ld_kv, ld_out,
                  static_cast<int32_t>(q_len), static_cast<int32_t>(kv_len), static_cast<int32_t>(heads),
                  static_cast<int32_t>(head_dim), static_cast<int32_t>(q_blocks), static_cast<int32_t>(splits),
                  static_cast<int32_t>(span), qscale};

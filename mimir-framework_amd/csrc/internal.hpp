@@ -31,9 +31,10 @@ struct mimir_ctx {
     // Device address of this GPU's fixed scratch array (backward.hip), for
     // the entry point that allocates nothing; set at context creation.
     void* noalloc_scratch = nullptr;
-    // Workspace of kFixedWorkBytes, allocated with the context (so that the
-    // ops that use it allocate nothing): the partial outputs of a decoding
-    // step's splits (attention_decode.hip), in stream order.
+    // Workspace of kFixedWorkBytes for the forward attention core, which takes no
+    // scratch (a layer has its activations there): the partial outputs of keys
+    // dealt to several workgroups (attention.hip, attention_decode.hip), in stream
+    // order.  Made by the first call that deals them (fixed_work), kept.
     void* fixed_work = nullptr;
     // This GPU's columns of 1.0f then -0.0f (mimir::kUnitCols each), the
     // weights of a row kernel's absent scale / bias (norm.hip).
@@ -139,7 +140,12 @@ int gemm_lt_version(mimir_ctx* ctx);
 // (attention_decode.hip), of heads up to 128; qscale = scale * log2(e).  vec:
 // head_dim, the strides and the pointers are 16-byte multiples.
 constexpr int kDecodeQueries = 8;
-constexpr size_t kFixedWorkBytes = size_t(64) << 20;
+// What keys dealt to several workgroups need at most: 256 workgroups of 256 queries,
+// 128 dimensions and the max and sum of each.
+constexpr size_t kFixedWorkBytes = sizeof(float) * 256 * 256 * 130;
+// The workspace, null where there is no memory for it: the call then runs on one
+// workgroup per query block.
+float* fixed_work(mimir_ctx* ctx);
 bool attention_decode_applies(int64_t bh, int64_t q_len, int64_t kv_len, int64_t head_dim, bool causal);
 int attention_decode_launch(mimir_ctx* ctx, const float* q, int64_t ld_q, const float* k, const float* v, int64_t ld_kv,
                             float* out, int64_t ld_out, int64_t batch, int64_t q_len, int64_t kv_len, int64_t heads,

@@ -108,6 +108,21 @@ int mimir::ensure_scratch(mimir_ctx* ctx, size_t bytes, void** out) {
     return MIMIR_OK;
 }
 
+float* mimir::fixed_work(mimir_ctx* ctx) {
+    if (!ctx->fixed_work) {
+        // A stream may be capturing, this context's or another thread's: the
+        // allocation is no part of the graph.
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) return nullptr;
+        if (hipMalloc(&ctx->fixed_work, kFixedWorkBytes) != hipSuccess) {
+            (void)hipGetLastError();
+            ctx->fixed_work = nullptr;
+        }
+        (void)hipThreadExchangeStreamCaptureMode(&mode);
+    }
+    return static_cast<float*>(ctx->fixed_work);
+}
+
 extern "C" {
 
 int mimir_ctx_create(int device, mimir_ctx** out) {
@@ -126,16 +141,9 @@ int mimir_ctx_create(int device, mimir_ctx** out) {
         return MIMIR_EDEVICE;
     }
     ctx->stream = ctx->own_stream;
-    if (hipMalloc(&ctx->fixed_work, kFixedWorkBytes) != hipSuccess) {
-        (void)hipGetLastError();
-        (void)hipStreamDestroy(ctx->own_stream);
-        delete ctx;
-        return MIMIR_ENOMEM;
-    }
     int init_st = noalloc_scratch_init(ctx);
     if (init_st == MIMIR_OK) init_st = norm_init(ctx);
     if (int st = init_st) {
-        (void)hipFree(ctx->fixed_work);
         (void)hipStreamDestroy(ctx->own_stream);
         delete ctx;
         return st;
@@ -152,7 +160,7 @@ int mimir_ctx_destroy(mimir_ctx* ctx) {
         gemm_release(ctx);
         for (auto& kv : ctx->allocs) (void)hipFree(kv.first);
         if (ctx->scratch) (void)hipFree(ctx->scratch);
-        (void)hipFree(ctx->fixed_work);
+        if (ctx->fixed_work) (void)hipFree(ctx->fixed_work);
         for (void* p : ctx->retired) (void)hipFree(p);
         (void)hipStreamDestroy(ctx->own_stream);
     }

@@ -2,11 +2,13 @@
 both workgroup sizes at the edges of their query blocks and key tiles, every
 padded head size, and values that have no split (infinities, NaN, the largest
 floats), against float64."""
+import ctypes
 import time
 
 import numpy as np
 import pytest
 
+import mimir_hip as M
 import oracle as O
 from _attention import assert_attention_close, attention64
 from test_gpu_attention import gpu_attention, rand_qkv
@@ -115,3 +117,58 @@ def test_a_nan_costs_no_more_than_a_few_calls(ctx):
     finally:
         for b in bufs:
             b.free()
+
+
+def _hip():
+    for name in ("libamdhip64.so", "/opt/rocm/lib/libamdhip64.so"):
+        try:
+            return ctypes.CDLL(name)
+        except OSError:
+            continue
+    pytest.skip("libamdhip64 not loadable")
+
+
+def test_a_context_takes_no_workspace_before_it_needs_it():
+    hip = _hip()
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    with M.Context(0):  # what the process and the GPU keep exists now
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        before = free.value
+        with M.Context(0):
+            assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+            assert before - free.value < 16 << 20
+
+
+@pytest.mark.parametrize("lq", [1, 300])
+def test_first_split_call_under_capture(lq):
+    """The first call that deals its keys to several workgroups, made while the
+    stream is captured: replayed three times, the eager call's bits each time."""
+    hip = _hip()
+    lk, heads, hd = 1500, 2, 64
+    q, k, v = rand_qkv(3, 1, lq, lk, heads * hd)
+    graph, execution = ctypes.c_void_p(), ctypes.c_void_p()
+    with M.Context(0) as c:
+        bufs = [c.to_device(a) for a in (q, k, v)] + [c.empty(q.shape), c.empty(q.shape)]
+        dq, dk, dv, out, eager = bufs
+        c.sync()
+        stream = ctypes.c_void_p(c.lib.mimir_ctx_stream(c.handle))
+        try:
+            assert hip.hipStreamBeginCapture(stream, 0) == 0  # the strictest mode
+            c.attention(dq, dk, dv, out, 1, lq, lk, heads, hd)
+            assert hip.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+            assert hip.hipGraphInstantiate(ctypes.byref(execution), graph, None, None, ctypes.c_size_t(0)) == 0
+            c.attention(dq, dk, dv, eager, 1, lq, lk, heads, hd)
+            want = eager.numpy()
+            for _ in range(3):
+                c.fill(out.ptr, np.nan, out.size)
+                assert hip.hipGraphLaunch(execution, stream) == 0
+                np.testing.assert_array_equal(out.numpy(), want)
+                c.attention(dq, dk, dv, eager, 1, lq, lk, heads, hd)
+        finally:
+            if execution:
+                hip.hipGraphExecDestroy(execution)
+            if graph:
+                hip.hipGraphDestroy(graph)
+            for b in bufs:
+                b.free()
+    assert_attention_close(want.reshape(lq, -1), *attention64(q[0], k[0], v[0], heads, False, O.attention_scale(hd)), "captured")
