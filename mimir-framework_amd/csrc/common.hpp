@@ -109,13 +109,18 @@ __device__ __forceinline__ void st_out(float* p, f4 v) {
 // ---------------------------------------------------------------------------
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 
-// A row of 513 to 1536 floats gets a wave where there are more rows than this
-// (two for each SIMD), else a workgroup: fewer waves leave the GPU idle.
-// Measured on MI355X, us (wave / workgroup per row): add + RMSNorm, 1024 rows of
-// 1001 6.8 / 5.0, of 1535 8.1 / 6.3, 4096 rows of 1535 17.3 / 18.7; LayerNorm, 512
-// rows of 1535 6.2 / 5.1, 8192 of 1001 12.4 / 14.9.  Wider rows are a workgroup's at
-// any count: LayerNorm of 2047, 64 rows 6.2 / 4.9, 4096 13.2 / 14.3, 8192 31.8 / 26.7.
-constexpr int64_t kAnyWaveRows = 2048;
+// A row of 513 to 1536 floats gets a wave where there are more rows than this (2.5
+// for each SIMD), else a workgroup: fewer waves leave the GPU idle.  Measured on
+// MI355X, us (wave / workgroup per row): add + RMSNorm, 2049 rows of 1001 8.5 / 6.1,
+// 2560 9.2 / 8.4, 3500 10.6 / 10.7; 2560 of 1535 12.8 / 12.3, 4096 16.9 / 18.9; softmax,
+// 2560 rows of 1201 7.7 / 7.3, 3500 8.4 / 9.0; LayerNorm, 2560 of 1001 6.7 / 6.2, 8192
+// of 1001 12.4 / 14.9.  Wider rows are a workgroup's at any count: LayerNorm of 2047,
+// 64 rows 6.2 / 4.9, 4096 13.2 / 14.3, 8192 31.8 / 26.7.
+constexpr int64_t kAnyWaveRows = 2560;
+
+// Threads of a workgroup that gives TPR of them to a row: one row each from two waves
+// a row on.
+constexpr int any_block(int tpr) { return tpr < 2 * kWave ? 4 * kWave : tpr; }
 
 struct RowSpan {
     int full, rem;  // whole vectors, floats left

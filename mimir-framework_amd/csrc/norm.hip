@@ -365,16 +365,16 @@ int launch_vec(mimir_ctx* ctx, const NormArgs& args) {
 // Rows the vector kernel cannot take (a width that is not a multiple of 4, or
 // unaligned pointers), up to 16384 floats: the row in registers as 16-byte
 // vectors at 4-byte addresses, TPR threads per row (a wave up to 1536 floats,
-// so its sums need no barrier; a workgroup above, and where the rows are few).  One read of the row (and of
-// the residual for add + RMSNorm, whose sum is written once, after the
-// reduction's barrier: r_out may be r, and a row's last vector overlaps
-// nothing).  Bound by HBM like the vector kernel; measured at 8191 x 1001,
+// so its sums need no barrier; a workgroup above, and where the rows are few).
+// One read of the row (and of the residual for add + RMSNorm, whose sum is
+// written once, after the reduction's barrier: r_out may be r, and a row's last
+// vector overlaps nothing).  Bound by HBM like the vector kernel; measured at 8191 x 1001,
 // LayerNorm 12.5-13.7 us (4.8-5.2 TB/s) against 21.6 in 4-byte columns, one
 // workgroup per row.
 template <Norm K, int TPR, int VPT, bool KEEP>
-__global__ __launch_bounds__(kBlock) void norm_rows_any(NormArgs a) {
-    constexpr int RPB = kBlock / TPR, NW = TPR / kWave;
-    __shared__ float lds[2][kBlock / kWave];
+__global__ __launch_bounds__(any_block(TPR)) void norm_rows_any(NormArgs a) {
+    constexpr int RPB = any_block(TPR) / TPR, NW = TPR / kWave;
+    __shared__ float lds[2][RPB * NW];
     const int t = threadIdx.x % TPR, sub = threadIdx.x / TPR;
     const int64_t row = static_cast<int64_t>(blockIdx.x) * RPB + sub;
     if constexpr (NW == 1) {
@@ -391,6 +391,18 @@ __global__ __launch_bounds__(kBlock) void norm_rows_any(NormArgs a) {
     }
     const float n = static_cast<float>(a.cols);
     if constexpr (K == Norm::Layer) {
+        // Where a row has few vectors a thread, too few waves hide another latency
+        // after the sums: the weights are on their way with the row.
+        constexpr bool kEarly = NW > 1 && VPT <= 3;
+        f4 g[kEarly ? VPT : 1], b[kEarly ? VPT : 1];
+        if constexpr (kEarly) {
+            const RowSpan gw(a.g ? a.cols : 0), bw(a.g && a.b ? a.cols : 0);
+#pragma unroll
+            for (int j = 0; j < VPT; ++j) {
+                g[j] = ld_slot<false>(a.g, j * TPR + t, gw, 1.0f);
+                b[j] = ld_slot<false>(a.b, j * TPR + t, bw, -0.0f);  // x 1 and + -0 change no bit
+            }
+        }
         float s = 0.0f;
 #pragma unroll
         for (int j = 0; j < VPT; ++j) s += (v[j].x + v[j].y) + (v[j].z + v[j].w);
@@ -411,7 +423,10 @@ __global__ __launch_bounds__(kBlock) void norm_rows_any(NormArgs a) {
         for (int j = 0; j < VPT; ++j) {
             const int c4 = j * TPR + t;
             f4 o = (v[j] - mean) * inv_std;
-            if (a.g) {
+            if constexpr (kEarly) {
+                o *= g[j];
+                o += b[j];
+            } else if (a.g) {
                 o *= ld_slot<false>(a.g, c4, w, 1.0f);
                 if (a.b) o += ld_slot<false>(a.b, c4, w, 0.0f);
             }
@@ -434,11 +449,12 @@ __global__ __launch_bounds__(kBlock) void norm_rows_any(NormArgs a) {
 
 template <Norm K, int TPR, int VPT>
 int launch_any(mimir_ctx* ctx, const NormArgs& a) {
+    constexpr int kBS = any_block(TPR);
     unsigned grid;
-    if (!grid_for(a.rows, kBlock / TPR, kBlock, &grid))
+    if (!grid_for(a.rows, kBS / TPR, kBS, &grid))
         return fail(ctx, MIMIR_EINVAL, "norm: %lld rows exceed the grid limit", (long long)a.rows);
-    if (ctx->keep_outputs) norm_rows_any<K, TPR, VPT, true><<<grid, kBlock, 0, ctx->stream>>>(a);
-    else norm_rows_any<K, TPR, VPT, false><<<grid, kBlock, 0, ctx->stream>>>(a);
+    if (ctx->keep_outputs) norm_rows_any<K, TPR, VPT, true><<<grid, kBS, 0, ctx->stream>>>(a);
+    else norm_rows_any<K, TPR, VPT, false><<<grid, kBS, 0, ctx->stream>>>(a);
     return launched(ctx, "norm_rows_any");
 }
 
@@ -468,6 +484,12 @@ int dispatch(mimir_ctx* ctx, const NormArgs& a) {
         if (a.cols <= 512) return launch_any<K, 64, 2>(ctx, a);
         const bool wave = a.rows > kAnyWaveRows;
         if (a.cols <= 1024) return wave ? launch_any<K, 64, 4>(ctx, a) : launch_any<K, 256, 1>(ctx, a);
+        // LayerNorm, two sums: two waves a row, three vectors a thread, up to 3072 rows.
+        // us (256 threads or a wave / this): 2048 rows of 1201 6.6 / 6.0, of 1535 7.0 /
+        // 6.7, 2560 of 1535 8.2 / 7.0; 4096 of 1535 9.7 / 10.5.
+        if constexpr (K == Norm::Layer) {
+            if (a.cols <= 1536 && a.rows <= 3072) return launch_any<K, 128, 3>(ctx, a);
+        }
         if (a.cols <= 1536 && wave) return launch_any<K, 64, 6>(ctx, a);
         if (a.cols <= 2048) return launch_any<K, 256, 2>(ctx, a);
         if (a.cols <= 4096) return launch_any<K, 256, 4>(ctx, a);

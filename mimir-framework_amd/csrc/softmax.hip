@@ -128,14 +128,14 @@ __global__ __launch_bounds__(kBlock) void softmax_rows_generic(SoftmaxArgs a) {
 // Rows the vector kernel cannot take (a width that is not a multiple of 4, or
 // unaligned pointers), up to 16384 floats: the row in registers as 16-byte
 // vectors at 4-byte addresses, TPR threads per row (a wave up to 1536 floats: no
-// barrier in its reductions; a workgroup above and where the rows are few) -- one read of the row, and the
-// same max / sum / finish as softmax_rows_generic.  Measured on
-// MI355X at 8191 x 1001: 11.4-12.7 us against 19.5 in 4-byte columns, one
+// barrier in its reductions; a workgroup above and where the rows are few) -- one
+// read of the row, and the same max / sum / finish as softmax_rows_generic.
+// Measured on MI355X at 8191 x 1001: 11.4-12.7 us against 19.5 in 4-byte columns, one
 // workgroup per row; 40000 x 1001 57 / 81 us.
 template <int MODE, int TPR, int VPT, bool KEEP>
-__global__ __launch_bounds__(kBlock) void softmax_rows_any(SoftmaxArgs a) {
-    constexpr int RPB = kBlock / TPR, NW = TPR / kWave;
-    __shared__ float lds[2][kBlock / kWave];
+__global__ __launch_bounds__(any_block(TPR)) void softmax_rows_any(SoftmaxArgs a) {
+    constexpr int RPB = any_block(TPR) / TPR, NW = TPR / kWave;
+    __shared__ float lds[2][RPB * NW];
     const int t = threadIdx.x % TPR, sub = threadIdx.x / TPR;
     const int64_t row = static_cast<int64_t>(blockIdx.x) * RPB + sub;
     if constexpr (NW == 1) {
@@ -172,11 +172,12 @@ __global__ __launch_bounds__(kBlock) void softmax_rows_any(SoftmaxArgs a) {
 
 template <int MODE, int TPR, int VPT>
 int launch_any(mimir_ctx* ctx, const SoftmaxArgs& a) {
+    constexpr int kBS = any_block(TPR);
     unsigned grid;
-    if (!grid_for(a.rows, kBlock / TPR, kBlock, &grid))
+    if (!grid_for(a.rows, kBS / TPR, kBS, &grid))
         return fail(ctx, MIMIR_EINVAL, "softmax: %lld rows exceed the grid limit", (long long)a.rows);
-    if (ctx->keep_outputs) softmax_rows_any<MODE, TPR, VPT, true><<<grid, kBlock, 0, ctx->stream>>>(a);
-    else softmax_rows_any<MODE, TPR, VPT, false><<<grid, kBlock, 0, ctx->stream>>>(a);
+    if (ctx->keep_outputs) softmax_rows_any<MODE, TPR, VPT, true><<<grid, kBS, 0, ctx->stream>>>(a);
+    else softmax_rows_any<MODE, TPR, VPT, false><<<grid, kBS, 0, ctx->stream>>>(a);
     return launched(ctx, "softmax_rows_any");
 }
 

@@ -55,7 +55,9 @@ def ln64(x, eps):
 
 CASES = [(rows, cols, 0) for cols in WIDTHS for rows in (1, 5)] + [(131, 1001, 0), (2500, 67, 0), (7, 64, 1), (6, 1024, 3),
                                                                   (3, 4096, 2), (600, 260, 1), (2048, 515, 0), (2049, 515, 0),
-                                                                  (2048, 1535, 0), (2049, 1535, 0), (2049, 1537, 0)]
+                                                                  (2048, 1535, 0), (2049, 1535, 0), (2049, 1537, 0),
+                                                                  (2560, 1001, 0), (2561, 1001, 0), (2561, 1535, 0),
+                                                                  (3072, 1027, 0), (3073, 1535, 0)]
 
 
 @pytest.mark.parametrize("rows,cols,shift", CASES)
