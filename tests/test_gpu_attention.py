@@ -211,9 +211,9 @@ def test_full_size_properties(ctx):
 @pytest.mark.parametrize("seq,e,heads", [(1, 16, 2), (50, 64, 4), (130, 96, 3), (64, 128, 1), (300, 256, 2)])
 @pytest.mark.parametrize("causal", [False, True])
 def test_self_attention_layer(ctx, seq, e, heads, causal):
-    """mimir_self_attention_fwd (projections + fused core) against the
-    compiled reference's self_attention_forward with random weights and
-    float64, under the whole-layer tolerance (tests/_attention.py)."""
+    """mimir_self_attention_fwd (projections + fused core) against float64 and,
+    where it is built, the compiled reference's self_attention_forward, with
+    random weights, under the whole-layer tolerance (tests/_attention.py)."""
     from _attention import assert_within, attention_layer64, layer_case
     x, w = layer_case(seq, e, seq * 7 + e, 1.5)
     wqkv, wout = w[:3 * e * e].reshape(e, 3 * e), w[3 * e * e:].reshape(e, e)
@@ -227,7 +227,8 @@ def test_self_attention_layer(ctx, seq, e, heads, causal):
             d.free()
     want, tol = attention_layer64(x, wqkv, wout, heads, causal)
     assert_within(got, want, tol, "layer vs float64")
-    assert_within(got, O.ref_self_attention(x, wqkv, wout, seq, e, heads, causal), 2 * tol, "layer vs reference")
+    if O.ref_available():
+        assert_within(got, O.ref_self_attention(x, wqkv, wout, seq, e, heads, causal), 2 * tol, "layer vs reference")
 
 
 @pytest.mark.parametrize("lq,lk,e,heads", [(37, 90, 64, 4), (200, 33, 128, 2), (1, 1, 32, 1)])
@@ -249,8 +250,9 @@ def test_cross_attention_layer(ctx, lq, lk, e, heads, causal):
             d.free()
     want, tol = cross_attention_layer64(xq, xkv, wq, wkv, wout, heads, causal)
     assert_within(got, want, tol, "cross layer vs float64")
-    assert_within(got, O.ref_cross_attention(xq, xkv, wq, wkv, wout, lq, lk, e, heads, causal), 2 * tol,
-                  "cross layer vs reference")
+    if O.ref_available():
+        assert_within(got, O.ref_cross_attention(xq, xkv, wq, wkv, wout, lq, lk, e, heads, causal), 2 * tol,
+                      "cross layer vs reference")
 
 
 def test_attention_layer_refusals(ctx):

@@ -100,15 +100,17 @@ def check_core(got, q, k, v, dout, heads, causal, what, oracle=True):
                                  2 * NORM_REL)
 
 
-# (batch, q_len, kv_len, heads, head_dim, causal, amp): the softmax kernels'
-# register forms (kv_len <= 256, <= 1024, <= 4096) and the streamed form
-# (> 4096), self and cross shapes, causal rows past the last key, head_dim
-# above 128.
+# (batch, q_len, kv_len, heads, head_dim, causal, amp): heads up to 128 (the
+# matrix-core kernels) and above (library products, and the softmax kernels'
+# register forms, kv_len <= 256, <= 1024, <= 4096, and streamed form, > 4096),
+# self and cross shapes, causal rows past the last key.
 CORE = [(1, 64, 64, 2, 32, True, 1.0), (1, 64, 64, 2, 32, False, 1.0), (3, 33, 33, 3, 20, True, 1.0),
         (1, 37, 90, 4, 16, False, 1.0), (1, 90, 37, 1, 64, True, 2.0), (1, 128, 128, 1, 128, True, 3.0),
         (1, 300, 300, 2, 48, True, 1.0), (1, 17, 1500, 2, 40, False, 1.0), (1, 5, 5000, 1, 32, True, 1.0),
         (1, 5, 5000, 1, 32, False, 1.0), (1, 1, 1, 1, 8, True, 1.0), (1, 1, 7, 3, 8, False, 1.0),
-        (2, 257, 257, 1, 200, True, 1.0),
+        (2, 257, 257, 1, 200, True, 1.0), (2, 130, 130, 3, 136, False, 1.0), (1, 17, 1500, 2, 136, False, 1.0),
+        (1, 5, 5000, 2, 131, True, 1.0), (1, 5, 5000, 1, 132, False, 1.0), (1, 700, 300, 2, 131, True, 1.0),
+        (1, 300, 700, 2, 140, True, 1.0),
         # longer causal rows and cross shapes with keys past every query
         (1, 600, 600, 2, 32, True, 1.0), (1, 1000, 1000, 1, 64, True, 1.0), (1, 700, 300, 1, 32, True, 1.0),
         (1, 300, 700, 1, 32, True, 1.0), (2, 520, 520, 2, 16, True, 2.0),
@@ -144,13 +146,14 @@ def _tuned_context(tune):
             os.environ["MIMIR_TUNE"] = old
 
 
+@pytest.mark.parametrize("hd", [16, 136])
 @pytest.mark.parametrize("group", [1, 2])
-def test_core_backward_head_groups(group):
+def test_core_backward_head_groups(group, hd):
     """Heads processed in groups (the scratch cap; forced small here through
     the tuning override) give the same gradients as one group."""
     c = _tuned_context(f"attnbwd_heads={group}")
     try:
-        q, k, v, dout = rand_core(12, 2, 50, 60, 5 * 16, 1.0)
+        q, k, v, dout = rand_core(12, 2, 50, 60, 5 * hd, 1.0)
         check_core(gpu_core_bwd(c, q, k, v, dout, 5, True), q, k, v, dout, 5, True, f"groups of {group}")
     finally:
         c.close()
@@ -159,12 +162,12 @@ def test_core_backward_head_groups(group):
 @pytest.mark.parametrize("blocks", [2, 3, 4])
 @pytest.mark.parametrize("lq,lk", [(1000, 1000), (700, 300), (520, 900)])
 def test_core_backward_causal_blocks(blocks, lq, lk):
-    """The causal products over query / key blocks in other counts than the
-    default two (a tuning override): ragged last blocks, cross shapes, and
-    key blocks that no query sees (zeroed)."""
+    """The causal products of wide heads over query / key blocks in other counts
+    than the default two (a tuning override): ragged last blocks, cross shapes,
+    and key blocks that no query sees (zeroed)."""
     c = _tuned_context(f"attnbwd_blocks={blocks}")
     try:
-        q, k, v, dout = rand_core(lq + lk + blocks, 1, lq, lk, 2 * 32, 1.0)
+        q, k, v, dout = rand_core(lq + lk + blocks, 1, lq, lk, 2 * 136, 1.0)
         check_core(gpu_core_bwd(c, q, k, v, dout, 2, True), q, k, v, dout, 2, True, f"{blocks} blocks")
     finally:
         c.close()
@@ -173,15 +176,15 @@ def test_core_backward_causal_blocks(blocks, lq, lk):
 @pytest.mark.parametrize("tune", ["blas=0", "blas=0,attnbwd_blocks=2"])
 @pytest.mark.parametrize("causal", [False, True])
 def test_core_backward_rocblas(tune, causal):
-    """The rocBLAS-only path (MIMIR_TUNE blas=0): K and V transposed for the
+    """The rocBLAS-only path of wide heads (MIMIR_TUNE blas=0): K and V transposed for the
     plain-form score products, dQ / dK / dV written in place, with and
     without causal blocks, and an odd head size."""
     c = _tuned_context(tune)
     try:
-        q, k, v, dout = rand_core(15, 1, 520, 520, 3 * 20, 1.0)
+        q, k, v, dout = rand_core(15, 1, 520, 520, 3 * 132, 1.0)
         check_core(gpu_core_bwd(c, q, k, v, dout, 3, causal), q, k, v, dout, 3, causal, tune)
-        q, k, v, dout = rand_core(16, 1, 260, 260, 2 * 13, 1.0)
-        check_core(gpu_core_bwd(c, q, k, v, dout, 2, causal), q, k, v, dout, 2, causal, tune + ", head size 13")
+        q, k, v, dout = rand_core(16, 1, 260, 260, 2 * 131, 1.0)
+        check_core(gpu_core_bwd(c, q, k, v, dout, 2, causal), q, k, v, dout, 2, causal, tune + ", head size 131")
     finally:
         c.close()
 

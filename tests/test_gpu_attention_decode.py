@@ -7,6 +7,7 @@ import pytest
 import oracle as O
 from _attention import assert_attention_close, attention64
 from test_gpu_attention import gpu_attention, rand_qkv
+from test_gpu_attention_bwd import _tuned_context
 
 pytestmark = pytest.mark.gpu
 
@@ -24,6 +25,21 @@ def test_decode(ctx, b, lq, lk, heads, hd):
     for i in range(b):
         out, mag, cond = attention64(q[i], k[i], v[i], heads, False, O.attention_scale(hd))
         assert_attention_close(got[i], out, mag, cond, f"decode {b} {lq} {lk} {heads} {hd} [{i}]")
+
+
+@pytest.mark.parametrize("splits", [1, 5, 64])
+def test_decode_splits(splits):
+    """Keys over a set number of workgroups, among them fewer keys than 64 each."""
+    c = _tuned_context(f"decode={splits}")
+    try:
+        for lq, lk, hd in ((1, 1000, 64), (3, 130, 100), (8, 61, 33)):
+            q, k, v = rand_qkv(lk, 2, lq, lk, 2 * hd)
+            got = gpu_attention(c, q, k, v, 2, False)
+            for i in range(2):
+                out, mag, cond = attention64(q[i], k[i], v[i], 2, False, O.attention_scale(hd))
+                assert_attention_close(got[i], out, mag, cond, f"decode splits {splits} {lq} {lk} {hd} [{i}]")
+    finally:
+        c.close()
 
 
 @pytest.mark.parametrize("lk", [40, 700])

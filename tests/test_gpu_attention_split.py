@@ -12,6 +12,7 @@ import mimir_hip as M
 import oracle as O
 from _attention import assert_attention_close, attention64
 from test_gpu_attention import gpu_attention, rand_qkv
+from test_gpu_attention_bwd import _tuned_context
 
 pytestmark = pytest.mark.gpu
 
@@ -78,6 +79,37 @@ def check_special_values(ctx, lq, lk, causal, low, inf_row, big_row, nan_key):
 @pytest.mark.parametrize("causal", [False, True])
 def test_split_core_special_values_over_key_splits(ctx, lq, lk, causal, rows):
     check_special_values(ctx, lq, lk, causal, *rows)
+
+
+# Keys over several workgroups: what splits_for chooses (737 keys and more, few
+# workgroups), and counts and workgroup sizes set by MIMIR_TUNE, among them more
+# splits than a causal block has tiles.
+@pytest.mark.parametrize("tune", ["", "attnsplits=3", "attnsplits=7,attnwaves=4", "attnsplits=40,attnwaves=8"])
+@pytest.mark.parametrize("b,lq,lk,heads,hd", [(1, 1000, 1000, 1, 128), (1, 40, 1500, 2, 80), (2, 130, 900, 1, 5),
+                                               (1, 300, 737, 3, 64)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_split_core_over_key_splits(tune, b, lq, lk, heads, hd, causal):
+    q, k, v = rand_qkv(lq + lk + hd, b, lq, lk, heads * hd)
+    c = _tuned_context(tune)
+    try:
+        got = gpu_attention(c, q, k, v, heads, causal)
+    finally:
+        c.close()
+    for i in range(b):
+        out, mag, cond = attention64(q[i], k[i], v[i], heads, causal, O.attention_scale(hd))
+        assert_attention_close(got[i], out, mag, cond, f"key splits {tune} {b} {lq} {lk} {heads} {hd} {causal} [{i}]")
+
+
+@pytest.mark.parametrize("waves", [4, 8])
+def test_split_core_workgroup_sizes(waves):
+    c = _tuned_context(f"attnwaves={waves}")
+    try:
+        for lq, lk, hd, causal in ((40, 70, 32, False), (260, 260, 96, True), (513, 100, 64, True)):
+            q, k, v = rand_qkv(lq + hd, 1, lq, lk, 2 * hd)
+            out, mag, cond = attention64(q[0], k[0], v[0], 2, causal, O.attention_scale(hd))
+            assert_attention_close(gpu_attention(c, q, k, v, 2, causal)[0], out, mag, cond, f"{waves} waves {lq} {lk} {hd}")
+    finally:
+        c.close()
 
 
 def call_us(ctx, run, reps):

@@ -673,7 +673,8 @@ def test_output_caching_gives_the_same_bits(ctx):
 @pytest.mark.parametrize("cols", [1023, 2047, 4095])
 def test_odd_widths_register_resident(ctx, cols):
     """Widths that are not a multiple of 4 (rows start off 16-byte alignment)
-    take the 4-byte-column kernels (norm_rows_scalar, softmax_rows_scalar):
+    take the kernels with vectors at 4-byte addresses (norm_rows_any,
+    softmax_rows_any):
     LayerNorm, RMSNorm with a weight block shorter than the row, add + RMSNorm
     with the residual updated in place (bit-exact), and softmax
     with a masked column, an all -inf row (NaN, as the reference) and a NaN
