@@ -652,12 +652,18 @@ int64_t group_of(const mimir_ctx* ctx, const CoreBwd& c) {
 // until the workgroups fill the GPU, four tiles each at least.  The target of
 // 512 against 256 / 1024 (us): 16 heads x 2048 x 64 causal 304 / 349 / 330, 16 x
 // 1024 x 128 218 / 210 / 267 (unsplit 364), 64 x 512 x 64 120 / 116 / 143.
-int64_t splits_of(int64_t blocks, int64_t steps) {
-    constexpr int64_t kTarget = 512;
-    return std::max<int64_t>(1, std::min<int64_t>(kTarget / blocks, steps / 4));
+int64_t splits_of(int64_t blocks, int64_t steps, int64_t target = 512) {
+    return std::max<int64_t>(1, std::min<int64_t>(target / blocks, steps / 4));
 }
 int64_t kv_splits(const CoreBwd& c, int64_t n_bh) { return splits_of(n_bh * key_blocks(c), tiles(c.q_len)); }
 int64_t q_splits(const CoreBwd& c, int64_t n_bh) { return splits_of(n_bh * query_blocks(c), tiles(c.kv_len)); }
+// The statistics' workgroups run one to a CU: 256 fill it, and only a causal call's
+// uneven blocks gain from more.  256 / 512, whole backward, us: 16 x 4 heads x 40 x 1500
+// x 64 91 / 98, 8 x 16 x 512 x 512 x 128 390 / 408; causal, 2 x 16 x 2048 x 128 823 / 761,
+// 4 x 12 x 700 x 80 195 / 182, 4 x 16 x 512 x 128 200 / 211.
+int64_t stats_splits(const CoreBwd& c, int64_t n_bh) {
+    return splits_of(n_bh * query_blocks(c), tiles(c.kv_len), c.causal ? 512 : 256);
+}
 // Floats of one partial result (rounded so that the next is 16-byte aligned).
 int64_t part_floats(int64_t splits, int64_t n_bh, int64_t rows, int64_t head_dim) {
     return splits > 1 ? (splits * n_bh * rows * head_dim + 3) / 4 * 4 : 0;
@@ -666,8 +672,9 @@ int64_t ds_floats(const CoreBwd& c, int64_t n_bh) { return n_bh * tiles(c.q_len)
 int64_t stats_floats(const CoreBwd& c, int64_t n_bh) { return 3 * n_bh * tiles(c.q_len) * kTileRows; }
 int64_t parts_floats(const CoreBwd& c, int64_t n_bh) {
     // The statistics' partial results are gone before the others are written.
-    const int64_t s = q_splits(c, n_bh);
-    return std::max(2 * part_floats(kv_splits(c, n_bh), n_bh, c.kv_len, c.head_dim) + part_floats(s, n_bh, c.q_len, c.head_dim),
+    const int64_t s = stats_splits(c, n_bh);
+    return std::max(2 * part_floats(kv_splits(c, n_bh), n_bh, c.kv_len, c.head_dim) +
+                        part_floats(q_splits(c, n_bh), n_bh, c.q_len, c.head_dim),
                     s > 1 ? s * stats_floats(c, n_bh) : 0);
 }
 
@@ -714,7 +721,7 @@ int attention_bwd_mfma(mimir_ctx* ctx, const CoreBwd& c, float* work) {
         float* const parts = a.stats + stats_floats(c, group);
         a.splits = static_cast<int32_t>(kv_splits(c, a.n_bh));
         a.q_splits = static_cast<int32_t>(q_splits(c, a.n_bh));
-        a.stats_splits = a.q_splits;
+        a.stats_splits = static_cast<int32_t>(stats_splits(c, a.n_bh));
         a.stats_part = a.stats_splits > 1 ? parts : nullptr;
         const int64_t one = part_floats(a.splits, a.n_bh, c.kv_len, c.head_dim);
         a.part[0] = a.splits > 1 ? parts : nullptr;
