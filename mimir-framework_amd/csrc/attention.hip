@@ -46,9 +46,9 @@
 // Bound by the power the matrix cores draw: at 8 x 32 heads x 1024 tokens x 128,
 // causal, the bf16 MFMAs hold the matrix pipes 51% of the cycles at 1.9 GHz (a
 // loop of nothing else runs at 1.6 GHz), beside 350 VALU operations per 96
-// MFMAs.  Measured there 400 us = 172 TFLOP/s of fp32 work, against 627 us on
-// the fp32 MFMAs (157 TFLOP/s peak); 16 heads x 1024 x 128 99 / 152 us, 96 heads
-// x 333 x 777 x 80 77 / 213 us.  Within noise of that: two accumulators in
+// MFMAs.  Measured there 404 to 413 us = 167 to 170 TFLOP/s of fp32 work, against
+// 627 us on the fp32 MFMAs (157 TFLOP/s peak); 16 heads x 1024 x 128 70 / 152 us, 96
+// heads x 333 x 777 x 80 80 / 213 us.  Within noise of that: two accumulators in
 // turns, LDS reads ordered ahead of the MFMAs, the split interleaved with them,
 // raised priority for half the waves; four waves with two workgroups' worth of
 // LDS are slower (the tile is split twice as often).
@@ -100,7 +100,8 @@ __device__ __forceinline__ int tiles_of(const AttnArgs& a, int q0, int n) {
     return (end + kKeyTile - 1) / kKeyTile;
 }
 
-// Workgroup -> (sequence * heads + head, query block): see the file comment.
+// Workgroup (without its split) -> (sequence * heads + head, query block): see the
+// file comment; the XCDs own whole (sequence, head) pairs where keys are not split.
 __device__ __forceinline__ void block_coords(const AttnArgs& a, uint32_t bid, uint32_t* bh, int* qb) {
     const uint32_t n_bh = a.total_blocks / static_cast<uint32_t>(a.n_qblocks);
     uint32_t first = 0, owned = n_bh, idx = bid;

@@ -30,12 +30,14 @@
 // whose blocks fit kDsBytes), written and read once.
 //
 // Bound by latency and the barriers as much as by the matrix cores: at 8 x 32
-// heads x 1024 x 128, causal, step 2 takes 925 us with the matrix pipes busy
-// 45% of the cycles (1020 us with its tile in one buffer and three barriers),
-// step 1 445 us, step 3 235 us: 1.53 ms = 112 TFLOP/s of the
-// five products, against 3.30 ms for the same products as library fp32 GEMMs
-// with P and dS in memory; 64 heads x 512 x 64 120 / 964 us, 128 heads x 100 x 64
-// 42 / 1059 us (the GEMMs ran sequence by sequence).
+// heads x 1024 x 128, causal, 1640 to 1680 us = 102 to 105 TFLOP/s of the five
+// products counted (seven are run: S and dP in steps 1 and 2, then dV, dK and dQ).
+// The kernels alone, traced: step 1 450 us, step 2 950 us with the matrix pipes
+// busy 45% of the cycles (10% more with its tile in one buffer and three
+// barriers), step 3 250 us.  Step 1 as the forward with out . dout took as long.
+// 3.30 ms for the same products as library fp32 GEMMs with P and dS in memory; 4 x
+// 16 heads x 512 x 128 causal 202 us, 96 x 333 x 777 x 80 273 us, against 1.2 ms (the
+// GEMMs ran sequence by sequence).
 //
 // LDS of step 2: Q rows, dO rows, Q^T and dO^T of one tile in bf16 planes
 // (114 KB at 128 dimensions), the pairs' P (16 KB) and the tile's max / sum /
@@ -86,8 +88,9 @@ struct BwdArgs {
     float* part[3];            // dV, dK, dQ
 };
 
-// Workgroup -> (sequence, head) and its block, the longest first; each XCD
-// keeps whole (sequence, head) pairs where they divide by the XCDs.
+// Workgroup (without its split) -> (sequence, head) and its block, the longest
+// first; unsplit, each XCD keeps whole (sequence, head) pairs where they divide by
+// the XCDs.
 __device__ __forceinline__ void coords(const BwdArgs& a, uint32_t bid, uint32_t* bh, uint32_t* block) {
     uint32_t first = 0, owned = a.n_bh, idx = bid;
     if (a.n_bh % kXcds == 0) {

@@ -67,7 +67,8 @@ struct Tuning {
     int attn_waves = 0;       // attention forward: waves per workgroup (4, 8; 0: measured default)
     int attn_splits = 0;      // attention forward: splits of the keys (0: measured default)
     int decode_splits = 0;    // attention_decode: workgroups per (sequence, head) (0: measured default)
-    int attn_bwd_heads = 0;   // heads per group of the attention backward (0: what 1 GiB of P / dS holds)
+    int attn_bwd_heads = 0;   // attention backward: (sequence, head) pairs per group (0: what 512 MiB of dS, or, heads
+                              // over 128, 1 GiB of P and dS hold)
     int attn_bwd_blocks = 0;  // causal attention backward: query / key blocks of the products (0: default)
     int embed_bwd_sort = -1;    // embedding backward: counting sort where it applies (-1, 1) or rocPRIM's (0)
     int embed_bwd_runs = -1;    // embedding backward: rows kernel over the counting sort's run list (-1, 1) or

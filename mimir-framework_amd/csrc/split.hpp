@@ -1,5 +1,9 @@
 // split.hpp -- fp32 products on the bf16 matrix cores.
 //
+// After Henry, Tang and Heinecke, "Leveraging the bfloat16 Artificial Intelligence
+// Datatype For Higher-Precision Computations" (ARITH 2019), which describes the
+// three-term split and how many of its nine products to take.
+//
 // gfx950 multiplies fp32 operands at 157 TFLOP/s dense and bf16 operands at
 // 16 times that.  An fp32 value is the exact sum of three bf16 values
 // x = h + m + l (each the round-to-nearest bf16 of what the ones before it
@@ -13,14 +17,18 @@
 // float64, relative error of dot products of N(0,1) values, this form / the
 // fp32 MFMA chain: length 32 0.69e-7 / 1.03e-7, 128 1.6e-7 / 2.0e-7, 1024
 // 4.9e-7 / 5.7e-7.  The builtin rounds to nearest even and keeps subnormal
-// inputs and results (checked on the same GPU).
+// inputs and results (checked on the same GPU).  Contractions of one or two terms
+// have nothing to gain there: a single product is up to 8.7e-8 off, one fp32
+// rounding 5.9e-8 (gemm_split.hip leaves fewer than four terms to the library;
+// the attention core's results are no further off down to heads of 1, where the
+// errors of the weights are larger).
 //
 // A value that is infinite, NaN, or so near the largest float that its bf16
 // rounds to infinity has no such split: its residues are NaN, so every
 // result it reaches is NaN.  The kernels redo the results that come out NaN
 // with fp32 products, which gives them the values (infinite, NaN or finite)
 // that fp32 arithmetic gives.  Values below 2^-110 lose their last bits to
-// bf16's smallest subnormal, 2^-133.
+// bf16's smallest subnormal, 2^-133 (mimir_hip.h says so).
 #pragma once
 
 #include "common.hpp"
