@@ -549,7 +549,7 @@ int mimir_self_attention_bwd(mimir_ctx* ctx, const float* input, const float* gr
     a.dq = dqkv;
     a.dk = dqkv + e;
     a.dv = dqkv + 2 * e;
-    a.att = att;
+    a.att = grad_weights ? att : nullptr;  // dWout alone reads it
     if (int st = gemm_f32(ctx, T, 3 * e, e, input, e, wqkv, 3 * e, qkv, 3 * e)) return st;  // :6868-6880
     if (int st = gemm_f32_ex(ctx, false, true, T, e, e, 1.0f, grad_out, e, 0, wout, e, 0, 0.0f, datt, e, 0, 1))
         return st;  // :6935-6947
@@ -609,7 +609,7 @@ int mimir_cross_attention_bwd(mimir_ctx* ctx, const float* query_input, int64_t 
     a.dq = dqp;
     a.dk = dkv;
     a.dv = dkv + e;
-    a.att = att;
+    a.att = grad_weights ? att : nullptr;  // dWout alone reads it
     if (int st = gemm_f32(ctx, Tq, e, e, query_input, e, wq, e, qp, e)) return st;           // :7095-7105
     if (int st = gemm_f32(ctx, Tk, 2 * e, e, kv_input, e, wkv, 2 * e, kv, 2 * e)) return st;  // :7106-7116
     if (int st = gemm_f32_ex(ctx, false, true, Tq, e, e, 1.0f, grad_out, e, 0, wout, e, 0, 0.0f, datt, e, 0, 1))
