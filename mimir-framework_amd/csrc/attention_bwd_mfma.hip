@@ -13,7 +13,8 @@
 //    has all the weight, dP - delta cancels to what the other keys leave, and to 0
 //    where there is no other.  (out . dout, from the forward's output, is the
 //    same number with another rounding: it left 1e-7 of dP there, up to a
-//    hundred times dQ itself.)
+//    hundred times dQ itself.)  A layer's output comes from it too, or, heads over
+//    kOutDim, from the forward.
 // 2. attention_bwd_kv: a workgroup owns 128 keys and streams tiles of 32
 //    queries.  Its eight waves are four pairs, a pair for 32 keys: one wave
 //    holds the K rows and computes S, then P, then dV += dO P; the other holds
@@ -61,6 +62,11 @@ constexpr int kKeysPerBlock = 128;
 constexpr int kXcds = 8;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kBlockFloats = kTileRows * kTileRows;
+// Heads up to this have their output from attention_bwd_stats too, where a layer
+// wants it; at 96 dimensions a hundred registers would spill.  Layer backward, us (the
+// forward beside the statistics / this): 2048 tokens, 16 heads of 64 713 / 624, 300 tokens,
+// 8 heads of 64 115 / 103, 777 tokens, 8 heads of 32 107 / 93.
+constexpr int kOutDim = 64;
 
 struct BwdArgs {
     CoreBwd c;
@@ -74,7 +80,8 @@ struct BwdArgs {
     float* stats;
     int64_t stats_ld;
     // The keys of attention_bwd_stats dealt to several workgroups: max, sum and
-    // sum_j e_j dp_j of each, [split][3][n_bh][stats_ld]; null: one workgroup.
+    // sum_j e_j dp_j of each, [split][3][n_bh][stats_ld]; null: one workgroup.  Then,
+    // where the output is wanted (c.att), sum_j e_j v_j, [split][n_bh][q_len][head_dim].
     float* stats_part;
     int32_t stats_splits;
     float* ds;                 // [n_bh][key tile][query tile][32 keys][32 queries]
@@ -113,8 +120,9 @@ __device__ __forceinline__ float weight(const BwdArgs& a, float product, float m
 // the sums.
 struct RowStats {
     float m, l, d;
-    // One tile: products s and dP, of which the first `lim` of the lane's half count.
-    __device__ __forceinline__ void add(const BwdArgs& a, const f16v& s, const f16v& dp, int lim) {
+    // One tile: products s, which become weights, and dP, of which the first `lim` of
+    // the lane's half count.  Returns what earlier weights are scaled by.
+    __device__ __forceinline__ float add(const BwdArgs& a, f16v& s, const f16v& dp, int lim) {
         f16v x;
 #pragma unroll
         for (int r = 0; r < 16; ++r) x[r] = 8 * (r / 4) + r % 4 < lim ? s[r] * a.sign : -INFINITY;
@@ -128,23 +136,28 @@ struct RowStats {
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const bool sees = 8 * (r / 4) + r % 4 < lim;
-            const float e = weight(a, s[r], top);
-            sum += sees ? e : 0.f;
-            dot += sees ? e * dp[r] : 0.f;
+            s[r] = sees ? weight(a, s[r], top) : 0.f;
+            sum += s[r];
+            dot += sees ? s[r] * dp[r] : 0.f;
         }
         l = l * alpha + sum;
         d = d * alpha + dot;
+        return alpha;
     }
 };
 
 // Step 1: a wave for 32 queries (their rows of Q and dO in registers), streaming 32
 // keys and values.  The scores come out as S^T = K Q^T, dP as V dO^T, the products
-// of step 2 transposed.
-template <int DP, bool VEC>
+// of step 2 transposed.  OUT: and the output, out += V P^T as in attention.hip, from
+// the same weights; heads up to kOutDim, above which the registers do not hold it
+// (the forward runs beside this kernel there).
+template <int DP, bool VEC, bool OUT>
 __global__ __launch_bounds__(kThreads, 2) void attention_bwd_stats(BwdArgs a) {
     using Rows = RowTile<DP, kThreads, VEC>;
-    constexpr int kC = DP / 16;
-    __shared__ __attribute__((aligned(16))) char lds[4 * Rows::kBytes];  // K and V rows of two tiles
+    using Cols = ColTile<DP, kThreads>;
+    constexpr int kC = DP / 16, kDb = DP / 32;
+    constexpr int kBuf = 2 * Rows::kBytes + (OUT ? Cols::kBytes : 0);  // K and V rows of a tile, V^T
+    __shared__ __attribute__((aligned(16))) char lds[2 * kBuf];
 
     uint32_t bh, qblock;
     const int split = static_cast<int>(blockIdx.x % static_cast<uint32_t>(a.stats_splits));
@@ -170,11 +183,19 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_stats(BwdArgs a) {
     const float* dout = a.c.dout + (b * a.q_len + row) * a.c.ld_dout + hd;
 
     Rows keys, values;
+    Cols cols;
     keys.init(a.c.ld_kv, a.head_dim);
     values.init(a.c.ld_kv, a.head_dim);
+    if constexpr (OUT) cols.init(a.c.ld_kv, a.head_dim);
     auto load = [&](int t) {
         keys.load(k, t, a.c.ld_kv, a.kv_len, a.head_dim);
         values.load(v, t, a.c.ld_kv, a.kv_len, a.head_dim);
+        if constexpr (OUT) cols.load(v, t, a.c.ld_kv, a.kv_len, a.head_dim);
+    };
+    auto stash = [&](char* to) {
+        keys.stash(to);
+        values.stash(to + Rows::kBytes);
+        if constexpr (OUT) cols.stash(to + 2 * Rows::kBytes);
     };
     if (t0 < n_tiles) load(t0);
     Split8 qx[kC], ox[kC];
@@ -184,19 +205,22 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_stats(BwdArgs a) {
     // the max starts at -1e30 (LayerOps.hpp:1052).
     const RowStats none{fmaxf((end < a.kv_len ? -1e9f : -1e30f) * kLog2e / a.qscale, -FLT_MAX), 0.f, 0.f};
     RowStats st = none;
-    auto add = [&](RowStats& to, const f16v& s, const f16v& dp, int t) {
-        if ((t + 1) * kTileRows > a.kv_len || (a.c.causal && t == qt)) to.add(a, s, dp, end - t * kTileRows - 4 * hf);
-        else to.add(a, s, dp, kTileRows);
+    auto add = [&](RowStats& to, f16v& s, const f16v& dp, int t) {
+        if ((t + 1) * kTileRows > a.kv_len || (a.c.causal && t == qt))
+            return to.add(a, s, dp, end - t * kTileRows - 4 * hf);
+        return to.add(a, s, dp, kTileRows);
     };
+    f16v o[OUT ? kDb : 1];
+#pragma unroll
+    for (int d = 0; d < (OUT ? kDb : 1); ++d) o[d] = f16v{};
     if (t0 < n_tiles) {
-        keys.stash(lds);
-        values.stash(lds + Rows::kBytes);
+        stash(lds);
         load(min(t0 + 1, n_tiles - 1));
     }
     __syncthreads();
     for (int t = t0; t < n_tiles; ++t) {
-        const char* cur = lds + ((t - t0) & 1) * 2 * Rows::kBytes;
-        char* const next = lds + ((t - t0 + 1) & 1) * 2 * Rows::kBytes;
+        const char* cur = lds + ((t - t0) & 1) * kBuf;
+        char* const next = lds + ((t - t0 + 1) & 1) * kBuf;
         f16v s = f16v{}, dp = f16v{};
         if (t < wave_tiles) {
 #pragma unroll
@@ -204,13 +228,27 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_stats(BwdArgs a) {
         }
         // Past the last tile the stash rewrites a buffer that is not read again,
         // and the load repeats the last tile.
-        keys.stash(next);
-        values.stash(next + Rows::kBytes);
+        stash(next);
         load(min(t + 2, n_tiles - 1));
         if (t < wave_tiles) {
 #pragma unroll
             for (int c = 0; c < kC; ++c) dp = mfma_split_mirror(Rows::at(cur + Rows::kBytes, li, hf, c), ox[c], dp);
-            add(st, s, dp, t);
+            const float alpha = add(st, s, dp, t);
+            if constexpr (OUT) {
+                if (__any(alpha != 1.f)) {
+#pragma unroll
+                    for (int d = 0; d < kDb; ++d) o[d] *= alpha;
+                }
+#pragma unroll
+                for (int c = 0; c < 2; ++c) {
+                    float x[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) x[e] = s[8 * c + e];
+                    const Split8 p = split8(x);
+#pragma unroll
+                    for (int d = 0; d < kDb; ++d) o[d] = mfma_split(Cols::at(cur + 2 * Rows::kBytes, li, hf, d, c), p, o[d]);
+                }
+            }
         }
         __syncthreads();
     }
@@ -221,7 +259,7 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_stats(BwdArgs a) {
         RowStats redo = none;
 #pragma unroll 1
         for (int t = t0; t < wave_tiles; ++t) {
-            const f16v s = f32_scores(k, a.c.ld_kv, t * kTileRows, a.kv_len, a.head_dim, q, 1.0f);
+            f16v s = f32_scores(k, a.c.ld_kv, t * kTileRows, a.kv_len, a.head_dim, q, 1.0f);
             const f16v dp = f32_scores(v, a.c.ld_kv, t * kTileRows, a.kv_len, a.head_dim, dout, 1.0f);
             add(redo, s, dp, t);
         }
@@ -229,9 +267,31 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_stats(BwdArgs a) {
     }
     st.l += __shfl_xor(st.l, 32);
     st.d += __shfl_xor(st.d, 32);
-    if (hf || my_q >= a.stats_ld) return;
     const int64_t plane = a.n_bh * a.stats_ld;
     const float inv = 1.0f / (st.l + 1e-9f);
+    if constexpr (OUT) {
+        float* to = a.stats_part ? a.stats_part + 3 * a.stats_splits * plane + ((split * int64_t{a.n_bh} + bh) * a.q_len + row) * a.head_dim
+                                 : a.c.att + (b * a.q_len + row) * a.c.ld_att + hd;
+        const float scale = a.stats_part ? 1.0f : inv;
+        const float check = store_columns<DP, VEC>(o, scale, to, in, hf, a.head_dim);
+        // Not finite: with the final max, in fp32.
+        if (const uint32_t bad = bad_rows(check, in)) {
+#pragma unroll 1
+            for (int d0 = 0; d0 < a.head_dim; d0 += 32) {
+                f16v x = f16v{};
+#pragma unroll 1
+                for (int t = t0; t < wave_tiles; ++t) {
+                    f16v s = f32_scores(k, a.c.ld_kv, t * kTileRows, a.kv_len, a.head_dim, q, 1.0f);
+#pragma unroll
+                    for (int r = 0; r < 16; ++r)
+                        s[r] = t * kTileRows + 8 * (r / 4) + 4 * hf + r % 4 < end ? weight(a, s[r], st.m) : 0.f;
+                    f32_accumulate<1>(v + d0, a.c.ld_kv, t * kTileRows, a.kv_len, a.head_dim - d0, s, 0, end, &x);
+                }
+                store_columns<32, VEC>(&x, scale, to + d0, in && (bad >> li & 1), hf, a.head_dim - d0);
+            }
+        }
+    }
+    if (hf || my_q >= a.stats_ld) return;
     float* out = a.stats + bh * a.stats_ld + my_q;
     if (a.stats_part) out = a.stats_part + (split * 3ll * a.n_bh + bh) * a.stats_ld + my_q;
     // Rows past the sequence, up to the tile's end: no weight.
@@ -240,23 +300,42 @@ __global__ __launch_bounds__(kThreads, 2) void attention_bwd_stats(BwdArgs a) {
     out[2 * plane] = in ? (a.stats_part ? st.d : st.d * inv) : 0.f;
 }
 
-// The splits' results of one query each, brought to one max.
+// The splits' results of one query each, brought to one max; W floats of the
+// output a thread (0: none is wanted).
+template <int W>
 __global__ __launch_bounds__(256) void attention_bwd_stats_sum(BwdArgs a) {
-    const int64_t plane = a.n_bh * a.stats_ld, at = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const int64_t plane = a.n_bh * a.stats_ld, id = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+    const int per = W ? a.head_dim / W : 1;
+    const int64_t at = id / per;
     if (at >= plane) return;
     const float* p = a.stats_part + at;
     float m = p[0], l = 0.f, d = 0.f;
     for (int s = 1; s < a.stats_splits; ++s) m = fmaxf(m, p[3 * s * plane]);
-    for (int s = 0; s < a.stats_splits; ++s, p += 3 * plane) {
-        const float f = __builtin_amdgcn_exp2f((p[0] - m) * a.qscale);
-        l += p[plane] * f;
-        d += p[2 * plane] * f;
+    for (int s = 0; s < a.stats_splits; ++s) {
+        const float f = __builtin_amdgcn_exp2f((p[3 * s * plane] - m) * a.qscale);
+        l += p[(3 * s + 1) * plane] * f;
+        d += p[(3 * s + 2) * plane] * f;
     }
-    const bool in = at % a.stats_ld < a.q_len;
+    const int64_t bh = at / a.stats_ld, i = at % a.stats_ld;
+    const bool in = i < a.q_len;
     const float inv = 1.0f / (l + 1e-9f);
-    a.stats[at] = in ? m : 0.f;
-    a.stats[plane + at] = in ? inv : 0.f;
-    a.stats[2 * plane + at] = in ? d * inv : 0.f;
+    const int col = static_cast<int>(id % per) * W;
+    if (col == 0) {
+        a.stats[at] = in ? m : 0.f;
+        a.stats[plane + at] = in ? inv : 0.f;
+        a.stats[2 * plane + at] = in ? d * inv : 0.f;
+    }
+    if constexpr (W > 0) {
+        if (!in) return;
+        const int64_t head = a.bh0 + bh, next = a.n_bh * int64_t{a.q_len} * a.head_dim;
+        const float* x = a.stats_part + 3 * a.stats_splits * plane + (bh * a.q_len + i) * a.head_dim + col;
+        float* to = a.c.att + (head / a.heads * a.q_len + i) * a.c.ld_att + head % a.heads * a.head_dim + col;
+        typedef float fw __attribute__((ext_vector_type(W)));
+        fw sum = fw(0.f);
+        for (int s = 0; s < a.stats_splits; ++s)
+            sum += *reinterpret_cast<const fw*>(x + s * next) * __builtin_amdgcn_exp2f((p[3 * s * plane] - m) * a.qscale);
+        *reinterpret_cast<fw*>(to) = sum * inv;
+    }
 }
 
 // The gradient of a wave's 32 keys on the fp32 matrix cores (attention_tile.hpp),
@@ -609,13 +688,26 @@ template <int DP>
 int launch(mimir_ctx* ctx, BwdArgs a, bool vec) {
     a.blocks = static_cast<uint32_t>(query_blocks(a.c));
     const int64_t w = static_cast<int64_t>(a.n_bh) * a.blocks * a.stats_splits;
-    const int64_t rows_blocks = (a.n_bh * a.stats_ld + 255) / 256;
-    MIMIR_REQUIRE(ctx, dispatch_fits(w, kThreads) && dispatch_fits(rows_blocks, 256), "attention backward: grid too large");
-    if (vec) attention_bwd_stats<DP, true><<<static_cast<unsigned>(w), kThreads, 0, ctx->stream>>>(a);
-    else attention_bwd_stats<DP, false><<<static_cast<unsigned>(w), kThreads, 0, ctx->stream>>>(a);
+    const int per = !a.c.att ? 1 : vec ? a.head_dim / 4 : a.head_dim;  // threads a query in the sum
+    const int64_t sums = (a.n_bh * a.stats_ld * per + 255) / 256;
+    MIMIR_REQUIRE(ctx, dispatch_fits(w, kThreads) && dispatch_fits(sums, 256), "attention backward: grid too large");
+    const auto wgs = static_cast<unsigned>(w);
+    if (a.c.att) {
+        if constexpr (DP <= kOutDim) {
+            if (vec) attention_bwd_stats<DP, true, true><<<wgs, kThreads, 0, ctx->stream>>>(a);
+            else attention_bwd_stats<DP, false, true><<<wgs, kThreads, 0, ctx->stream>>>(a);
+        }
+    } else if (vec) {
+        attention_bwd_stats<DP, true, false><<<wgs, kThreads, 0, ctx->stream>>>(a);
+    } else {
+        attention_bwd_stats<DP, false, false><<<wgs, kThreads, 0, ctx->stream>>>(a);
+    }
     if (int st = launched(ctx, "attention_bwd_stats")) return st;
     if (a.stats_part) {
-        attention_bwd_stats_sum<<<static_cast<unsigned>(rows_blocks), 256, 0, ctx->stream>>>(a);
+        const auto blocks = static_cast<unsigned>(sums);
+        if (!a.c.att) attention_bwd_stats_sum<0><<<blocks, 256, 0, ctx->stream>>>(a);
+        else if (vec) attention_bwd_stats_sum<4><<<blocks, 256, 0, ctx->stream>>>(a);
+        else attention_bwd_stats_sum<1><<<blocks, 256, 0, ctx->stream>>>(a);
         if (int st = launched(ctx, "attention_bwd_stats_sum")) return st;
     }
     a.blocks = static_cast<uint32_t>(key_blocks(a.c));
@@ -678,7 +770,7 @@ int64_t parts_floats(const CoreBwd& c, int64_t n_bh) {
     const int64_t s = stats_splits(c, n_bh);
     return std::max(2 * part_floats(kv_splits(c, n_bh), n_bh, c.kv_len, c.head_dim) +
                         part_floats(q_splits(c, n_bh), n_bh, c.q_len, c.head_dim),
-                    s > 1 ? s * stats_floats(c, n_bh) : 0);
+                    s > 1 ? s * (stats_floats(c, n_bh) + (c.head_dim <= kOutDim ? n_bh * c.q_len * c.head_dim : 0)) : 0);
 }
 
 }  // namespace
@@ -700,13 +792,16 @@ int attention_bwd_mfma(mimir_ctx* ctx, const CoreBwd& c, float* work) {
     const int64_t stats_ld = tiles(c.q_len) * kTileRows;
     auto vec4 = [](const float* p, int64_t ld) { return ld % 4 == 0 && aligned16(p); };
     const bool vec = c.head_dim % 4 == 0 && vec4(c.q, c.ld_q) && vec4(c.k, c.ld_kv) && vec4(c.v, c.ld_kv) &&
-                     vec4(c.dout, c.ld_dout) && vec4(c.dq, c.ld_dq) && vec4(c.dk, c.ld_dkv) && vec4(c.dv, c.ld_dkv);
-    if (c.att)
+                     vec4(c.dout, c.ld_dout) && vec4(c.dq, c.ld_dq) && vec4(c.dk, c.ld_dkv) && vec4(c.dv, c.ld_dkv) &&
+                     (!c.att || vec4(c.att, c.ld_att));
+    BwdArgs a{};
+    a.c = c;
+    if (c.att && c.head_dim > kOutDim) {
         if (int st = mimir_attention_fwd(ctx, c.q, c.ld_q, c.k, c.v, c.ld_kv, c.att, c.ld_att, c.batch, c.q_len, c.kv_len,
                                          c.heads, c.head_dim, c.scale, c.causal))
             return st;
-    BwdArgs a{};
-    a.c = c;
+        a.c.att = nullptr;
+    }
     a.q_len = static_cast<int32_t>(c.q_len);
     a.kv_len = static_cast<int32_t>(c.kv_len);
     a.heads = static_cast<int32_t>(c.heads);

@@ -5,8 +5,8 @@ import numpy as np
 import pytest
 
 import oracle as O
-from _attention import assert_bwd_close, attention_bwd64
-from test_gpu_attention_bwd import _tuned_context, check_core, gpu_core_bwd, rand_core
+from _attention import assert_bwd_close, attention_bwd64, layer_case, self_attention_bwd64
+from test_gpu_attention_bwd import _dev, _tuned_context, check_core, gpu_core_bwd, rand_core
 
 pytestmark = pytest.mark.gpu
 
@@ -147,3 +147,58 @@ def test_split_backward_large_scores(ctx, causal, scale):
         e = np.linalg.norm(g[0] - w) / np.linalg.norm(w)
         print(f"  {name} {e:.3g}", flush=True)
         assert e <= 2 * rel, name
+
+
+def layer_bwd(ctx, x, w, dy, heads, causal):
+    seq, e = x.shape
+    bufs = [_dev(ctx, a) for a in (x, dy, w, np.zeros(w.size, np.float32), np.zeros_like(x))]
+    xb, dyb, wb, gwb, gxb = bufs
+    try:
+        ctx.self_attention_bwd(xb, dyb, seq, e, heads, causal, wb, w.size, gwb, gxb)
+        return gxb.numpy().reshape(seq, e), gwb.numpy()
+    finally:
+        for b in bufs:
+            b.free()
+
+
+# Heads up to 64 take the output from the statistics' kernel, unsplit and with the
+# keys dealt to several workgroups (256 tokens and more); wider ones from the
+# forward.  Head sizes that are and are not 16-byte multiples.
+@pytest.mark.parametrize("seq,e,heads", [(33, 64, 1), (130, 96, 3), (300, 128, 2), (700, 96, 3), (290, 60, 3), (300, 42, 2),
+                                         (270, 192, 2)])
+@pytest.mark.parametrize("causal", [False, True])
+def test_layer_output_beside_the_statistics(ctx, seq, e, heads, causal):
+    x, w = layer_case(seq, e, seq + e, amp=1.5)
+    dy = np.random.default_rng(e).standard_normal((seq, e)).astype(np.float32)
+    wqkv, wout = w[:3 * e * e].reshape(e, 3 * e), w[3 * e * e:].reshape(e, e)
+    (dx, dwqkv, dwout), (tx, twqkv, twout) = self_attention_bwd64(x, wqkv, wout, dy, heads, causal)
+    gx, gw = layer_bwd(ctx, x, w, dy, heads, causal)
+    assert_bwd_close(gx, dx, tx, "dx")
+    assert_bwd_close(gw[:3 * e * e], dwqkv, twqkv, "dWqkv")
+    assert_bwd_close(gw[3 * e * e:], dwout, twout, "dWout")
+
+
+@pytest.mark.parametrize("seq", [100, 300])
+def test_layer_output_without_a_split(ctx, seq):
+    """A value that rounds to infinity in bf16 reaches its dimension of the output,
+    which dWout = att^T dy shows."""
+    e, hd = 64, 32
+    x, w = layer_case(seq, e, 3)
+    wqkv, wout = w[:3 * e * e].reshape(e, 3 * e), w[3 * e * e:].reshape(e, e)
+    x[:, 7] = 0.0
+    x[5, 7] = 3.4e38
+    wqkv[7] = 0.0
+    wqkv[7, 2 * e + 3] = 1.0  # v[5, 3] = 3.4e38
+    wout[3] = 0.0             # and no gradient through it
+    dy = (1e-3 * np.random.default_rng(1).standard_normal((seq, e))).astype(np.float32)
+    qkv = x.astype(np.float64) @ wqkv.astype(np.float64)
+    att = np.zeros((seq, e))
+    for h in range(2):
+        q, k, v = (qkv[:, i * e + h * hd:i * e + (h + 1) * hd] for i in range(3))
+        s = q @ k.T * O.attention_scale(hd)
+        p = np.exp(s - s.max(1, keepdims=True))
+        att[:, h * hd:(h + 1) * hd] = p / p.sum(1, keepdims=True) @ v
+    want = att.T @ dy.astype(np.float64)
+    mag = np.abs(att).T @ np.abs(dy).astype(np.float64)
+    got = layer_bwd(ctx, x, w, dy, 2, False)[1][3 * e * e:].reshape(e, e)
+    assert (np.abs(got - want) <= 2e-5 * mag + 1e-9).all()
