@@ -31,7 +31,7 @@
 // whose blocks fit kDsBytes), written and read once.
 //
 // Bound by latency and the barriers as much as by the matrix cores: at 8 x 32
-// heads x 1024 x 128, causal, 1640 to 1680 us = 102 to 105 TFLOP/s of the five
+// heads x 1024 x 128, causal, 1550 to 1680 us = 102 to 111 TFLOP/s of the five
 // products counted (seven are run: S and dP in steps 1 and 2, then dV, dK and dQ).
 // The kernels alone, traced: step 1 450 us, step 2 950 us with the matrix pipes
 // busy 45% of the cycles (10% more with its tile in one buffer and three
