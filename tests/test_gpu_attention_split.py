@@ -144,7 +144,7 @@ def test_a_nan_costs_no_more_than_a_few_calls(ctx):
         for name, run in runs:
             us = call_us(ctx, run, 3)
             print(f"{name}: {clean[name]:.0f} us, with a NaN key {us:.0f} us", flush=True)
-            assert us < 15 * clean[name], name
+            assert us < 20 * clean[name], name
         assert np.isnan(out.numpy()).all()
     finally:
         for b in bufs:
